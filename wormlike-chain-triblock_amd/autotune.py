@@ -5,7 +5,8 @@ the device inside a short forward + backward sweep (per-launch HIP events, timin
 each step kernel with the GPU to itself) on a cubic grid of edge nz, and the fastest is
 written to csrc/wlc_tune.inc, the table the library compiles in (wlc_tune.cpp).  Variants:
 the one-wave nz = 64 kernel at one or two waves per SIMD, the degree-split two-column and
-whole-tile nz = 64 kernels (Lmax 5-7), the nz = 128 kernels, and the generic kernel with
+whole-tile nz = 64 kernels (Lmax 5-7), the column kernel of the short axes (nz = 24, 32, 48),
+the nz = 128 kernels, and the generic kernel with
 every admissible number of kx columns per workgroup, with and without the degree split
 (Lmax 4-7).  Candidates are selected through the library's measurement switches
 (WLC_GENERIC_ZSOLVE, WLC_ZSOLVE_SPLIT, WLC_ZSOLVE_OCC, WLC_ZSOLVE_TX).
@@ -24,7 +25,6 @@ sys.path.insert(0, HERE)
 # (nz, Lmax values, spectrum precisions): the grids and Lmax of the batched instances, the
 # 64^3 benchmark, the 128^3 precision workload
 SPACE = [
-    (16, (2, 4), (0,)),
     (24, (4, 6), (0,)),
     (32, (4, 6), (0,)),
     (48, (4, 6), (0,)),

@@ -37,6 +37,7 @@ def _units():
     ]
     for L in range(MAX_L + 1):
         units.append(("wlc_zsolve.hip", f"wlc_zsolve_L{L}.o", [f"-DWLC_L={L}"]))
+        units.append(("wlc_zcol.hip", f"wlc_zcol_L{L}.o", [f"-DWLC_L={L}"]))
     return units
 
 

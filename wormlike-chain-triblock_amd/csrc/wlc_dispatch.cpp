@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "wlc_kernels.h"
+#include "wlc_zcol.h"
 
 namespace wlc {
 
@@ -12,11 +13,48 @@ namespace wlc {
   LaunchKey zsolve_key_L##L(const Geom&, const SolveArgs&);                                  \
   hipError_t test_solve_L##L(int, const double*, double, double, double, double, double2*,   \
                              hipStream_t);                                                   \
+  const void* zcol_kernel_L##L(bool, bool);
 
 WLC_DECL(0) WLC_DECL(1) WLC_DECL(2) WLC_DECL(3) WLC_DECL(4) WLC_DECL(5) WLC_DECL(6) WLC_DECL(7) WLC_DECL(8)
 #undef WLC_DECL
 
+namespace {
+// short z axes take the column kernel unless the generic kernel or its degree split (1) is asked
+// for
+bool use_zcol(const Geom& g, const SolveArgs& a) {
+  return zcol_nz(g.nz) && !a.generic && a.split >= 2 && a.M == (a.L + 1) * (a.L + 1);
+}
+
+const void* zcol_kernel(const Geom& g, const SolveArgs& a, bool batch) {
+  switch (a.L) {
+#define WLC_CASE(L) \
+  case L: return zcol_kernel_L##L(g.spec32 != 0, batch);
+    WLC_CASE(0) WLC_CASE(1) WLC_CASE(2) WLC_CASE(3) WLC_CASE(4) WLC_CASE(5) WLC_CASE(6) WLC_CASE(7) WLC_CASE(8)
+#undef WLC_CASE
+  }
+  return nullptr;
+}
+
+hipError_t zcol_launch(const Geom& g, const SolveArgs& a, const ZJob* jobs, int n, hipStream_t st) {
+  const void* k = zcol_kernel(g, a, jobs != nullptr);
+  if (!k) return hipErrorInvalidValue;
+  const size_t lds = zcol_lds_bytes(g.nz, a.M);
+  if (lds > 64 * 1024) {
+    hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  Geom gg = g;
+  SolveArgs aa = a;
+  const ZJob* jp = jobs;
+  void* one[] = {&gg, &aa};
+  void* many[] = {&jp};
+  return hipLaunchKernel(k, dim3(zcol_grid(g), 1, n),
+                         dim3(zcol_threads(g.nz)), jobs ? many : one, lds, st);
+}
+}  // namespace
+
 hipError_t launch_zsolve(const Geom& g, const SolveArgs& a, hipStream_t st) {
+  if (use_zcol(g, a)) return zcol_launch(g, a, nullptr, 1, st);
   switch (a.L) {
 #define WLC_CASE(L) \
   case L: return zsolve_launch_L##L(g, a, st);
@@ -27,6 +65,8 @@ hipError_t launch_zsolve(const Geom& g, const SolveArgs& a, hipStream_t st) {
 }
 
 hipError_t launch_zsolve_batch(const ZJob& rep, const ZJob* jobs, int n, hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+  if (use_zcol(rep.g, rep.a)) return zcol_launch(rep.g, rep.a, jobs, n, st);
   switch (rep.a.L) {
 #define WLC_CASE(L) \
   case L: return zsolve_batch_L##L(rep, jobs, n, st);
@@ -37,6 +77,9 @@ hipError_t launch_zsolve_batch(const ZJob& rep, const ZJob* jobs, int n, hipStre
 }
 
 LaunchKey zsolve_key(const Geom& g, const SolveArgs& a) {
+  if (use_zcol(g, a))
+    return LaunchKey{zcol_kernel(g, a, false), zcol_grid(g), 1u,
+                     (unsigned)zcol_threads(g.nz), zcol_lds_bytes(g.nz, a.M)};
   switch (a.L) {
 #define WLC_CASE(L) \
   case L: return zsolve_key_L##L(g, a);

@@ -30,10 +30,10 @@ ZOpts zsolve_opts(int nz, int L, int spec32) {
   ZOpts o;
   o.generic = 0;
   o.occ = 1;
-  o.split = 2;  // Lmax 5-7 at nz = 64: the whole-tile split kernel; elsewhere a degree split
-  if ((nz == 24 || nz == 32 || nz == 48) && L >= 4 && L <= 7 && !spec32)
-    o.split = 3;  // the half-tile kernel with a wave-local transform (measured faster at every
-                  // tabulated Lmax of these edges)
+  // short nz: the column kernel, at every Lmax and precision (24^3 / Lmax 6 11.2 against 20.5 us of
+  // the half-tile kernel before it, 36^3 / Lmax 4 13.1 against 27 us of the generic one); Lmax 5-7
+  // at nz = 64: the whole-tile split kernel; elsewhere a degree split
+  o.split = 2;
   o.tx = zsolve_tx(nz);
   o.tuned = 0;
   for (const TuneRow& r : kTune) {

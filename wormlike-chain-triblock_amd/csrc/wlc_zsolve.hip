@@ -698,207 +698,6 @@ __global__ void __launch_bounds__(256, 2) k_zsolve64p_b(const ZJob* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// nz = 24, 32, 48, 4 <= Lmax <= 7: the half-tile split kernel with a wave-local transform
-// ---------------------------------------------------------------------------
-// Same workgroup shape as k_zsolve64p (four waves: two columns x two degree parts, two
-// workgroups per CU; the halves of a tile are blocks b and b + 8 on one XCD), lane = z for
-// lanes 0..NZ-1 (the others hold zeros through the solve).  The NZ-point transform of a
-// batch of eight harmonics is a four-step N1 x 8 (N1 = NZ / 8 = 3, 4, 6) in the wave's LDS
-// region: with n = j + N1 m and k = k1 + 8 k2, a DFT-8 over m for each (harmonic, j) (NZ
-// lanes), the twiddle W_NZ^(j k1), then a DFT-N1 over j for each (harmonic, k1) (64 lanes).
-// The generic kernel it replaces reads 16 of every 64 bytes of a tile per thread and runs
-// runtime-planned block-wide Stockham passes.
-template <int NZ>
-struct HalfTile {
-  static constexpr int N1 = NZ / 8;
-  static constexpr int kPad = NZ + NZ / 8;  // padded units per harmonic (pad8(NZ - 1) < kPad)
-  static constexpr int kRegion = (kHB * kPad + 2) > (kXch + 2) ? (kHB * kPad + 2) : (kXch + 2);
-};
-
-// X[k] = sum_n x[n] exp(DIR 2 pi i n k / 6): two DFT-3 and one radix-2 step
-template <int DIR>
-__device__ __forceinline__ void dft6(double2 (&v)[6]) {
-  double2 e[3] = {v[0], v[2], v[4]};
-  double2 o[3] = {v[1], v[3], v[5]};
-  Dft<3, DIR>::run(e);
-  Dft<3, DIR>::run(o);
-  const double s = 0.86602540378443864676;  // sqrt(3)/2
-  // W6^k = exp(DIR 2 pi i k / 6): W6 = (1/2, DIR s), W6^2 = (-1/2, DIR s)
-  const double2 o1 = make_double2(0.5 * o[1].x - DIR * s * o[1].y, 0.5 * o[1].y + DIR * s * o[1].x);
-  const double2 o2 = make_double2(-0.5 * o[2].x - DIR * s * o[2].y, -0.5 * o[2].y + DIR * s * o[2].x);
-  v[0] = cadd(e[0], o[0]);
-  v[3] = csub(e[0], o[0]);
-  v[1] = cadd(e[1], o1);
-  v[4] = csub(e[1], o1);
-  v[2] = cadd(e[2], o2);
-  v[5] = csub(e[2], o2);
-}
-
-template <int N, int DIR>
-__device__ __forceinline__ void small_dft(double2 (&v)[N]) {
-  if constexpr (N == 6) dft6<DIR>(v);
-  else Dft<N, DIR>::run(v);
-}
-
-// the NZ-point transforms of the eight harmonics in region wl (element z of slot h at
-// wl[h kPad + pad8(z)]), in place; DIR < 0 forward, DIR > 0 inverse (unnormalised)
-template <int NZ, int DIR>
-__device__ __forceinline__ void zh_batch(double2* wl, int lane, const double2* __restrict__ twz) {
-  constexpr int N1 = HalfTile<NZ>::N1, P = HalfTile<NZ>::kPad;
-  if (lane < NZ) {
-    const int h = lane / N1, j = lane - N1 * (lane / N1);
-    double2 u[8];
-#pragma unroll
-    for (int m = 0; m < 8; ++m) u[m] = wl[h * P + pad8(j + N1 * m)];
-    Dft<8, DIR>::run(u);
-#pragma unroll
-    for (int k1 = 1; k1 < 8; ++k1) u[k1] = twiddle<DIR>(u[k1], twz[j * k1]);
-    // the positions j + N1 k1 this lane writes are the ones it read
-#pragma unroll
-    for (int k1 = 0; k1 < 8; ++k1) wl[h * P + pad8(j + N1 * k1)] = u[k1];
-  }
-  wave_sync();
-  {
-    const int h = lane >> 3, k1 = lane & 7;
-    double2 u[N1];
-#pragma unroll
-    for (int j = 0; j < N1; ++j) u[j] = wl[h * P + pad8(j + N1 * k1)];
-    small_dft<N1, DIR>(u);
-    wave_sync();  // every lane has read its inputs before any output overwrites them
-#pragma unroll
-    for (int k2 = 0; k2 < N1; ++k2) wl[h * P + pad8(k1 + 8 * k2)] = u[k2];
-  }
-  wave_sync();
-}
-
-template <int NZ, class S>
-__device__ __forceinline__ void k_zsolvehp_body(const Geom& g, const SolveArgs& a) {
-  constexpr int kPadZ = HalfTile<NZ>::kPad, kRegionZ = HalfTile<NZ>::kRegion;
-  extern __shared__ double2 lds[];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int part = wv >> 1, c = wv & 1, gi = threadIdx.x & 127;
-  const int ny = g.ny, nxh = g.nxh, nt = g.nt;
-  const int nb = gridDim.x, b = blockIdx.x;
-  int tl, half;
-  if ((nb & 15) == 0) {
-    const int t = b >> 3;
-    half = t & 1;
-    tl = (t >> 1) * 8 + (b & 7);
-  } else {
-    half = b & 1;
-    tl = b >> 1;
-  }
-  const int t4 = tl % nt, ky = tl / nt;
-  if (t4 * kKxTile + 2 * half >= nxh) return;  // both columns are padding (uniform)
-  const int kx = t4 * kKxTile + 2 * half + c;
-  const bool real_col = kx < nxh;  // wave-uniform
-  // thread gi of a part moves element (z = gi / 2, column gi % 2) of each harmonic
-  const int tz = gi >> 1, tc = gi & 1;
-  const bool io = tz < NZ && t4 * kKxTile + 2 * half + tc < nxh;
-  const int go = kKxTile * tz + tc;
-  const bool active = a.solve && real_col;
-  const long long istride = spec_index(1, 0, 0, 0, ny, nt, NZ);
-  const int nh = part ? PartHi::NH : PartLo::NH;
-  const int hb0 = part ? PartHi::B0 : PartLo::B0;
-  S* hp = reinterpret_cast<S*>(a.spec) + spec_index(0, ky, t4 * kKxTile, 0, ny, nt, NZ) + 2 * half +
-          (long long)hb0 * istride;
-  double2* glds = lds + part * (2 * kRegionZ);
-  double2* wl = glds + c * kRegionZ;
-  double2* xch = lds + c * kRegionZ;  // the Lo wave's region of column c
-  const double2* twz = g.az.tw;        // exp(-2 pi i t / NZ)
-  const int zl = lane < NZ ? lane : 0;
-  const KFrame f(signed_k(kx, g.nx) * a.kfac[0], signed_k(ky, ny) * a.kfac[1],
-                 signed_k(zl, NZ) * a.kfac[2], a.sigma, a.ds);
-  double2 v[kNV];
-#pragma unroll
-  for (int q = 0; q < kNV; ++q) v[q] = make_double2(0.0, 0.0);
-  // forward: per batch of eight harmonics, the part's tiles into LDS (the next batch's loads
-  // in flight), the 48-point transforms, lane = kz back into registers
-  double2 nxt[kHB];
-#pragma unroll
-  for (int q = 0; q < kHB; ++q)
-    nxt[q] = (io && q < nh) ? spec_ld(hp + (long long)q * istride + go) : make_double2(0.0, 0.0);
-#pragma unroll
-  for (int bb = 0; bb < kNBt; ++bb) {
-    const int b0 = bb * kHB;
-    __syncthreads();  // every wave of the part has read the previous batch out of its region
-    if (tz < NZ) {
-#pragma unroll
-      for (int q = 0; q < kHB; ++q)
-        if (b0 + q < nh) glds[tc * kRegionZ + q * kPadZ + pad8(tz)] = nxt[q];
-    }
-    if (bb + 1 < kNBt) {
-#pragma unroll
-      for (int q = 0; q < kHB; ++q) {
-        const int hq = b0 + kHB + q;
-        nxt[q] = (io && hq < nh) ? spec_ld(hp + (long long)hq * istride + go) : make_double2(0.0, 0.0);
-      }
-    }
-    __syncthreads();
-    if (real_col && b0 < nh) {
-      zh_batch<NZ, -1>(wl, lane, twz);
-      if (lane < NZ) {
-#pragma unroll
-        for (int q = 0; q < kHB; ++q)
-          if (b0 + q < kNV && b0 + q < nh) v[b0 + q] = wl[q * kPadZ + pad8(lane)];
-      }
-    }
-  }
-  if (active) {
-    if (part == 0) {
-      PartLo::to_frame(v, f);
-      tri_lower_forward<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
-    } else {
-      PartHi::to_frame(v, f);
-    }
-  }
-  __syncthreads();
-  if (part == 1 && active) tri_upper<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
-  __syncthreads();
-  if (active) {
-    if (part == 0) {
-      tri_lower_back<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
-      PartLo::from_frame(v, f);
-    } else {
-      PartHi::from_frame(v, f);
-    }
-  }
-  // inverse: per batch, lane = kz into LDS, the inverse transforms, the tiles out
-#pragma unroll
-  for (int bb = 0; bb < kNBt; ++bb) {
-    const int b0 = bb * kHB;
-    __syncthreads();  // the previous batch's tiles (and the crossing chains) have been read
-    if (real_col && b0 < nh) {
-      if (lane < NZ) {
-#pragma unroll
-        for (int q = 0; q < kHB; ++q)
-          if (b0 + q < kNV && b0 + q < nh) wl[q * kPadZ + pad8(lane)] = v[b0 + q];
-      }
-      wave_sync();
-      zh_batch<NZ, +1>(wl, lane, twz);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < kHB; ++q)
-      if (io && b0 + q < nh)
-        spec_st(hp + (long long)(b0 + q) * istride + go, glds[tc * kRegionZ + q * kPadZ + pad8(tz)]);
-  }
-}
-
-template <int NZ, class S>
-__global__ void __launch_bounds__(256, 2) k_zsolvehp(Geom g, SolveArgs a) {
-  k_zsolvehp_body<NZ, S>(g, a);
-}
-
-// the same for one instance of a batch per blockIdx.z
-template <int NZ, class S>
-__global__ void __launch_bounds__(256, 2) k_zsolvehp_b(const ZJob* __restrict__ jobs) {
-  const ZJob& j = jobs[blockIdx.z];
-  if (j.skip && *j.skip) return;
-  k_zsolvehp_body<NZ, S>(j.g, j.a);
-}
-
-// ---------------------------------------------------------------------------
 // nz = 128: two waves per (kx, ky) column
 // ---------------------------------------------------------------------------
 // Wave p of a column works on z = m + 64 p (lane m).  Forward: one radix-2 decimation-
@@ -1350,25 +1149,6 @@ hipError_t zsolve_plan(const Geom& g, const SolveArgs& a, ZPlan* z) {
   if constexpr (std::is_same<S, double2>::value) {
     // one workgroup of eight waves per 4-kx tile; FP64 spectrum only: with the FP32 half
     // spectrum (2 KB tiles) the two-column kernel below is faster (64^3/L6: 69 vs 93 us)
-    if ((g.nz == 24 || g.nz == 32 || g.nz == 48) && !a.generic && kL >= 4 && kL <= 7 && a.split == 3) {
-      // two workgroups of four waves per 4-kx tile, wave-local NZ-point transforms
-      z->grid = dim3(2 * g.nt * g.ny);
-      z->block = dim3(256);
-      if (g.nz == 24) {
-        z->k1 = (const void*)k_zsolvehp<24, S>;
-        z->kb = (const void*)k_zsolvehp_b<24, S>;
-        z->lds = sizeof(double2) * (size_t)(2 * 2 * HalfTile<24>::kRegion);
-      } else if (g.nz == 32) {
-        z->k1 = (const void*)k_zsolvehp<32, S>;
-        z->kb = (const void*)k_zsolvehp_b<32, S>;
-        z->lds = sizeof(double2) * (size_t)(2 * 2 * HalfTile<32>::kRegion);
-      } else {
-        z->k1 = (const void*)k_zsolvehp<48, S>;
-        z->kb = (const void*)k_zsolvehp_b<48, S>;
-        z->lds = sizeof(double2) * (size_t)(2 * 2 * HalfTile<48>::kRegion);
-      }
-      return hipSuccess;
-    }
     if (g.nz == 64 && !a.generic && kL >= 5 && kL <= 7 && a.split == 3) {
       // two workgroups of four waves per 4-kx tile (half a tile each)
       z->k1 = (const void*)k_zsolve64p<S>;
