@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/wlc_mde.h"
+#include "wlc_fields.h"
 #include "wlc_host.h"
 #include "wlc_internal.h"
 #include "wlc_kernels.h"
@@ -85,9 +86,10 @@ struct wlc_handle {
   double* w = nullptr;
   double* zero = nullptr;  // one field of zeros: the history plane of a harmonic a slice lacks
   double* rho = nullptr;
-  double* phi = nullptr;
+  double* phi = nullptr;       // dense [nblk][nz][ny][nx]; also the landing place of set_w
   double* partial = nullptr;
-  double* scal = nullptr;      // [0] = int q_0(Ns), [1] = totden
+  double* scal = nullptr;      // [0] = int q_0(Ns), [1] = totden, [2] = 1: phi not finite
+  double* hscal = nullptr;     // pinned copy
   int nparts = 256;
   double2* tw[3] = {nullptr, nullptr, nullptr};
   wlc::AxisPlan plan[3];
@@ -102,18 +104,26 @@ struct wlc_handle {
   hipEvent_t ev_dens[4] = {nullptr, nullptr, nullptr, nullptr};
   bool dens_used[4] = {false, false, false, false};
   // Concurrent sweeps (when the full backward store fits): the backward sweep runs on
-  // stb with its own half spectrum specb while the forward sweep runs on st; slice s of
-  // either sweep records evf[s] / evb[s].  Density term s runs once both slices exist:
-  // on st2 into rho for s <= Ns/2 (ready as the backward sweep reaches s), on st3 into
-  // rho2 for s > Ns/2 (ready as the forward sweep reaches s).  The backward sweep starts
-  // after ev_pre, recorded on st before the forward sweep is queued; every stream is
-  // joined into st before wlc_mde_backward returns.
+  // stb with its own half spectrum specb while the forward sweep runs on st.  A density term
+  // needs slice s of both; the terms are queued on st2 in runs from the middle of the chain
+  // outwards, in the order the sweeps complete them: runs_lo (s <= Ns/2, each complete as the
+  // backward sweep reaches its lower end) and runs_hi (each complete as the forward sweep
+  // reaches its upper end).  evf[0] / evb[0] mark slice Ns/2 of the forward and Ns/2 + 1 of the
+  // backward sweep, evb[1 + k] / evf[1 + k] the ends of runs_lo[k] / runs_hi[k]; fmark / bmark
+  // give the event a slice records (-1: none).  rho holds `parts` accumulators.  The backward
+  // sweep starts after ev_pre, recorded on st before the forward sweep is queued; every stream
+  // is joined into st before wlc_mde_backward returns.
+  struct Run { int lo, hi; };
   bool conc = false;
-  hipStream_t stb = nullptr, st3 = nullptr;
+  hipStream_t stb = nullptr;
   double2* specb = nullptr;
-  double* rho2 = nullptr;
+  int parts = 1;
+  double* cwd = nullptr;               // contour weights of every block on the device
+  std::vector<long long> cwoff;        // of block b: cwd + cwoff[b]
+  std::vector<Run> runs_lo, runs_hi;
   std::vector<hipEvent_t> evf, evb;
-  hipEvent_t ev_pre = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
+  std::vector<int> fmark, bmark;
+  hipEvent_t ev_pre = nullptr, ev_join[2] = {nullptr, nullptr};
   bool pre_recorded = false;
   // Forward-store checkpointing (ck > 0, when the full store does not fit or on request):
   // the forward sweep keeps a 4-slot ring `fr` and copies slices jK-2, jK-1, jK of every
@@ -143,7 +153,7 @@ struct wlc_handle {
   // timing
   bool timing = false;
   bool timing_serial = false;  // timing mode 2: the backward sweep waits for the forward
-  struct Rec { int k; hipEvent_t a, b; };
+  struct Rec { int k; hipEvent_t a, b; int n; };
   std::vector<Rec> recs;
   std::vector<hipEvent_t> pool;
   double ms[5] = {0, 0, 0, 0, 0};
@@ -208,12 +218,11 @@ int flush_timing(wlc_handle* h) {
   HIPCHK(hipStreamSynchronize(h->st));
   HIPCHK(hipStreamSynchronize(h->st2));
   if (h->stb) HIPCHK(hipStreamSynchronize(h->stb));
-  if (h->st3) HIPCHK(hipStreamSynchronize(h->st3));
   for (auto& r : h->recs) {
     float t = 0.f;
     HIPCHK(hipEventElapsedTime(&t, r.a, r.b));
     h->ms[r.k] += t;
-    h->cnt[r.k] += 1;
+    h->cnt[r.k] += r.n;
     h->pool.push_back(r.a);
     h->pool.push_back(r.b);
   }
@@ -225,8 +234,10 @@ struct TimedLaunch {
   wlc_handle* h;
   int k;
   hipStream_t s;
+  int n;  // launches (contour points of a density run) it counts for
   hipEvent_t a = nullptr, b = nullptr;
-  TimedLaunch(wlc_handle* hh, int kk, hipStream_t ss = nullptr) : h(hh), k(kk), s(ss ? ss : hh->st) {
+  TimedLaunch(wlc_handle* hh, int kk, hipStream_t ss = nullptr, int nn = 1)
+      : h(hh), k(kk), s(ss ? ss : hh->st), n(nn) {
     if (h->timing) {
       a = take_event(h);
       b = take_event(h);
@@ -236,22 +247,12 @@ struct TimedLaunch {
   ~TimedLaunch() {
     if (h->timing && a && b) {
       (void)hipEventRecord(b, s);
-      h->recs.push_back({k, a, b});
+      h->recs.push_back({k, a, b, n});
     }
   }
 };
 
-// dense [nf][nz][ny][nx] <-> padded device layout (plane stride zs, field stride hs)
-hipError_t copy_fields_in(wlc_handle* h, double* dst, const double* src, int nf, hipMemcpyKind kind) {
-  const size_t row = sizeof(double) * (size_t)h->p.nx * h->p.ny;
-  for (int f = 0; f < nf; ++f) {
-    hipError_t e = hipMemcpy2DAsync(dst + (long long)f * h->hs, sizeof(double) * h->zs,
-                                    src + (long long)f * h->N, row, row, h->p.nz, kind, h->st);
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
-}
-
+// padded device layout (plane stride zs, field stride hs) -> dense [nf][nz][ny][nx]
 hipError_t copy_fields_out(wlc_handle* h, double* dst, const double* src, int nf, hipMemcpyKind kind) {
   const size_t row = sizeof(double) * (size_t)h->p.nx * h->p.ny;
   for (int f = 0; f < nf; ++f) {
@@ -386,7 +387,10 @@ int step_inverse(wlc_handle* h, const SweepCtx& sw, int s, bool next) {
     TimedLaunch t(h, 4, ss);
     HIPCHK(wlc::launch_inv_rhs(h->geom, ia, ra, order, ss));
   }
-  if (h->conc && sw.fl.mode == 0) HIPCHK(hipEventRecord(dir > 0 ? h->evf[s] : h->evb[s], ss));
+  if (h->conc) {
+    const int m = dir > 0 ? h->fmark[s] : h->bmark[s];
+    if (m >= 0) HIPCHK(hipEventRecord(dir > 0 ? h->evf[m] : h->evb[m], ss));
+  }
   return WLC_OK;
 }
 
@@ -477,26 +481,62 @@ int recompute_segment(wlc_handle* h, int j) {
   return WLC_OK;
 }
 
-// density term s (up to two blocks own slice s) into accumulator `acc` on stream `sd`
-int density_launch(wlc_handle* h, int s, const double* qf, double* acc, hipStream_t sd) {
-  double* rho[2] = {nullptr, nullptr};
-  int lim[2] = {0, 0};
-  double wt[2] = {0.0, 0.0};
-  int n = 0;
-  const int Ms = h->Mb[block_of(h, s)];
-  for (int b = 0; b < h->p.nblk && n < 2; ++b) {
-    const int j = s - h->start[b];
-    if (j < 0 || j > h->p.Nblk[b]) continue;
-    rho[n] = acc + (long long)b * h->hs;
-    lim[n] = std::min(Ms, h->Mb[b]);
-    wt[n] = h->cw[b][j];
-    ++n;
+// density terms lo .. hi on st2 (concurrent sweeps), from hi downwards when step < 0.  A run
+// is cut at the junctions: block b owns the slices start_b < s <= start_b + N_b (0 too for the
+// first block), and its first point is the junction slice of the block before, with the
+// harmonics both hold.
+int density_run(wlc_handle* h, int lo, int hi, int step) {
+  for (int b = 0; b < h->p.nblk; ++b) {
+    const int s0 = h->start[b];
+    wlc::DensityRun r{};
+    r.rho = h->rho + (long long)b * h->hs;
+    r.parts = h->parts;
+    r.pstride = (long long)h->p.nblk * h->hs;
+    r.step = step;
+    if (b > 0 && lo <= s0 && s0 <= hi) {
+      r.q = h->q + h->off[s0];
+      r.qs = qs_slot(h, s0);
+      r.n = 1;
+      r.lim = std::min(h->Mb[b - 1], h->Mb[b]);
+      r.w = h->cwd + h->cwoff[b];
+      TimedLaunch t(h, 3, h->st2, 0);
+      HIPCHK(wlc::launch_density_run(h->geom, r, h->st2));
+    }
+    const int a = std::max(lo, b == 0 ? 0 : s0 + 1), z = std::min(hi, s0 + h->p.Nblk[b]);
+    if (a > z) continue;
+    r.q = h->q + h->off[a];
+    r.qs = qs_slot(h, a);
+    r.stride = (long long)h->Mb[b] * h->hs;
+    r.n = z - a + 1;
+    r.lim = h->Mb[b];
+    r.w = h->cwd + h->cwoff[b] + (a - s0);
+    TimedLaunch t(h, 3, h->st2, r.n);
+    HIPCHK(wlc::launch_density_run(h->geom, r, h->st2));
   }
-  if (n == 0) return WLC_OK;
-  TimedLaunch t(h, 3, sd);
-  HIPCHK(wlc::launch_density_acc(h->geom, qf, qs_slot(h, s), rho[0], lim[0], wt[0], rho[1],
-                                 lim[1], wt[1], sd));
   return WLC_OK;
+}
+
+// the runs and marked slices of the concurrent sweeps: each run takes two fifths of the terms
+// left on its side, so the last ones, which no sweep hides, are short
+void plan_runs(wlc_handle* h) {
+  const int Ns = h->Ns, mid = Ns / 2;
+  auto take = [](int left) { return left <= 2 ? left : std::max(2, (2 * left + 4) / 5); };
+  for (int hi = mid; hi >= 0;) {
+    const int n = take(hi + 1);
+    h->runs_lo.push_back({hi - n + 1, hi});
+    hi -= n;
+  }
+  for (int lo = mid + 1; lo <= Ns;) {
+    const int n = take(Ns - lo + 1);
+    h->runs_hi.push_back({lo, lo + n - 1});
+    lo += n;
+  }
+  h->fmark.assign(Ns + 1, -1);
+  h->bmark.assign(Ns + 1, -1);
+  for (size_t k = 0; k < h->runs_hi.size(); ++k) h->fmark[h->runs_hi[k].hi] = 1 + (int)k;
+  for (size_t k = 0; k < h->runs_lo.size(); ++k) h->bmark[h->runs_lo[k].lo] = 1 + (int)k;
+  h->fmark[mid] = 0;
+  h->bmark[mid + 1] = 0;
 }
 
 int density_at(wlc_handle* h, int s) {
@@ -560,7 +600,6 @@ void free_handle(wlc_handle* h) {
   if (h->st) (void)hipStreamSynchronize(h->st);
   if (h->st2) (void)hipStreamSynchronize(h->st2);
   if (h->stb) (void)hipStreamSynchronize(h->stb);
-  if (h->st3) (void)hipStreamSynchronize(h->st3);
   if (h->str) (void)hipStreamSynchronize(h->str);
   for (auto& r : h->recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
   for (auto e : h->pool) (void)hipEventDestroy(e);
@@ -574,16 +613,16 @@ void free_handle(wlc_handle* h) {
   (void)hipFree(h->phi);
   (void)hipFree(h->partial);
   (void)hipFree(h->scal);
+  if (h->hscal) (void)hipHostFree(h->hscal);
+  (void)hipFree(h->cwd);
   for (auto t : h->tw) (void)hipFree(t);
   if (h->ev_step) (void)hipEventDestroy(h->ev_step);
   for (auto e : h->evf) if (e) (void)hipEventDestroy(e);
   for (auto e : h->evb) if (e) (void)hipEventDestroy(e);
   if (h->ev_pre) (void)hipEventDestroy(h->ev_pre);
   for (auto e : h->ev_join) if (e) (void)hipEventDestroy(e);
-  if (h->st3) (void)hipStreamDestroy(h->st3);
   if (h->stb) (void)hipStreamDestroy(h->stb);
   (void)hipFree(h->specb);
-  (void)hipFree(h->rho2);
   (void)hipFree(h->fr);
   (void)hipFree(h->store);
   (void)hipFree(h->ckpt);
@@ -650,34 +689,32 @@ int backward_concurrent(wlc_handle* h) {
   h->pre_recorded = false;
   HIPCHK(hipStreamWaitEvent(h->stb, h->ev_pre, 0));
   const long long nacc = (long long)h->p.nblk * h->hs;
-  HIPCHK(wlc::launch_fill(h->rho, 0.0, nacc, h->stb));
-  HIPCHK(wlc::launch_fill(h->rho2, 0.0, nacc, h->stb));
+  HIPCHK(wlc::launch_fill(h->rho, 0.0, nacc * h->parts, h->stb));
   HIPCHK(wlc::launch_set_delta(h->geom, qs_slot(h, Ns), h->Mb[block_of(h, Ns)], h->stb));
-  HIPCHK(hipEventRecord(h->evb[Ns], h->stb));
   int rc = sweep(h, main_sweep(h, -1), Ns - 1, 0, false);
   if (rc == WLC_OK && dens) {
-    const int mid = Ns / 2;
-    // s <= Ns/2: ready when the backward sweep reaches s, in decreasing s
-    for (int s = mid; s >= 0 && rc == WLC_OK; --s) {
-      HIPCHK(hipStreamWaitEvent(h->st2, h->evf[s], 0));
-      HIPCHK(hipStreamWaitEvent(h->st2, h->evb[s], 0));
-      rc = density_launch(h, s, h->q + h->off[s], h->rho, h->st2);
-    }
-    // s > Ns/2: ready when the forward sweep reaches s, in increasing s
-    for (int s = mid + 1; s <= Ns && rc == WLC_OK; ++s) {
-      HIPCHK(hipStreamWaitEvent(h->st3, h->evf[s], 0));
-      HIPCHK(hipStreamWaitEvent(h->st3, h->evb[s], 0));
-      rc = density_launch(h, s, h->q + h->off[s], h->rho2, h->st3);
+    HIPCHK(hipStreamWaitEvent(h->st2, h->evf[0], 0));
+    HIPCHK(hipStreamWaitEvent(h->st2, h->evb[0], 0));
+    const size_t nlo = h->runs_lo.size(), nhi = h->runs_hi.size();
+    for (size_t k = 0; k < std::max(nlo, nhi) && rc == WLC_OK; ++k) {
+      if (k < nlo) {
+        HIPCHK(hipStreamWaitEvent(h->st2, h->evb[1 + k], 0));
+        rc = density_run(h, h->runs_lo[k].lo, h->runs_lo[k].hi, -1);
+      }
+      if (k < nhi && rc == WLC_OK) {
+        HIPCHK(hipStreamWaitEvent(h->st2, h->evf[1 + k], 0));
+        rc = density_run(h, h->runs_hi[k].lo, h->runs_hi[k].hi, +1);
+      }
     }
   }
   // join every stream into st, also on failure
-  const hipStream_t side[3] = {h->stb, h->st2, h->st3};
-  for (int k = 0; k < 3; ++k) {
+  const hipStream_t side[2] = {h->stb, h->st2};
+  for (int k = 0; k < 2; ++k) {
     HIPCHK(hipEventRecord(h->ev_join[k], side[k]));
     HIPCHK(hipStreamWaitEvent(h->st, h->ev_join[k], 0));
   }
   if (rc) return rc;
-  if (dens) HIPCHK(wlc::launch_axpy(h->rho, 1.0, h->rho2, nacc, h->st));
+  if (dens) HIPCHK(wlc::launch_sum_parts(h->rho, nacc, h->parts, nacc, h->st));
   h->bwd_done = dens;
   return WLC_OK;
 }
@@ -895,7 +932,11 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
       return fail(WLC_ENOMEM, std::string("device allocation failed: ") + #ptr); \
     }                                                                            \
   } while (0)
+  // the two sweeps' streams one after the other: the runtime gives a new stream the hardware
+  // queue with the fewest users, so the two land on different ones and can overlap (24^3 /
+  // Lmax 6: 3.8 ms a pair of sweeps, 5.7 ms when they share one)
   if (hipStreamCreateWithFlags(&h->st, hipStreamNonBlocking) != hipSuccess ||
+      hipStreamCreateWithFlags(&h->stb, hipStreamNonBlocking) != hipSuccess ||
       hipStreamCreateWithFlags(&h->st2, hipStreamNonBlocking) != hipSuccess) {
     free_handle(h);
     return fail(WLC_EHIP, "stream creation failed");
@@ -968,26 +1009,39 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
     // concurrent sweeps need the full backward store, a second spectrum and a second
     // accumulator; take them when they fit with 2 GiB to spare
     size_t free_b = 0, total_b = 0;
+    wlc::Geom gp{};
+    gp.nx = p->nx; gp.ny = p->ny; gp.nz = p->nz;
+    h->parts = wlc::density_parts(gp);
     const size_t extra = (p->keep_qstar ? 0 : store_bytes) + spec_bytes +
-                         sizeof(double) * (size_t)p->nblk * h->hs;
+                         sizeof(double) * (size_t)p->nblk * h->hs * h->parts;
     const char* ce = std::getenv("WLC_CONCURRENT");
     const bool want = !(ce && std::atoi(ce) == 0);
     h->conc = want && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
               free_b > extra + spec_bytes + (size_t(2) << 30);
+    if (!h->conc) h->parts = 1;
+  }
+  if (!h->conc) {
+    (void)hipStreamDestroy(h->stb);
+    h->stb = nullptr;
   }
   if (p->keep_qstar || h->conc) ALLOC(h->qs, store_bytes);
   else ALLOC(h->qs, sizeof(double) * (size_t)4 * h->Mmax * h->hs);
   ALLOC(h->spec, spec_bytes);
   if (h->conc) {
     ALLOC(h->specb, spec_bytes);
-    ALLOC(h->rho2, sizeof(double) * (size_t)p->nblk * h->hs);
-    if (hipStreamCreateWithFlags(&h->stb, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&h->st3, hipStreamNonBlocking) != hipSuccess) {
-      free_handle(h);
-      return fail(WLC_EHIP, "stream creation failed");
+    std::vector<double> cw;
+    for (int b = 0; b < p->nblk; ++b) {
+      h->cwoff.push_back((long long)cw.size());
+      cw.insert(cw.end(), h->cw[b].begin(), h->cw[b].end());
     }
-    h->evf.assign(h->Ns + 1, nullptr);
-    h->evb.assign(h->Ns + 1, nullptr);
+    ALLOC(h->cwd, sizeof(double) * cw.size());
+    if (hipMemcpy(h->cwd, cw.data(), sizeof(double) * cw.size(), hipMemcpyHostToDevice) != hipSuccess) {
+      free_handle(h);
+      return fail(WLC_EHIP, "contour weight upload failed");
+    }
+    plan_runs(h);
+    h->evf.assign(h->runs_hi.size() + 1, nullptr);
+    h->evb.assign(h->runs_lo.size() + 1, nullptr);
     bool ok = hipEventCreateWithFlags(&h->ev_pre, hipEventDisableTiming) == hipSuccess;
     for (auto& e : h->ev_join) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     for (auto& e : h->evf) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
@@ -1003,10 +1057,14 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
     free_handle(h);
     return fail(WLC_EHIP, "zero field initialisation failed");
   }
-  ALLOC(h->rho, sizeof(double) * (size_t)p->nblk * h->hs);
+  ALLOC(h->rho, sizeof(double) * (size_t)p->nblk * h->hs * h->parts);
   ALLOC(h->phi, sizeof(double) * (size_t)p->nblk * h->hs);
   ALLOC(h->partial, sizeof(double) * h->nparts);
   ALLOC(h->scal, sizeof(double) * 4);
+  if (hipHostMalloc((void**)&h->hscal, sizeof(double) * 4) != hipSuccess) {
+    free_handle(h);
+    return fail(WLC_ENOMEM, "pinned host allocation failed");
+  }
   for (int a = 0; a < 3; ++a) {
     ALLOC(h->tw[a], sizeof(double2) * (size_t)edges[a]);
     if (hipMemcpy(h->tw[a], h->plan[a].tw.data(), sizeof(double2) * edges[a], hipMemcpyHostToDevice) != hipSuccess) {
@@ -1048,7 +1106,9 @@ int wlc_mde_set_box(wlc_handle* h, const double box[3]) {
 int wlc_mde_set_w(wlc_handle* h, const double* w_host) {
   if (!h || !w_host) return fail(WLC_EINVAL, "NULL argument");
   HIPCHK(hipSetDevice(h->device));
-  HIPCHK(copy_fields_in(h, h->w, w_host, h->p.nblk, hipMemcpyHostToDevice));
+  // one contiguous copy, then the padded layout on the device
+  HIPCHK(hipMemcpyAsync(h->phi, w_host, sizeof(double) * (size_t)h->p.nblk * h->N, hipMemcpyHostToDevice, h->st));
+  HIPCHK(wlc::launch_scatter_fields(h->geom, h->phi, h->p.nblk, h->w, h->st));
   HIPCHK(hipStreamSynchronize(h->st));
   h->have_w = true;
   h->fwd_done = h->bwd_done = false;
@@ -1059,7 +1119,8 @@ int wlc_mde_set_w(wlc_handle* h, const double* w_host) {
 int wlc_mde_set_w_device(wlc_handle* h, const double* w_dev) {
   if (!h || !w_dev) return fail(WLC_EINVAL, "NULL argument");
   HIPCHK(hipSetDevice(h->device));
-  HIPCHK(copy_fields_in(h, h->w, w_dev, h->p.nblk, hipMemcpyDeviceToDevice));
+  HIPCHK(hipMemcpyAsync(h->phi, w_dev, sizeof(double) * (size_t)h->p.nblk * h->N, hipMemcpyDeviceToDevice, h->st));
+  HIPCHK(wlc::launch_scatter_fields(h->geom, h->phi, h->p.nblk, h->w, h->st));
   h->have_w = true;
   h->fwd_done = h->bwd_done = false;
   h->pre_recorded = false;  // a concurrent backward sweep must start after the copy
@@ -1081,7 +1142,6 @@ int wlc_mde_forward(wlc_handle* h) {
   }
   const SweepCtx sw = main_sweep(h, +1);
   HIPCHK(wlc::launch_set_delta(h->geom, fwd_slice(h, sw.fl, 0), h->Mb[block_of(h, 0)], h->st));
-  if (h->conc) HIPCHK(hipEventRecord(h->evf[0], h->st));
   int rc = sweep(h, sw, 1, h->Ns, false);
   if (rc) return rc;
   h->fwd_done = true;
@@ -1132,9 +1192,10 @@ static int density_common(wlc_handle* h, double* Q, double* totden) {
   const double V = h->p.box[0] * h->p.box[1] * h->p.box[2];
   HIPCHK(wlc::launch_weighted_sum(h->geom, fwd_last(h), 1, dV, h->partial, h->nparts, h->scal, h->st));
   HIPCHK(wlc::launch_weighted_sum(h->geom, h->rho, h->p.nblk, dV, h->partial, h->nparts, h->scal + 1, h->st));
-  HIPCHK(wlc::launch_phi(h->geom, h->rho, h->p.nblk, V, h->scal + 1, h->phi, h->st));
-  double sc[2];
-  HIPCHK(hipMemcpyAsync(sc, h->scal, sizeof(sc), hipMemcpyDeviceToHost, h->st));
+  HIPCHK(wlc::launch_fill(h->scal + 2, 0.0, 1, h->st));
+  HIPCHK(wlc::launch_phi_dense(h->geom, h->rho, h->p.nblk, V, h->scal + 1, h->phi, h->scal + 2, h->st));
+  const double* sc = h->hscal;
+  HIPCHK(hipMemcpyAsync(h->hscal, h->scal, 3 * sizeof(double), hipMemcpyDeviceToHost, h->st));
   HIPCHK(hipStreamSynchronize(h->st));
   // timed launches are read out here, where the host waits anyway, so that timing does not
   // add a synchronisation between the forward and the backward sweep
@@ -1154,10 +1215,9 @@ int wlc_mde_density(wlc_handle* h, double* phi_host, double* Q, double* totden) 
   int rc = density_common(h, Q, totden);
   if (rc) return rc;
   if (phi_host) {
-    HIPCHK(copy_fields_out(h, phi_host, h->phi, h->p.nblk, hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpyAsync(phi_host, h->phi, sizeof(double) * (size_t)h->p.nblk * h->N, hipMemcpyDeviceToHost, h->st));
     HIPCHK(hipStreamSynchronize(h->st));
-    for (long long e = 0; e < (long long)h->p.nblk * h->N; ++e)
-      if (!std::isfinite(phi_host[e])) return fail(WLC_ENONFINITE, "phi not finite");
+    if (h->hscal[2] != 0.0) return fail(WLC_ENONFINITE, "phi not finite");
   }
   return WLC_OK;
 }
@@ -1166,7 +1226,8 @@ int wlc_mde_density_device(wlc_handle* h, double* phi_dev, double* Q, double* to
   if (!h) return fail(WLC_EINVAL, "NULL handle");
   int rc = density_common(h, Q, totden);
   if (rc) return rc;
-  if (phi_dev) HIPCHK(copy_fields_out(h, phi_dev, h->phi, h->p.nblk, hipMemcpyDeviceToDevice));
+  if (phi_dev)
+    HIPCHK(hipMemcpyAsync(phi_dev, h->phi, sizeof(double) * (size_t)h->p.nblk * h->N, hipMemcpyDeviceToDevice, h->st));
   return WLC_OK;
 }
 
