@@ -1,6 +1,7 @@
 """Kernels of the short axes (two-factor plans) against the oracle: the column z solve at every
 nz it takes, at the smallest and largest Lmax, with ragged column groups, both storage types of
-the spectrum, and as batched jobs."""
+the spectrum, and as batched jobs; the two-pass plane kernels at every edge along x and along y,
+and fused against unfused."""
 import numpy as np
 import pytest
 
@@ -79,6 +80,57 @@ def test_z_columns_batched(wlc):
         phi, Q, td = g.density()
         bphi, bQ, btd = b.density(i)
         # the twins run the same operations; contraction may differ
+        assert _rel(bphi, phi) < 1e-13 and abs(bQ - Q) / Q < 1e-13 and abs(btd - td) / td < 1e-13
+        g.close()
+    b.close()
+
+
+# every edge as nx and as ny, short with long (idle lanes in one role), compile-time squares
+PLANES = [(8, 72), (72, 8), (12, 54), (54, 12), (16, 36), (36, 16), (18, 48), (48, 18), (24, 32),
+          (32, 24), (64, 18), (12, 64), (24, 24), (32, 32), (48, 48), (72, 72), (36, 54)]
+
+
+@pytest.mark.parametrize("ny,nx", PLANES)
+def test_two_pass_planes(wlc, oracle, ny, nx):
+    # the basis shrinks, then grows; nz = 2 walks contiguous (harmonic, z)
+    _check(wlc, oracle, (2, ny, nx), (3, 2, 3), (2, 1, 3))
+
+
+@pytest.mark.parametrize("shape,spec32", [((8, 18, 24), False), ((6, 54, 36), False), ((4, 32, 32), True),
+                                          ((4, 16, 72), True)])
+def test_two_pass_planes_fused_equals_unfused(wlc, monkeypatch, shape, spec32):
+    Nblk, L = (3, 3, 2), (3, 1, 2)
+    box, lam, w = _case(shape, Nblk, L, 9)
+    out = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("WLC_FUSE", fuse)
+        g = wlc.WormlikeMDE(shape, box, Nblk, L, lam, keep_qstar=True, spectrum_fp32=spec32)
+        g.set_w(w)
+        g.MDE_q()
+        g.MDE_qstar()
+        out.append([g.get_q(d, s) for d in (1, -1) for s in range(sum(Nblk) + 1)])
+        g.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+def test_two_pass_planes_batched(wlc):
+    cases = []
+    for shape, L in (((4, 24, 18), 2), ((4, 24, 18), 2), ((8, 36, 54), 1), ((4, 48, 48), 3)):
+        box, lam, w = _case(shape, (3, 4), (L, L), sum(shape) + len(cases))
+        cases.append(dict(shape=shape, box=box, Nblk=(3, 4), L=(L, L), lam=lam, w=w,
+                          chi=np.array([[0, 15, 0], [15, 0, 0], [0, 0, 0]], float)))
+    b = wlc.Batch(cases)
+    for i, c in enumerate(cases):
+        b.set_w(i, c["w"])
+    b.sweep()
+    for i, c in enumerate(cases):
+        g = wlc.WormlikeMDE(c["shape"], c["box"], c["Nblk"], c["L"], c["lam"])
+        g.set_w(c["w"])
+        g.MDE_q()
+        g.MDE_qstar()
+        phi, Q, td = g.density()
+        bphi, bQ, btd = b.density(i)
         assert _rel(bphi, phi) < 1e-13 and abs(bQ - Q) / Q < 1e-13 and abs(btd - td) / td < 1e-13
         g.close()
     b.close()

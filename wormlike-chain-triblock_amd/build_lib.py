@@ -31,6 +31,7 @@ def _units():
         ("wlc_batch.hip", "wlc_batch.o", []),
         ("wlc_unet.hip", "wlc_unet.o", []),
         ("wlc_plane.hip", "wlc_plane.o", []),
+        ("wlc_plane2.hip", "wlc_plane2.o", []),
         ("wlc_fields.hip", "wlc_fields.o", []),
         ("wlc_dispatch.cpp", "wlc_dispatch.o", ["-x", "hip"]),
         ("sh_setup.cpp", "sh_setup.o", []),
