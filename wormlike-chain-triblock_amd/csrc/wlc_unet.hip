@@ -5,12 +5,11 @@
 // still decides the converged state.
 //
 // Layout: activations channels-last [B][D][H][W][C] with C a multiple of 16, stored as
-// bfloat16 where a convolution reads them; pre-activations, gradients and master weights
-// FP32.  Convolutions are 3x3x3, zero padding 1, stride 1, weights [Cout][27][Cin] (tap
-// t = 9 kz + 3 ky + kx).  Every convolution (forward, gradient with respect to the input,
-// gradient with respect to the weights) is an implicit GEMM on the bf16 matrix cores
-// (v_mfma_f32_16x16x16_bf16, FP32 accumulation):
-//   forward   M = voxels, N = Cout, K = 27 Cin
+// bfloat16 where a convolution reads them; gradients and master weights FP32.  Convolutions are
+// 3x3x3, zero padding 1, stride 1, weights [Cout][27][Cin] (tap t = 9 kz + 3 ky + kx).  Every
+// convolution (forward, gradient with respect to the input, gradient with respect to the weights)
+// is an implicit GEMM on the bf16 matrix cores (FP32 accumulation):
+//   forward   M = Cout, N = voxels, K = 27 Cin
 //   input     the forward kernel on the output gradient with the flipped, transposed kernel
 //             W'[ci][26 - t][co] = W[co][t][ci]
 //   weights   M = Cout, N = Cin per tap, K = voxels, split over voxel chunks whose partial
@@ -24,6 +23,7 @@
 // first 3 of 16 channels (the others have zero weights and no loss).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstdint>
@@ -76,158 +76,222 @@ __device__ __forceinline__ long long neighbour(const Vol& g, long long v, int t)
   return ((b * g.D + zz) * g.H + yy) * g.W + xx;
 }
 
-// Y[v][co] = bias[co] + sum_{t, ci} W[co][t][ci] X[nbr(v, t)][ci] (zero outside the grid).
-// Workgroup = 64 consecutive voxels x 16 NT output channels, wave w its voxels 16 w .. 16 w + 15.
-// Matrix-core step (16 voxels x 16 channels x KI input channels): lane l holds the input
-// channels KI/4 (l / 16) .. of voxel l % 16 (A) and of output channel l % 16 (B), contiguous
-// in both tensors, so each operand is one 8- or 16-byte load; it receives D[4 (l / 16) + r]
-// [l % 16].  KI = 32 (v_mfma_f32_16x16x32_bf16) when Cin is a multiple of 32, else 16.  The
-// voxel's coordinates are decoded once; a tap only adds an offset and checks the bounds.
-template <int NT, int KI>
-__global__ void __launch_bounds__(256) k_conv_fwd(const bf16* __restrict__ X, const bf16* __restrict__ Wt,
-                                                  const float* __restrict__ bias, float* __restrict__ Y,
-                                                  Vol g, int Cin, int Cout) {
-  constexpr int CPL = KI / 4;  // input channels per lane and step
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int row = lane & 15, kq = lane >> 4;
-  const int V = (int)g.voxels();
-  const int vb = blockIdx.x * 64 + 16 * wv;
-  const int v = vb + row;
-  const int co0 = blockIdx.y * 16 * NT;
-  const bool vin = v < V;
-  int x = 0, y = 0, z = 0;
-  if (vin) {
-    x = v % g.W;
-    const int r = v / g.W;
-    y = r % g.H;
-    z = (r / g.H) % g.D;
+// The weights in the order the matrix cores read them: K input channels (KI = 32 of them per step
+// when K is a multiple of 32, else 16), N output channels; one step of 16 output channels is a
+// run of 64 lanes x KI / 4 values, lane l holding the channels KI/4 (l / 16) .. of output
+// channel l % 16.
+__host__ __device__ inline size_t packed_at(int K, int N, int t, int k, int n) {
+  if (K % 32 == 0)
+    return ((((size_t)t * (K / 32) + k / 32) * (N / 16) + n / 16) * 64 + n % 16 + 16 * ((k % 32) / 8)) * 8 + k % 8;
+  return ((((size_t)t * (K / 16) + k / 16) * (N / 16) + n / 16) * 64 + n % 16 + 16 * ((k % 16) / 4)) * 4 + k % 4;
+}
+
+typedef unsigned short us4 __attribute__((ext_vector_type(4)));
+
+// What a convolution does with four consecutive output channels co .. co + 3 of voxel v.
+struct EpiF32 {  // Y = sum + bias
+  float* Y;
+  const float* bias;
+  int C;
+  __device__ __forceinline__ void operator()(int v, int co, f32x4 s) const {
+    if (bias) s += *reinterpret_cast<const f32x4*>(bias + co);
+    *reinterpret_cast<f32x4*>(Y + (size_t)v * C + co) = s;
   }
-  f32x4 acc[NT];
+};
+struct EpiOut {  // the network's output: the first 3 channels
+  float* Y;
+  const float* bias;
+  __device__ __forceinline__ void operator()(int v, int co, f32x4 s) const {
+    if (co) return;
+    s += *reinterpret_cast<const f32x4*>(bias);
+    Y[(size_t)v * 3] = s[0];
+    Y[(size_t)v * 3 + 1] = s[1];
+    Y[(size_t)v * 3 + 2] = s[2];
+  }
+};
+// bf16(relu(sum + bias)) into channels off .. of a tensor of Ct channels, or (up) into those of
+// the eight voxels of the next finer grid it is upsampled to
+template <bool UP>
+struct EpiAct {
+  bf16* a;
+  const float* bias;
+  int Ct, off;
+  Vol g;
+  __device__ __forceinline__ void operator()(int v, int co, f32x4 s) const {
+    s += *reinterpret_cast<const f32x4*>(bias + co);
+    us4 h;
 #pragma unroll
-  for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const size_t wstride = (size_t)16 * 27 * Cin;  // between the NT output-channel tiles
-  for (int t = 0; t < 27; ++t) {
-    const int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
-    const bool ok = vin && (unsigned)(z + dz) < (unsigned)g.D && (unsigned)(y + dy) < (unsigned)g.H &&
-                    (unsigned)(x + dx) < (unsigned)g.W;
-    const int nb = ok ? v + (dz * g.H + dy) * g.W + dx : 0;
-    const bf16* xr = X + (size_t)nb * Cin + CPL * kq;
-    const bf16* wr = Wt + ((size_t)(co0 + row) * 27 + t) * Cin + CPL * kq;
-    for (int c0 = 0; c0 < Cin; c0 += KI) {
-      if constexpr (KI == 32) {
-        const s16x8 a = ok ? *reinterpret_cast<const s16x8*>(xr + c0) : s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int r = 0; r < 4; ++r) h[r] = f2bf(s[r] < 0.f ? 0.f : s[r]);
+    if constexpr (!UP) {
+      *reinterpret_cast<us4*>(a + (size_t)v * Ct + off + co) = h;
+    } else {
+      const int x = v % g.W;
+      int q = v / g.W;
+      const int y = q % g.H;
+      q /= g.H;  // b D + z
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          const s16x8 b = *reinterpret_cast<const s16x8*>(wr + j * wstride + c0);
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                           __builtin_bit_cast(bf16x8, b), acc[j], 0, 0, 0);
-        }
-      } else {
-        const bf16x4 a = ok ? *reinterpret_cast<const bf16x4*>(xr + c0) : bf16x4{0, 0, 0, 0};
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          const bf16x4 b = *reinterpret_cast<const bf16x4*>(wr + j * wstride + c0);
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[j], 0, 0, 0);
-        }
+      for (int d = 0; d < 8; ++d) {
+        const size_t f = ((size_t)(2 * q + (d >> 2)) * 2 * g.H + 2 * y + ((d >> 1) & 1)) * 2 * g.W + 2 * x + (d & 1);
+        *reinterpret_cast<us4*>(a + f * Ct + off + co) = h;
       }
     }
   }
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int co = co0 + 16 * j + row;
-    const float bv = bias ? bias[co] : 0.f;
+};
+// gradient of a pre-activation: the sum where the activation is positive, FP32 and bf16
+struct EpiMask {
+  const bf16* act;
+  float* dy;
+  bf16* dyb;
+  int C;
+  __device__ __forceinline__ void operator()(int v, int co, f32x4 s) const {
+    const size_t at = (size_t)v * C + co;
+    const us4 m = *reinterpret_cast<const us4*>(act + at);
+    us4 h;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int vv = vb + 4 * kq + r;
-      if (vv < V) Y[(size_t)vv * Cout + co] = acc[j][r] + bv;
+      s[r] = m[r] ? s[r] : 0.f;  // an activation is never negative
+      h[r] = f2bf(s[r]);
     }
+    *reinterpret_cast<f32x4*>(dy + at) = s;
+    *reinterpret_cast<us4*>(dyb + at) = h;
   }
-}
+};
 
-// The same convolution (Cin a multiple of 32) with the weights staged through LDS and the
-// next step's operands in flight: per K step (tap t, 32 input channels) the workgroup's
-// 16 NT x 32 weight block (NT KB) is loaded once by 64 NT threads into one of two LDS buffers
-// instead of once per wave, every wave reads its B fragments from there (16 lanes of equal
-// kq read 256 contiguous bytes), and the global loads of step k + 1 (weights and the gathered
-// input run) are issued before the matrix-core steps of step k.  One barrier per step: a
-// thread reaching barrier k has finished its reads of step k - 1, so the buffer written next
-// is free.
-template <int NT>
-__global__ void __launch_bounds__(256) k_conv_fwd_l(const bf16* __restrict__ X, const bf16* __restrict__ Wt,
-                                                    const float* __restrict__ bias, float* __restrict__ Y,
-                                                    Vol g, int Cin, int Cout) {
-  __shared__ s16x8 wbuf[2][4 * 16 * NT];  // [kq][output channel] 16-byte pieces
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int row = lane & 15, kq = lane >> 4;
+// sum_{t, ci} W[co][t][ci] X[nbr(v, t)][ci] (zero outside the grid) for 16 MT voxels x 16 NT
+// output channels per wave, four waves (64 MT voxels) per workgroup.  Matrix-core step: A the
+// packed weights (16 output channels x KI), B the KI channels of 16 voxels; lane l receives the
+// sums of output channels 4 (l / 16) .. + 3 of voxel l % 16, so the epilogue stores 8 or 16 bytes.
+// A voxel outside the grid is read from a zero row: a tap's neighbour is one bit of a mask per
+// voxel and an address select, every load is unconditional, and the operands of the next D steps
+// are in flight.  The steps run in the order tap, then channel.
+// The first version loaded each step's operands one step ahead, the weights through LDS with a
+// barrier per step (64^3: 32 -> 32 channels 57 us, 64 -> 32 130 us, 16^3: 128 -> 128 49 us).
+template <int MT, int NT, int KI, int D, class Epi>
+__global__ void __launch_bounds__(256) k_conv(const bf16* __restrict__ X, const bf16* __restrict__ Wp,
+                                              const bf16* __restrict__ zrow, Vol g, int Cin, int Cout, Epi epi) {
+  constexpr int CPL = KI / 4;  // channels per lane and step
+  typedef short frag __attribute__((ext_vector_type(CPL)));
+  const int lane = threadIdx.x & 63, row = lane & 15, kq = lane >> 4;
   const int V = (int)g.voxels();
-  const int vb = blockIdx.x * 64 + 16 * wv;
-  const int v = vb + row;
+  const int vb = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (16 * MT);
   const int co0 = blockIdx.y * 16 * NT;
-  const bool vin = v < V;
-  int x = 0, y = 0, z = 0;
-  if (vin) {
-    x = v % g.W;
-    const int r = v / g.W;
-    y = r % g.H;
-    z = (r / g.H) % g.D;
+  const bf16* xb[MT];
+  unsigned mask[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int v = vb + 16 * m + row;
+    const int x = v % g.W, q = v / g.W, y = q % g.H, z = (q / g.H) % g.D;
+    const unsigned mx = (x > 0 ? 1u : 0u) | 2u | (x + 1 < g.W ? 4u : 0u);
+    const unsigned my = (y > 0 ? 1u : 0u) | 2u | (y + 1 < g.H ? 4u : 0u);
+    const unsigned mz = (z > 0 ? 1u : 0u) | 2u | (z + 1 < g.D ? 4u : 0u);
+    unsigned b = 0;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+      b |= ((my >> (t / 3)) & 1u) && ((mx >> (t % 3)) & 1u) ? 1u << t : 0u;
+    mask[m] = v < V ? ((mz & 1u) ? b : 0u) | (b << 9) | ((mz & 4u) ? b << 18 : 0u) : 0u;
+    xb[m] = X + (size_t)v * Cin + CPL * kq;
   }
-  const int nch = Cin >> 5;
-  const int K = 27 * nch;
-  // staging role: thread st < 64 NT moves the 8 channels 8 (st & 3) .. of output channel st >> 2
-  const int st = threadIdx.x;
-  const bool stager = st < 64 * NT;
-  const int sco = st >> 2, skq = st & 3;
-  const bf16* wrow = Wt + (size_t)(co0 + (stager ? sco : 0)) * 27 * Cin + 8 * skq;
-  const s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto load_w = [&](int ks) -> s16x8 {
-    const int t = ks / nch, c0 = (ks - t * nch) << 5;
-    return stager ? *reinterpret_cast<const s16x8*>(wrow + (size_t)t * Cin + c0) : zero;
-  };
-  auto load_a = [&](int ks) -> s16x8 {
-    const int t = ks / nch, c0 = (ks - t * nch) << 5;
-    const int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
-    const bool ok = vin && (unsigned)(z + dz) < (unsigned)g.D && (unsigned)(y + dy) < (unsigned)g.H &&
-                    (unsigned)(x + dx) < (unsigned)g.W;
-    const int nb = ok ? v + (dz * g.H + dy) * g.W + dx : 0;
-    return ok ? *reinterpret_cast<const s16x8*>(X + (size_t)nb * Cin + c0 + 8 * kq) : zero;
-  };
-  f32x4 acc[NT];
+  const int nch = Cin / KI, K = 27 * nch;
+  const bf16* wp = Wp + ((size_t)(co0 / 16) * 64 + lane) * CPL;
+  const size_t wstep = (size_t)(Cout / 16) * 64 * CPL;
+  const bf16* zr = zrow + CPL * kq;
+  // the step loaded next: tap, channel, offset of the tap's neighbour
+  int lt = 0, lc = 0;
+  long long shift = (long long)(-g.H * g.W - g.W - 1) * Cin;
+  frag a[D][NT], b[D][MT];
+  auto load = [&](int d) {
 #pragma unroll
-  for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  s16x8 wn = load_w(0), an = load_a(0);
-  for (int ks = 0; ks < K; ++ks) {
-    const s16x8 wc = wn, ac = an;
-    if (stager) wbuf[ks & 1][skq * (16 * NT) + sco] = wc;
-    if (ks + 1 < K) {
-      wn = load_w(ks + 1);
-      an = load_a(ks + 1);
+    for (int j = 0; j < NT; ++j) a[d][j] = *reinterpret_cast<const frag*>(wp + j * 64 * CPL);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const bf16* p = (mask[m] >> lt) & 1u ? xb[m] + shift + lc : zr;
+      b[d][m] = *reinterpret_cast<const frag*>(p);
     }
-    __syncthreads();
+    wp += wstep;
+    lc += KI;
+    if (lc == Cin) {
+      lc = 0;
+      ++lt;
+      const int dz = lt / 9 - 1, dy = (lt / 3) % 3 - 1, dx = lt % 3 - 1;
+      shift = (long long)((dz * g.H + dy) * g.W + dx) * Cin;
+    }
+  };
+  f32x4 acc[MT][NT];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const s16x8 b = wbuf[ks & 1][kq * (16 * NT) + 16 * j + row];
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ac),
-                                                       __builtin_bit_cast(bf16x8, b), acc[j], 0, 0, 0);
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  static_assert(27 % D == 0, "K is a multiple of D");
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d);
+  for (int ks = 0; ks < K; ks += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          if constexpr (KI == 32)
+            acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[d][j]),
+                                                                __builtin_bit_cast(bf16x8, b[d][m]), acc[m][j], 0, 0, 0);
+          else
+            acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(bf16x4, a[d][j]),
+                                                                  __builtin_bit_cast(bf16x4, b[d][m]), acc[m][j], 0, 0, 0);
+        }
+      if (ks + d + D < K) load(d);
     }
   }
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int co = co0 + 16 * j + row;
-    const float bv = bias ? bias[co] : 0.f;
+  for (int m = 0; m < MT; ++m) {
+    const int v = vb + 16 * m + row;
+    if (v >= V) continue;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int vv = vb + 4 * kq + r;
-      if (vv < V) Y[(size_t)vv * Cout + co] = acc[j][r] + bv;
-    }
+    for (int j = 0; j < NT; ++j) epi(v, co0 + 16 * j + 4 * kq, acc[m][j]);
   }
 }
 
-// out[c][v] = in[v][c] (bf16), 32 x 32 tiles through LDS
-__global__ void __launch_bounds__(256) k_transpose(const bf16* __restrict__ in, bf16* __restrict__ out,
-                                                   int V, int C) {
+// One layer's weight and bias gradient.  All layers go through each kernel below in one launch
+// (their inputs are all there once the gradient has run down the network): a layer of the coarse
+// grids alone fills a fraction of the GPU.  first[k] is the layer's first workgroup in launch k.
+struct GradJob {
+  const bf16 *X, *dYb;  // input and output gradient, channels-last
+  const float* dYf;
+  bf16 *xt, *dyt;       // transposed: [C][V]
+  float *part, *bpart, *dW, *db;
+  Vol g;
+  int V, cin, cout;
+  int mc, nc;           // 16-channel tiles per wave: output, input
+  int chunk, nch;       // voxels per chunk, chunks
+  int nbp, bchunk;      // bias parts, voxels of each
+  int first[6];
+};
+enum { kTrX = 0, kTrY = 1, kDw = 2, kSum = 3, kBias = 4, kBiasEnd = 5 };
+constexpr int kMaxJobs = 11;
+struct GradJobs {
+  GradJob j[kMaxJobs];
+  int n;
+};
+
+// the job of workgroup b of launch k (uniform); b becomes its own count
+__device__ __forceinline__ const GradJob& job_of(const GradJobs* __restrict__ J, int k, int& b) {
+  int i = 0;
+  for (int t = 1; t < J->n; ++t)
+    if (b >= J->j[t].first[k]) i = t;
+  b -= J->j[i].first[k];
+  return J->j[i];
+}
+
+// xt[c][v] = X[v][c], dyt[c][v] = dYb[v][c] (bf16), 32 x 32 tiles through LDS
+__global__ void __launch_bounds__(256) k_transpose(const GradJobs* __restrict__ J, int which) {
   __shared__ bf16 tile[32][33];
+  int b = blockIdx.x;
+  const GradJob& q = job_of(J, which, b);
+  const bf16* in = which == kTrX ? q.X : q.dYb;
+  bf16* out = which == kTrX ? q.xt : q.dyt;
+  const int V = q.V, C = which == kTrX ? q.cin : q.cout;
+  const int nc = (C + 31) / 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const int v0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
+  const int v0 = (b / nc) * 32, c0 = (b % nc) * 32;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int v = v0 + ty + 8 * r, c = c0 + tx;
@@ -242,71 +306,100 @@ __global__ void __launch_bounds__(256) k_transpose(const bf16* __restrict__ in, 
 }
 
 // part[chunk][co][t][ci] = sum_{v in chunk} dY[v][co] X[nbr(v, t)][ci] from the transposed
-// operands dYT [Cout][V] and XT [Cin][V]: the voxels are the reduction index, so lane l's
-// eight consecutive voxels 8 (l / 16) .. of a 32-voxel step are one 16-byte load of a
-// channel row.  Needs W % 8 == 0 (eight consecutive voxels lie in one x row: their tap
-// neighbours are the same run shifted by dx, read as the aligned run and its left or right
-// neighbour run) and V, chunk multiples of 32.  One wave per (tap, 16 MC output channels,
-// 16 NC input channels, voxel chunk).
+// operands: the voxels are the reduction index, so lane l's eight consecutive voxels 8 (l / 16) ..
+// of a 32-voxel step are one 16-byte load of a channel row.  Needs W % 8 == 0 (eight consecutive
+// voxels lie in one x row: their tap neighbours are the same run shifted by dx, read as the
+// aligned run and one element of its left or right neighbour run) and V, chunk multiples of 32.
+// One wave per (dz, dy), 16 MC output channels, 16 NC input channels and voxel chunk: its three
+// taps dx = -1, 0, 1 share the output gradient's and the input's run.
 template <int MC, int NC>
-__global__ void __launch_bounds__(64) k_conv_dw_t(const bf16* __restrict__ dYT, const bf16* __restrict__ XT,
-                                                  float* __restrict__ part, Vol g, int Cin, int Cout, int chunk) {
+__device__ __forceinline__ void dw_wave(const GradJob& q, int idx) {
   const int lane = threadIdx.x, row = lane & 15, kq = lane >> 4;
-  const int nci = Cin / (16 * NC);
-  int idx = blockIdx.x;
-  const int t = idx % 27;
-  idx /= 27;
+  const Vol g = q.g;
+  const int V = q.V, Cin = q.cin, Cout = q.cout, nci = Cin / (16 * NC);
+  const int ch = idx % q.nch;
+  idx /= q.nch;
+  const int t3 = idx % 9;
+  idx /= 9;
   const int ci0 = (idx % nci) * 16 * NC, co0 = (idx / nci) * 16 * MC;
-  const int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
-  const int V = (int)g.voxels();
-  const int vb0 = blockIdx.y * chunk;
-  const int ve = vb0 + chunk < V ? vb0 + chunk : V;
+  const int dz = t3 / 3 - 1, dy = t3 % 3 - 1;
+  const int vb0 = ch * q.chunk, ve = min(vb0 + q.chunk, V);
   const int rowshift = (dz * g.H + dy) * g.W;
   const s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  f32x4 acc[MC][NC];
+  const bf16* dyr = q.dyt + (size_t)(co0 + row) * V;
+  const bf16* xr = q.xt + (size_t)(ci0 + row) * V + rowshift;
+  f32x4 acc[3][MC][NC];
 #pragma unroll
-  for (int i = 0; i < MC; ++i)
+  for (int d = 0; d < 3; ++d)
 #pragma unroll
-    for (int j = 0; j < NC; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int vb = vb0; vb < ve; vb += 32) {
+    for (int i = 0; i < MC; ++i)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) acc[d][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  s16x8 an[MC], cn[NC];
+  short ln[NC], rn[NC];
+  auto load = [&](int vb) {
     const int v = vb + 8 * kq;  // this lane's eight voxels v .. v + 7: one x-row run
-    const int x = v % g.W;
-    const int r1 = v / g.W;
-    const int y = r1 % g.H, z = (r1 / g.H) % g.D;
-    const bool rowok = (unsigned)(z + dz) < (unsigned)g.D && (unsigned)(y + dy) < (unsigned)g.H;
-    const int base = v + rowshift;  // neighbour run at dx = 0 (a multiple of 8)
-    s16x8 a[MC], b[NC];
+    const int x = v % g.W, r1 = v / g.W, y = r1 % g.H, z = (r1 / g.H) % g.D;
+    const bool ok = (unsigned)(z + dz) < (unsigned)g.D && (unsigned)(y + dy) < (unsigned)g.H;
+    const bool lok = ok && x > 0, rok = ok && x + 8 < g.W;
 #pragma unroll
-    for (int i = 0; i < MC; ++i) a[i] = *reinterpret_cast<const s16x8*>(dYT + (size_t)(co0 + 16 * i + row) * V + v);
+    for (int i = 0; i < MC; ++i) an[i] = *reinterpret_cast<const s16x8*>(dyr + (size_t)(16 * i) * V + v);
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-      const bf16* p = XT + (size_t)(ci0 + 16 * j + row) * V;
-      const s16x8 c = rowok ? *reinterpret_cast<const s16x8*>(p + base) : zero;
-      if (dx == 0) {
-        b[j] = c;
-      } else if (dx < 0) {  // voxels v - 1 .. v + 6: the last of the run to the left, then c[0..6]
-        const s16x8 l = (rowok && x > 0) ? *reinterpret_cast<const s16x8*>(p + base - 8) : zero;
-        b[j] = s16x8{l[7], c[0], c[1], c[2], c[3], c[4], c[5], c[6]};
-      } else {  // voxels v + 1 .. v + 8: c[1..7], then the first of the run to the right
-        const s16x8 r = (rowok && x + 8 < g.W) ? *reinterpret_cast<const s16x8*>(p + base + 8) : zero;
-        b[j] = s16x8{c[1], c[2], c[3], c[4], c[5], c[6], c[7], r[0]};
+      const bf16* p = xr + (size_t)(16 * j) * V + v;
+      cn[j] = ok ? *reinterpret_cast<const s16x8*>(p) : zero;
+      ln[j] = lok ? (short)p[-1] : (short)0;
+      rn[j] = rok ? (short)p[8] : (short)0;
+    }
+  };
+  if (vb0 < ve) load(vb0);
+  for (int vb = vb0; vb < ve; vb += 32) {
+    s16x8 a[MC], c[NC];
+    short l[NC], r[NC];
+#pragma unroll
+    for (int i = 0; i < MC; ++i) a[i] = an[i];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      c[j] = cn[j];
+      l[j] = ln[j];
+      r[j] = rn[j];
+    }
+    if (vb + 32 < ve) load(vb + 32);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const s16x8 bl = s16x8{l[j], c[j][0], c[j][1], c[j][2], c[j][3], c[j][4], c[j][5], c[j][6]};
+      const s16x8 br = s16x8{c[j][1], c[j][2], c[j][3], c[j][4], c[j][5], c[j][6], c[j][7], r[j]};
+#pragma unroll
+      for (int i = 0; i < MC; ++i) {
+        const bf16x8 av = __builtin_bit_cast(bf16x8, a[i]);
+        acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, bl), acc[0][i][j], 0, 0, 0);
+        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, c[j]), acc[1][i][j], 0, 0, 0);
+        acc[2][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, br), acc[2][i][j], 0, 0, 0);
       }
     }
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
 #pragma unroll
     for (int i = 0; i < MC; ++i)
 #pragma unroll
       for (int j = 0; j < NC; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[i]),
-                                                            __builtin_bit_cast(bf16x8, b[j]), acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          q.part[(((size_t)ch * Cout + co0 + 16 * i + 4 * kq + r) * 27 + 3 * t3 + d) * Cin + ci0 + 16 * j + row] =
+              acc[d][i][j][r];
+}
+
+__global__ void __launch_bounds__(64) k_conv_dw_t(const GradJobs* __restrict__ J) {
+  int b = blockIdx.x;
+  const GradJob& q = job_of(J, kDw, b);
+  if (q.mc == 2) {
+    if (q.nc == 2) dw_wave<2, 2>(q, b);
+    else dw_wave<2, 1>(q, b);
+  } else {
+    if (q.nc == 2) dw_wave<1, 2>(q, b);
+    else dw_wave<1, 1>(q, b);
   }
-#pragma unroll
-  for (int i = 0; i < MC; ++i)
-#pragma unroll
-    for (int j = 0; j < NC; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        part[(((size_t)blockIdx.y * Cout + co0 + 16 * i + 4 * kq + r) * 27 + t) * Cin + ci0 + 16 * j + row] =
-            acc[i][j][r];
 }
 
 // part[chunk][co][t][ci] = sum_{v in chunk} dY[v][co] X[nbr(v, t)][ci] on the channels-last
@@ -341,24 +434,30 @@ __global__ void __launch_bounds__(64) k_conv_dw(const bf16* __restrict__ dY, con
     part[(((long long)blockIdx.y * Cout + co0 + 4 * kq + r) * 27 + t) * Cin + ci0 + row] = acc[r];
 }
 
-// out[i] = sum_c part[c][i], chunks in order
-__global__ void k_sum_chunks(const float* __restrict__ part, float* __restrict__ out, long long n, int nch) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+// dW[i] = sum_c part[c][i], chunks in order
+__global__ void __launch_bounds__(256) k_sum_chunks(const GradJobs* __restrict__ J) {
+  int b = blockIdx.x;
+  const GradJob& q = job_of(J, kSum, b);
+  const long long n = (long long)q.cout * 27 * q.cin;
+  const long long i = b * 256LL + threadIdx.x;
   if (i >= n) return;
   float s = 0.f;
-  for (int c = 0; c < nch; ++c) s += part[(long long)c * n + i];
-  out[i] = s;
+#pragma unroll 8
+  for (int c = 0; c < q.nch; ++c) s += q.part[(long long)c * n + i];
+  q.dW[i] = s;
 }
 
 // bpart[p][c] = sum of dY[v][c] over the voxels of part p (FP32): the 256 threads are
 // 256 / C voxel lanes x C channels (C <= 256), so each pass reads 256 / C whole voxel rows;
 // every lane keeps four partial sums (independent loads in flight), and the sums are added
 // in a fixed order (deterministic)
-__global__ void __launch_bounds__(256) k_bias_partial(const float* __restrict__ dY, float* __restrict__ bpart,
-                                                      int V, int C, int vchunk) {
+__global__ void __launch_bounds__(256) k_bias_partial(const GradJobs* __restrict__ J) {
   __shared__ float red[256];
-  const int nr = 256 / C, c = threadIdx.x % C, r = threadIdx.x / C;
-  const int v0 = blockIdx.x * vchunk, v1 = v0 + vchunk < V ? v0 + vchunk : V;
+  int b = blockIdx.x;
+  const GradJob& q = job_of(J, kBias, b);
+  const float* __restrict__ dY = q.dYf;
+  const int C = q.cout, nr = 256 / C, c = threadIdx.x % C, r = threadIdx.x / C;
+  const int v0 = b * q.bchunk, v1 = min(v0 + q.bchunk, q.V);
   float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
   if (r < nr) {
     int v = v0 + r;
@@ -375,150 +474,160 @@ __global__ void __launch_bounds__(256) k_bias_partial(const float* __restrict__ 
   if (threadIdx.x < C) {
     float t = 0.f;
     for (int k = 0; k < nr; ++k) t += red[k * C + c];
-    bpart[(size_t)blockIdx.x * C + c] = t;
+    q.bpart[(size_t)b * C + c] = t;
   }
 }
 
-// db[c] = sum over the np parts of bpart[p][c]: one workgroup per channel, each thread adds
+// db[c] = sum over the parts of bpart[p][c]: one workgroup per channel, each thread adds
 // the parts t, t + 256, ... in order, then a tree in shared memory (fixed order)
-__global__ void __launch_bounds__(256) k_bias_final(const float* __restrict__ bpart, float* __restrict__ db,
-                                                    int np, int C) {
+__global__ void __launch_bounds__(256) k_bias_final(const GradJobs* __restrict__ J) {
   __shared__ float red[256];
-  const int c = blockIdx.x;
+  int c = blockIdx.x;
+  const GradJob& q = job_of(J, kBiasEnd, c);
   float s = 0.f;
-  for (int p = threadIdx.x; p < np; p += 256) s += bpart[(size_t)p * C + c];
+  for (int p = threadIdx.x; p < q.nbp; p += 256) s += q.bpart[(size_t)p * q.cout + c];
   red[threadIdx.x] = s;
   __syncthreads();
   for (int k = 128; k > 0; k >>= 1) {
     if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
     __syncthreads();
   }
-  if (threadIdx.x == 0) db[c] = red[0];
+  if (threadIdx.x == 0) q.db[c] = red[0];
 }
 
-// W'[ci][26 - t][co] = W[co][t][ci] (bf16)
-__global__ void k_flip_weights(const bf16* __restrict__ W, bf16* __restrict__ Wf, int Cin, int Cout) {
-  const long long n = (long long)Cout * 27 * Cin;
+// where a weight goes in the packed copies: fwd of the layer's own kernel, bwd of the flipped,
+// transposed one
+struct PackLayer {
+  long long woff;
+  int cin, cout;
+};
+struct PackTable {
+  PackLayer l[11];
+  int n;
+};
+__device__ __forceinline__ void pack_weight(const PackTable& T, bf16* fwd, bf16* bwd, long long i, bf16 h) {
+  int k = 0;
+  for (int t = 1; t < T.n; ++t)
+    if (i >= T.l[t].woff) k = t;
+  const int cin = T.l[k].cin, cout = T.l[k].cout;
+  const long long j = i - T.l[k].woff;
+  if (j >= (long long)cout * 27 * cin) return;  // a bias
+  const int ci = (int)(j % cin), r = (int)(j / cin), t = r % 27, co = r / 27;
+  fwd[T.l[k].woff + packed_at(cin, cout, t, ci, co)] = h;
+  bwd[T.l[k].woff + packed_at(cout, cin, 26 - t, co, ci)] = h;
+}
+__global__ void k_pack(const float* __restrict__ p, PackTable T, bf16* __restrict__ fwd, bf16* __restrict__ bwd,
+                       long long n) {
+  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (i < n) pack_weight(T, fwd, bwd, i, f2bf(p[i]));
+}
+
+// input [V][11] -> bf16 [V][16], the last five zero
+__global__ void k_input(const float* __restrict__ x, bf16* __restrict__ o, long long V) {
+  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (i >= V * 16) return;
+  const long long v = i >> 4;
+  const int c = (int)(i & 15);
+  o[i] = c < 11 ? f2bf(x[v * 11 + c]) : (bf16)0;
+}
+
+// 2x2x2 average pooling of channels [off, off + C) of a tensor of Ct (bf16 in and out)
+__global__ void k_pool(const bf16* __restrict__ x, bf16* __restrict__ o, Vol go, int C, int Ct, int off) {
+  const long long n = go.voxels() * (C / 4);
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int ci = (int)(i % Cin);
-  const int t = (int)((i / Cin) % 27);
-  const int co = (int)(i / ((long long)Cin * 27));
-  Wf[((long long)ci * 27 + (26 - t)) * Cout + co] = W[i];
-}
-
-// a = bf16(relu(y)) (relu = 0: a = bf16(y)) into channels [off, off + C) of a tensor of Ct
-// channels
-__global__ void k_act(const float* __restrict__ y, bf16* __restrict__ a, long long V, int C, int Ct,
-                      int off, int relu) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= V * C) return;
-  const long long v = i / C;
-  const int c = (int)(i - v * C);
-  float x = y[i];
-  if (relu && x < 0.f) x = 0.f;
-  a[v * Ct + off + c] = f2bf(x);
-}
-
-// dy = (y > 0) * da[channels off .. off + C of Ct]  (dy FP32; dyb its bf16 copy)
-__global__ void k_relu_back(const float* __restrict__ y, const float* __restrict__ da, float* __restrict__ dy,
-                            bf16* __restrict__ dyb, long long V, int C, int Ct, int off, int relu) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= V * C) return;
-  const long long v = i / C;
-  const int c = (int)(i - v * C);
-  const float g = da[v * Ct + off + c];
-  const float d = (!relu || y[i] > 0.f) ? g : 0.f;
-  dy[i] = d;
-  dyb[i] = f2bf(d);
-}
-
-// 2x2x2 average pooling of bf16 activations (out bf16)
-__global__ void k_pool(const bf16* __restrict__ x, bf16* __restrict__ o, Vol go, int C) {
-  const long long n = go.voxels() * C;
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int c = (int)(i % C);
-  long long v = i / C;
+  const int c = 4 * (int)(i % (C / 4));
+  long long v = i / (C / 4);
+  const long long vo = v;
   const int X = (int)(v % go.W);
   v /= go.W;
   const int Y = (int)(v % go.H);
-  v /= go.H;
-  const int Z = (int)(v % go.D);
-  const long long b = v / go.D;
-  const int Wi = 2 * go.W, Hi = 2 * go.H, Di = 2 * go.D;
-  float s = 0.f;
-  for (int dz = 0; dz < 2; ++dz)
-    for (int dy = 0; dy < 2; ++dy)
-      for (int dx = 0; dx < 2; ++dx)
-        s += bf2f(x[(((b * Di + 2 * Z + dz) * Hi + 2 * Y + dy) * Wi + 2 * X + dx) * C + c]);
-  o[i] = f2bf(s * 0.125f);
+  v /= go.H;  // b D + Z
+  const int Wi = 2 * go.W, Hi = 2 * go.H;
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int d = 0; d < 8; ++d) {
+    const size_t f = ((size_t)(2 * v + (d >> 2)) * Hi + 2 * Y + ((d >> 1) & 1)) * Wi + 2 * X + (d & 1);
+    const us4 h = *reinterpret_cast<const us4*>(x + f * Ct + off + c);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s[r] += bf2f(h[r]);
+  }
+  us4 h;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) h[r] = f2bf(s[r] * 0.125f);
+  *reinterpret_cast<us4*>(o + vo * C + c) = h;
 }
 
-// adjoint of the pooling: dx (fine, FP32) += do / 8 into channels [off, off + C) of Ct
-__global__ void k_pool_back(const float* __restrict__ dout, float* __restrict__ dx, Vol gi, int C, int Ct,
-                            int off) {
-  const long long n = gi.voxels() * C;
+// gradient of a pre-activation whose activation was upsampled into channels [0, C) of the Ct of
+// the next finer grid: the sum of the eight fine gradients where the activation (read at the first
+// of its eight copies) is positive
+__global__ void k_up_back(const float* __restrict__ dfine, const bf16* __restrict__ act, float* __restrict__ dy,
+                          bf16* __restrict__ dyb, Vol gc, int C, int Ct) {
+  const long long n = gc.voxels() * (C / 4);
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int c = (int)(i % C);
-  long long v = i / C;
-  const int X = (int)(v % gi.W);
-  long long r = v / gi.W;
-  const int Y = (int)(r % gi.H);
-  r /= gi.H;
-  const int Z = (int)(r % gi.D);
-  const long long b = r / gi.D;
-  const long long vc = ((b * (gi.D / 2) + Z / 2) * (gi.H / 2) + Y / 2) * (gi.W / 2) + X / 2;
-  dx[v * Ct + off + c] += dout[vc * C + c] * 0.125f;
-}
-
-// nearest 2x upsampling of bf16 activations into channels [off, off + C) of Ct (fine grid)
-__global__ void k_up(const bf16* __restrict__ x, bf16* __restrict__ o, Vol gf, int C, int Ct, int off) {
-  const long long n = gf.voxels() * C;
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int c = (int)(i % C);
-  long long v = i / C;
-  const int X = (int)(v % gf.W);
-  long long r = v / gf.W;
-  const int Y = (int)(r % gf.H);
-  r /= gf.H;
-  const int Z = (int)(r % gf.D);
-  const long long b = r / gf.D;
-  const long long vc = ((b * (gf.D / 2) + Z / 2) * (gf.H / 2) + Y / 2) * (gf.W / 2) + X / 2;
-  o[v * Ct + off + c] = x[vc * C + c];
-}
-
-// adjoint of the upsampling: dx (coarse, FP32) = sum of the 8 fine gradients of channels
-// [off, off + C) of Ct
-__global__ void k_up_back(const float* __restrict__ dfine, float* __restrict__ dx, Vol gc, int C, int Ct,
-                          int off) {
-  const long long n = gc.voxels() * C;
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int c = (int)(i % C);
-  long long v = i / C;
+  const int c = 4 * (int)(i % (C / 4));
+  long long v = i / (C / 4);
+  const long long vo = v;
   const int X = (int)(v % gc.W);
   v /= gc.W;
   const int Y = (int)(v % gc.H);
   v /= gc.H;
-  const int Z = (int)(v % gc.D);
-  const long long b = v / gc.D;
-  const int Wf = 2 * gc.W, Hf = 2 * gc.H, Df = 2 * gc.D;
-  float s = 0.f;
-  for (int dz = 0; dz < 2; ++dz)
-    for (int dy = 0; dy < 2; ++dy)
-      for (int dx2 = 0; dx2 < 2; ++dx2)
-        s += dfine[((((b * Df + 2 * Z + dz) * Hf + 2 * Y + dy) * Wf + 2 * X + dx2) * Ct) + off + c];
-  dx[i] += s;
+  const int Wf = 2 * gc.W, Hf = 2 * gc.H;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  us4 m = {0, 0, 0, 0};
+#pragma unroll
+  for (int d = 0; d < 8; ++d) {
+    const size_t f = ((size_t)(2 * v + (d >> 2)) * Hf + 2 * Y + ((d >> 1) & 1)) * Wf + 2 * X + (d & 1);
+    s += *reinterpret_cast<const f32x4*>(dfine + f * Ct + c);
+    if (d == 0) m = *reinterpret_cast<const us4*>(act + f * Ct + c);
+  }
+  us4 h;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    s[r] = m[r] ? s[r] : 0.f;
+    h[r] = f2bf(s[r]);
+  }
+  *reinterpret_cast<f32x4*>(dy + vo * C + c) = s;
+  *reinterpret_cast<us4*>(dyb + vo * C + c) = h;
 }
 
-// loss partials: sum over the first nout channels of (y - t)^2 and the gradient
-// 2 (y - t) / count (zero on the padding channels)
+// gradient of a pre-activation whose activation is the skip half [off, off + C) of a concatenated
+// tensor of Ct channels and was pooled: the skip's gradient plus an eighth of the pooled one,
+// where the activation is positive
+__global__ void k_skip_back(const float* __restrict__ dcat, const float* __restrict__ dpool,
+                            const bf16* __restrict__ act, float* __restrict__ dy, bf16* __restrict__ dyb, Vol g, int C,
+                            int Ct, int off) {
+  const long long n = g.voxels() * (C / 4);
+  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int c = 4 * (int)(i % (C / 4));
+  const long long v = i / (C / 4);
+  const int X = (int)(v % g.W);
+  long long r1 = v / g.W;
+  const int Y = (int)(r1 % g.H);
+  r1 /= g.H;  // b D + z
+  const long long vc = ((r1 / 2) * (g.H / 2) + Y / 2) * (g.W / 2) + X / 2;
+  f32x4 s = *reinterpret_cast<const f32x4*>(dcat + v * Ct + off + c);
+  const f32x4 p = *reinterpret_cast<const f32x4*>(dpool + vc * C + c);
+  const us4 m = *reinterpret_cast<const us4*>(act + v * Ct + off + c);
+  us4 h;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    s[r] += p[r] * 0.125f;
+    s[r] = m[r] ? s[r] : 0.f;
+    h[r] = f2bf(s[r]);
+  }
+  *reinterpret_cast<f32x4*>(dy + v * C + c) = s;
+  *reinterpret_cast<us4*>(dyb + v * C + c) = h;
+}
+
+// loss partials: sum over the nout channels of (y - t)^2 and the gradient 2 (y - t) / count, FP32
+// and bf16, of the C channels of the output convolution (zero on the padding)
 __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ y, const float* __restrict__ t,
-                                             float* __restrict__ dy, float* __restrict__ part, long long V,
-                                             int C, int nout, float inv_count) {
+                                             float* __restrict__ dy, bf16* __restrict__ dyb,
+                                             float* __restrict__ part, long long V, int C, int nout,
+                                             float inv_count) {
   __shared__ float red[256];
   float s = 0.f;
   for (long long i = blockIdx.x * 256LL + threadIdx.x; i < V * C; i += (long long)gridDim.x * 256) {
@@ -526,11 +635,12 @@ __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ y, const 
     const int c = (int)(i - v * C);
     float g = 0.f;
     if (c < nout) {
-      const float d = y[i] - t[v * nout + c];
+      const float d = y[v * nout + c] - t[v * nout + c];
       s += d * d;
       g = 2.f * d * inv_count;
     }
     dy[i] = g;
+    dyb[i] = f2bf(g);
   }
   red[threadIdx.x] = s;
   __syncthreads();
@@ -541,41 +651,25 @@ __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ y, const 
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// Adam on FP32 master weights with a bf16 copy for the matrix cores; `mask` zeroes the
+// Adam on FP32 master weights with the packed bf16 copies for the matrix cores; `mask` zeroes the
 // padding entries (kept exactly zero)
 __global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                       const float* __restrict__ g, bf16* __restrict__ pb, const unsigned char* __restrict__ mask,
-                       long long n, float lr, float b1, float b2, float eps, float c1, float c2) {
+                       const float* __restrict__ g, PackTable T, bf16* __restrict__ fwd, bf16* __restrict__ bwd,
+                       const unsigned char* __restrict__ mask, long long n, float lr, float b1, float b2, float eps,
+                       float c1, float c2) {
   const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  if (mask && !mask[i]) {
-    p[i] = 0.f;
-    if (pb) pb[i] = 0;
-    return;
+  float pi = 0.f;
+  if (mask[i]) {
+    const float gi = g[i];
+    const float mi = b1 * m[i] + (1.f - b1) * gi;
+    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   }
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   p[i] = pi;
-  if (pb) pb[i] = f2bf(pi);
-}
-
-__global__ void k_to_bf16(const float* __restrict__ x, bf16* __restrict__ o, long long n) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i < n) o[i] = f2bf(x[i]);
-}
-
-// dst[v][c] += src[v][off + c] (channels [off, off + C) of a tensor of Cs channels)
-__global__ void k_slice_add(const float* __restrict__ src, float* __restrict__ dst, long long V, int C, int Cs,
-                            int off) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= V * C) return;
-  const long long v = i / C;
-  const int c = (int)(i - v * C);
-  dst[i] += src[v * Cs + off + c];
+  pack_weight(T, fwd, bwd, i, f2bf(pi));
 }
 
 inline unsigned blocks(long long n, int t = 256) { return (unsigned)((n + t - 1) / t); }
@@ -624,29 +718,28 @@ struct wlc_unet {
   hipStream_t st = nullptr;
   int n = 0, B = 0;
   std::vector<Layer> layers;
+  PackTable pack{};
   long long np = 0;       // flat parameter count (padded)
   float *p = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;
-  bf16* pb = nullptr;     // bf16 copy of the parameters (weights used by the kernels)
+  bf16 *wf = nullptr, *wb = nullptr;  // packed bf16 weights of the convolutions and of their adjoints
+  bf16* zrow = nullptr;               // a row of zeros (a voxel outside the grid)
   unsigned char* mask = nullptr;
-  bf16* wflip = nullptr;  // flipped weights of one layer
-  float* part = nullptr;  // weight-gradient partial sums
-  float* bpart = nullptr; // bias-gradient partial sums
-  bf16 *xt = nullptr, *dyt = nullptr;  // a layer's input and output gradient, transposed
-  long long part_n = 0;
   float* lpart = nullptr;
   int adam_t = 0;
-  // activations (bf16) per tensor and level
-  bf16 *x0 = nullptr, *a0a = nullptr, *s0 = nullptr, *p1 = nullptr, *a1a = nullptr, *s1 = nullptr,
-       *p2 = nullptr, *a2a = nullptr, *s2 = nullptr, *p3 = nullptr, *bt = nullptr, *c2 = nullptr,
-       *d2 = nullptr, *c1 = nullptr, *d1 = nullptr, *c0 = nullptr, *d0 = nullptr;
-  // their gradients (FP32)
-  float *ga0a = nullptr, *gs0 = nullptr, *gp1 = nullptr, *ga1a = nullptr, *gs1 = nullptr, *gp2 = nullptr,
-        *ga2a = nullptr, *gs2 = nullptr, *gp3 = nullptr, *gbt = nullptr, *gc2 = nullptr, *gd2 = nullptr,
-        *gc1 = nullptr, *gd1 = nullptr, *gc0 = nullptr, *gd0 = nullptr;
-  float* y[11] = {};      // pre-activations
-  float* dy[11] = {};     // their gradients
+  // activations (bf16): cN holds the concatenation [upsampled, skip] of level N, pN the pooled skip
+  // of level N - 1
+  bf16 *x0 = nullptr, *a0a = nullptr, *p1 = nullptr, *a1a = nullptr, *p2 = nullptr, *a2a = nullptr, *p3 = nullptr,
+       *c2 = nullptr, *c1 = nullptr, *c0 = nullptr, *d0 = nullptr;
+  // gradients (FP32) of the concatenations and the pooled tensors
+  float *gp1 = nullptr, *gp2 = nullptr, *gp3 = nullptr, *gc2 = nullptr, *gc1 = nullptr, *gc0 = nullptr;
+  float* y = nullptr;     // output [V][3]
+  float* dy[11] = {};     // gradients of the pre-activations
   bf16* dyb[11] = {};     // bf16 copies (matrix-core operand)
-  float* target = nullptr;
+  float *xin = nullptr, *target = nullptr;
+  std::vector<GradJob> jobs;          // weight gradients in one launch per kernel ...
+  std::vector<GradJob> odd;           // ... and of the layers whose x edge is no multiple of 8
+  GradJobs *djobs = nullptr, *dall = nullptr;
+  unsigned grid[6] = {};              // workgroups of each launch
   std::vector<void*> allocs;  // parameters and optimiser state
   std::vector<void*> acts;    // activations, gradients and scratch of the current grid and batch
   Vol vol(int level) const { return Vol{B, n >> level, n >> level, n >> level}; }
@@ -689,10 +782,71 @@ void unet_free(wlc_unet* u) {
   delete u;
 }
 
-// voxel chunks of the weight-gradient reduction (at most 64, about 4096 voxels each)
-int wgrad_chunks(long long V) { return (int)std::min<long long>(64, std::max<long long>(1, V / 4096)); }
 // partial sums of the bias gradient (at most; about 256 voxels each)
 constexpr int kBiasParts = 1024;
+// voxel chunks of the weight-gradient reduction: 2048 voxels each (one wave's 64 steps), at most 128
+constexpr int kChunkVoxels = 2048, kMaxChunks = 128;
+
+// the transposed kernel takes the layer (else the element-wise one)
+bool grad_rows(const Vol& g) { return g.W % 8 == 0 && g.voxels() % 32 == 0; }
+
+// sizes of a layer's gradient job (the pointers are the caller's)
+GradJob grad_job(const Vol& g, int cin, int cout) {
+  GradJob q{};
+  q.g = g;
+  q.V = (int)g.voxels();
+  q.cin = cin;
+  q.cout = cout;
+  q.mc = cout % 32 == 0 ? 2 : 1;
+  q.nc = cin % 32 == 0 ? 2 : 1;
+  const int step = 32;
+  const int want = std::max(kChunkVoxels, (q.V + kMaxChunks - 1) / kMaxChunks);
+  q.chunk = (std::min(want, q.V) + step - 1) / step * step;
+  q.nch = (q.V + q.chunk - 1) / q.chunk;
+  q.nbp = (int)std::min<long long>(kBiasParts, std::max<long long>(1, q.V / 256));
+  q.bchunk = (q.V + q.nbp - 1) / q.nbp;
+  return q;
+}
+long long part_floats(const GradJob& q) { return (long long)q.nch * q.cout * 27 * q.cin; }
+
+// first workgroups of every job in every launch, and the launches' sizes
+void place_jobs(std::vector<GradJob>& rows, unsigned grid[6]) {
+  for (int k = 0; k < 6; ++k) {
+    long long b = 0;
+    for (GradJob& q : rows) {
+      q.first[k] = (int)b;
+      const long long v32 = (q.V + 31) / 32;
+      switch (k) {
+        case kTrX: b += v32 * ((q.cin + 31) / 32); break;
+        case kTrY: b += v32 * ((q.cout + 31) / 32); break;
+        case kDw: b += 9LL * q.nch * (q.cout / (16 * q.mc)) * (q.cin / (16 * q.nc)); break;
+        case kSum: b += ((long long)q.cout * 27 * q.cin + 255) / 256; break;
+        case kBias: b += q.nbp; break;
+        case kBiasEnd: b += q.cout; break;
+      }
+    }
+    grid[k] = (unsigned)b;
+  }
+}
+
+// weight and bias gradients: `jobs` (device: every layer, with the first workgroups of the sum and
+// bias launches) and `rows` (device: those of the transposed kernel), odd the element-wise layers
+int launch_grads(hipStream_t st, const GradJobs* all, const GradJobs* rows, bool any_rows,
+                 const std::vector<GradJob>& odd, const unsigned grid[6]) {
+  if (any_rows) {
+    hipLaunchKernelGGL(k_transpose, dim3(grid[kTrX]), dim3(256), 0, st, rows, (int)kTrX);
+    hipLaunchKernelGGL(k_transpose, dim3(grid[kTrY]), dim3(256), 0, st, rows, (int)kTrY);
+    hipLaunchKernelGGL(k_conv_dw_t, dim3(grid[kDw]), dim3(64), 0, st, rows);
+  }
+  for (const GradJob& q : odd)
+    hipLaunchKernelGGL(k_conv_dw, dim3(27 * (q.cout / 16) * (q.cin / 16), q.nch), dim3(64), 0, st, q.dYb, q.X, q.part,
+                       q.g, q.cin, q.cout, (long long)q.chunk);
+  hipLaunchKernelGGL(k_sum_chunks, dim3(grid[kSum]), dim3(256), 0, st, all);
+  hipLaunchKernelGGL(k_bias_partial, dim3(grid[kBias]), dim3(256), 0, st, all);
+  hipLaunchKernelGGL(k_bias_final, dim3(grid[kBiasEnd]), dim3(256), 0, st, all);
+  UCHK(hipGetLastError());
+  return WLC_OK;
+}
 
 // activation, gradient and scratch buffers for grid edge n and batch B
 int alloc_acts(wlc_unet* u, int n, int B) {
@@ -701,214 +855,163 @@ int alloc_acts(wlc_unet* u, int n, int B) {
   u->B = B;
   int rc;
 #define UA(ptr, cnt) if ((rc = ualloc(u->acts, &(ptr), (cnt)))) { free_acts(u); return rc; }
-  long long maxpart = 0, maxx = 0, maxdy = 0;
-  for (const Layer& l : u->layers) {
-    const long long nw = (long long)l.cout * 27 * l.cin;
-    const long long V = u->vol(l.level).voxels();
-    maxpart = std::max(maxpart, wgrad_chunks(V) * nw);
-    maxx = std::max(maxx, V * l.cin);
-    maxdy = std::max(maxdy, V * l.cout);
-  }
-  UA(u->part, maxpart); UA(u->lpart, 256); UA(u->bpart, (long long)kBiasParts * 256);
-  UA(u->xt, maxx); UA(u->dyt, maxdy);
   const long long V0 = u->vol(0).voxels(), V1 = u->vol(1).voxels(), V2 = u->vol(2).voxels(), V3 = u->vol(3).voxels();
-  UA(u->x0, V0 * 16); UA(u->a0a, V0 * 32); UA(u->s0, V0 * 32); UA(u->p1, V1 * 32); UA(u->a1a, V1 * 64);
-  UA(u->s1, V1 * 64); UA(u->p2, V2 * 64); UA(u->a2a, V2 * 128); UA(u->s2, V2 * 128); UA(u->p3, V3 * 128);
-  UA(u->bt, V3 * 128); UA(u->c2, V2 * 256); UA(u->d2, V2 * 64); UA(u->c1, V1 * 128); UA(u->d1, V1 * 32);
-  UA(u->c0, V0 * 64); UA(u->d0, V0 * 32);
-  UA(u->ga0a, V0 * 32); UA(u->gs0, V0 * 32); UA(u->gp1, V1 * 32); UA(u->ga1a, V1 * 64); UA(u->gs1, V1 * 64);
-  UA(u->gp2, V2 * 64); UA(u->ga2a, V2 * 128); UA(u->gs2, V2 * 128); UA(u->gp3, V3 * 128); UA(u->gbt, V3 * 128);
-  UA(u->gc2, V2 * 256); UA(u->gd2, V2 * 64); UA(u->gc1, V1 * 128); UA(u->gd1, V1 * 32); UA(u->gc0, V0 * 64);
-  UA(u->gd0, V0 * 32);
+  UA(u->lpart, 256);
+  UA(u->x0, V0 * 16); UA(u->a0a, V0 * 32); UA(u->p1, V1 * 32); UA(u->a1a, V1 * 64);
+  UA(u->p2, V2 * 64); UA(u->a2a, V2 * 128); UA(u->p3, V3 * 128);
+  UA(u->c2, V2 * 256); UA(u->c1, V1 * 128); UA(u->c0, V0 * 64); UA(u->d0, V0 * 32);
+  UA(u->gp1, V1 * 32); UA(u->gp2, V2 * 64); UA(u->gp3, V3 * 128);
+  UA(u->gc2, V2 * 256); UA(u->gc1, V1 * 128); UA(u->gc0, V0 * 64);
+  UA(u->y, V0 * 3); UA(u->xin, V0 * 11); UA(u->target, V0 * 3);
+  const bf16* X[11] = {u->x0, u->a0a, u->p1, u->a1a, u->p2, u->a2a, u->p3, u->c2, u->c1, u->c0, u->d0};
+  u->jobs.clear();
+  u->odd.clear();
+  std::vector<GradJob> all;
   for (int li = 0; li < 11; ++li) {
     const Layer& l = u->layers[li];
-    const long long V = u->vol(l.level).voxels();
-    UA(u->y[li], V * l.cout); UA(u->dy[li], V * l.cout); UA(u->dyb[li], V * l.cout);
+    const Vol g = u->vol(l.level);
+    const long long V = g.voxels();
+    UA(u->dy[li], V * l.cout); UA(u->dyb[li], V * l.cout);
+    GradJob q = grad_job(g, l.cin, l.cout);
+    q.X = X[li];
+    q.dYb = u->dyb[li];
+    q.dYf = u->dy[li];
+    q.dW = u->g + l.woff;
+    q.db = u->g + l.boff;
+    UA(q.part, part_floats(q));
+    UA(q.bpart, (long long)q.nbp * l.cout);
+    if (grad_rows(g)) {
+      UA(q.xt, V * l.cin);
+      UA(q.dyt, V * l.cout);
+    }
+    all.push_back(q);
   }
-  UA(u->target, V0 * 3);
+  // launches 0 .. 2 run over the layers of the transposed kernel, 3 .. 5 over all of them
+  for (const GradJob& q : all) (grad_rows(q.g) ? u->jobs : u->odd).push_back(q);
+  unsigned gr[6] = {}, ga[6] = {};
+  place_jobs(u->jobs, gr);
+  place_jobs(all, ga);
+  for (int k = 0; k < 6; ++k) u->grid[k] = k <= kDw ? gr[k] : ga[k];
+  GradJobs t{};
+  UA(u->djobs, 1); UA(u->dall, 1);
 #undef UA
+  t.n = (int)u->jobs.size();
+  std::copy(u->jobs.begin(), u->jobs.end(), t.j);
+  hipError_t e = hipMemcpy(u->djobs, &t, sizeof(t), hipMemcpyHostToDevice);
+  t.n = (int)all.size();
+  std::copy(all.begin(), all.end(), t.j);
+  if (e == hipSuccess) e = hipMemcpy(u->dall, &t, sizeof(t), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    free_acts(u);
+    return ufail(WLC_EHIP, "job table upload failed");
+  }
   return WLC_OK;
-}
-
-// the LDS-staged forward convolution (default; WLC_CONV_LDS=0 selects the direct one, for
-// measurements and tests)
-bool conv_lds_on() {
-  const char* e = std::getenv("WLC_CONV_LDS");
-  return !(e && e[0] == '0');
 }
 
 // launches shared by the network and the convolution test entry point (stream st)
 
-// y = conv(X) (+ bias); X has cin channels, Y cout (multiples of 16)
-int launch_conv_fwd(hipStream_t st, const bf16* X, const bf16* W, const float* bias, float* Y, Vol g, int cin,
-                    int cout) {
+// a convolution (adjoint: of packed flipped weights) of X with cin channels into cout (multiples
+// of 16).  Tile: the largest of 64 x 64, 64 x 32, 32 x 32, 16 x 32 and 16 x 16 voxels x output
+// channels per wave that divides cout and leaves a wave for every SIMD (1024); the smaller the
+// tile, the more steps in flight, since there the chain of steps is what takes the time (see
+// k_conv for the times of the tile this replaced)
+template <class Epi>
+int launch_conv(hipStream_t st, const bf16* X, const bf16* Wp, const bf16* zrow, Vol g, int cin, int cout,
+                const Epi& epi) {
   const long long V = g.voxels();
-  const int nt = cout % 64 == 0 ? 4 : (cout % 32 == 0 ? 2 : 1);
-  const dim3 grid(blocks(V, 64), cout / (16 * nt)), block(256);
-#define CONV_FWD(NT, KI) hipLaunchKernelGGL((k_conv_fwd<NT, KI>), grid, block, 0, st, X, W, bias, Y, g, cin, cout)
-#define CONV_FWD_L(NT) hipLaunchKernelGGL((k_conv_fwd_l<NT>), grid, block, 0, st, X, W, bias, Y, g, cin, cout)
-  if (cin % 32 == 0) {
-    if (conv_lds_on()) {
-      if (nt == 4) CONV_FWD_L(4); else if (nt == 2) CONV_FWD_L(2); else CONV_FWD_L(1);
-    } else {
-      if (nt == 4) CONV_FWD(4, 32); else if (nt == 2) CONV_FWD(2, 32); else CONV_FWD(1, 32);
-    }
-  } else {
-    if (nt == 4) CONV_FWD(4, 16); else if (nt == 2) CONV_FWD(2, 16); else CONV_FWD(1, 16);
-  }
-#undef CONV_FWD
-#undef CONV_FWD_L
+  const int nt = cout / 16;
+#define CONV(MT, NT, KI, D) \
+  hipLaunchKernelGGL((k_conv<MT, NT, KI, D, Epi>), dim3(blocks(V, 64 * (MT)), nt / (NT)), dim3(256), 0, st, X, Wp, zrow, g, cin, cout, epi)
+#define CONV_K(MT, NT, D) do { if (cin % 32 == 0) CONV(MT, NT, 32, D); else CONV(MT, NT, 16, D); } while (0)
+  auto waves = [&](int mt, int nn) { return (V + 16 * mt - 1) / (16 * mt) * (nt / nn); };
+  if (nt % 4 == 0 && waves(4, 4) >= 1024) CONV_K(4, 4, 3);
+  else if (nt % 2 == 0 && waves(4, 2) >= 1024) CONV_K(4, 2, 3);
+  else if (nt % 2 == 0 && waves(2, 2) >= 1024) CONV_K(2, 2, 3);
+  else if (nt % 2 == 0 && waves(1, 2) >= 1024) CONV_K(1, 2, 9);
+  else if (waves(4, 1) >= 1024) CONV_K(4, 1, 3);
+  else CONV_K(1, 1, 9);
+#undef CONV_K
+#undef CONV
   UCHK(hipGetLastError());
   return WLC_OK;
 }
 
-// dW [cout][27][cin] and db [cout] of one convolution (overwritten) from its input X
-// (channels-last bf16), the output gradient dYb (bf16) and dYf (FP32).  Scratch: xt >= V cin
-// and dyt >= V cout bf16, part >= wgrad_chunks(V) cout 27 cin floats, bpart >= kBiasParts cout.
-int launch_conv_wgrad(hipStream_t st, const bf16* X, const bf16* dYb, const float* dYf, Vol g, int cin, int cout,
-                      bf16* xt, bf16* dyt, float* part, float* bpart, float* dW, float* db) {
-  const long long V = g.voxels();
-  const long long nw = (long long)cout * 27 * cin;
-  const int nch = wgrad_chunks(V);
-  int nrun;
-  if (g.W % 8 == 0 && V % 32 == 0) {
-    const long long chunk = ((V + nch - 1) / nch + 31) / 32 * 32;
-    nrun = (int)((V + chunk - 1) / chunk);
-    hipLaunchKernelGGL(k_transpose, dim3(blocks(V, 32), blocks(cin, 32)), dim3(256), 0, st, X, xt, (int)V, cin);
-    hipLaunchKernelGGL(k_transpose, dim3(blocks(V, 32), blocks(cout, 32)), dim3(256), 0, st, dYb, dyt, (int)V, cout);
-    const int mc = cout % 32 == 0 ? 2 : 1, nc = cin % 32 == 0 ? 2 : 1;
-    const dim3 grid(27 * (cout / (16 * mc)) * (cin / (16 * nc)), nrun), block(64);
-#define CONV_DW(MC, NC) \
-  hipLaunchKernelGGL((k_conv_dw_t<MC, NC>), grid, block, 0, st, dyt, xt, part, g, cin, cout, (int)chunk)
-    if (mc == 2) {
-      if (nc == 2) CONV_DW(2, 2); else CONV_DW(2, 1);
-    } else {
-      if (nc == 2) CONV_DW(1, 2); else CONV_DW(1, 1);
-    }
-#undef CONV_DW
-  } else {
-    const long long chunk = ((V + nch - 1) / nch + 15) / 16 * 16;
-    nrun = (int)((V + chunk - 1) / chunk);
-    hipLaunchKernelGGL(k_conv_dw, dim3(27 * (cout / 16) * (cin / 16), nrun), dim3(64), 0, st, dYb, X, part, g, cin,
-                       cout, chunk);
-  }
-  UCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_sum_chunks, dim3(blocks(nw)), dim3(256), 0, st, part, dW, nw, nrun);
-  const int nbp = (int)std::min<long long>(kBiasParts, std::max<long long>(1, V / 256));
-  const int vchunk = (int)((V + nbp - 1) / nbp);
-  hipLaunchKernelGGL(k_bias_partial, dim3(nbp), dim3(256), 0, st, dYf, bpart, (int)V, cout, vchunk);
-  hipLaunchKernelGGL(k_bias_final, dim3(cout), dim3(256), 0, st, bpart, db, nbp, cout);
-  UCHK(hipGetLastError());
-  return WLC_OK;
-}
-
-int conv_forward(wlc_unet* u, const bf16* X, const bf16* W, const float* bias, float* Y, Vol g, int cin,
-                 int cout) {
-  return launch_conv_fwd(u->st, X, W, bias, Y, g, cin, cout);
-}
-
-// gradients of layer li: dW, db into u->g; dX (FP32, overwritten) when dX != nullptr
-int conv_backward(wlc_unet* u, const Layer& l, const bf16* X, float* dX) {
-  const int li = (int)(&l - u->layers.data());
-  const Vol g = u->vol(l.level);
-  const long long nw = (long long)l.cout * 27 * l.cin;
-  int rc = launch_conv_wgrad(u->st, X, u->dyb[li], u->dy[li], g, l.cin, l.cout, u->xt, u->dyt, u->part, u->bpart,
-                             u->g + l.woff, u->g + l.boff);
-  if (rc) return rc;
-  if (dX) {
-    hipLaunchKernelGGL(k_flip_weights, dim3(blocks(nw)), dim3(256), 0, u->st, u->pb + l.woff, u->wflip, l.cin, l.cout);
-    rc = conv_forward(u, u->dyb[li], u->wflip, nullptr, dX, g, l.cout, l.cin);
-    if (rc) return rc;
-  }
-  UCHK(hipGetLastError());
-  return WLC_OK;
-}
-
-int act(wlc_unet* u, int li, bf16* a, int Ct, int off) {
+template <class Epi>
+int conv(wlc_unet* u, int li, const bf16* X, const Epi& epi) {
   const Layer& l = u->layers[li];
-  const long long V = u->vol(l.level).voxels();
-  hipLaunchKernelGGL(k_act, dim3(blocks(V * l.cout)), dim3(256), 0, u->st, u->y[li], a, V, l.cout, Ct, off, l.relu);
-  UCHK(hipGetLastError());
-  return WLC_OK;
+  return launch_conv(u->st, X, u->wf + l.woff, u->zrow, u->vol(l.level), l.cin, l.cout, epi);
 }
-
-int relu_back(wlc_unet* u, int li, const float* da, int Ct, int off) {
+// gradient with respect to the input of layer li
+template <class Epi>
+int conv_back(wlc_unet* u, int li, const Epi& epi) {
   const Layer& l = u->layers[li];
-  const long long V = u->vol(l.level).voxels();
-  hipLaunchKernelGGL(k_relu_back, dim3(blocks(V * l.cout)), dim3(256), 0, u->st, u->y[li], da, u->dy[li],
-                     u->dyb[li], V, l.cout, Ct, off, l.relu);
-  UCHK(hipGetLastError());
-  return WLC_OK;
+  return launch_conv(u->st, u->dyb[li], u->wb + l.woff, u->zrow, u->vol(l.level), l.cout, l.cin, epi);
 }
 
 int forward(wlc_unet* u) {
-  auto& Ls = u->layers;
-  int rc;
-  auto C = [&](int li, const bf16* X) {
-    const Layer& l = Ls[li];
-    return conv_forward(u, X, u->pb + l.woff, u->p + l.boff, u->y[li], u->vol(l.level), l.cin, l.cout);
+  const Vol g0 = u->vol(0), g1 = u->vol(1), g2 = u->vol(2), g3 = u->vol(3);
+  auto act = [&](int li, bf16* a, int Ct, int off) {
+    return EpiAct<false>{a, u->p + u->layers[li].boff, Ct, off, u->vol(u->layers[li].level)};
   };
-  const Vol g1 = u->vol(1), g2 = u->vol(2), g3 = u->vol(3), g0 = u->vol(0);
-  if ((rc = C(0, u->x0)) || (rc = act(u, 0, u->a0a, 32, 0))) return rc;
-  if ((rc = C(1, u->a0a)) || (rc = act(u, 1, u->s0, 32, 0)) || (rc = act(u, 1, u->c0, 64, 32))) return rc;
-  hipLaunchKernelGGL(k_pool, dim3(blocks(g1.voxels() * 32)), dim3(256), 0, u->st, u->s0, u->p1, g1, 32);
-  if ((rc = C(2, u->p1)) || (rc = act(u, 2, u->a1a, 64, 0))) return rc;
-  if ((rc = C(3, u->a1a)) || (rc = act(u, 3, u->s1, 64, 0)) || (rc = act(u, 3, u->c1, 128, 64))) return rc;
-  hipLaunchKernelGGL(k_pool, dim3(blocks(g2.voxels() * 64)), dim3(256), 0, u->st, u->s1, u->p2, g2, 64);
-  if ((rc = C(4, u->p2)) || (rc = act(u, 4, u->a2a, 128, 0))) return rc;
-  if ((rc = C(5, u->a2a)) || (rc = act(u, 5, u->s2, 128, 0)) || (rc = act(u, 5, u->c2, 256, 128))) return rc;
-  hipLaunchKernelGGL(k_pool, dim3(blocks(g3.voxels() * 128)), dim3(256), 0, u->st, u->s2, u->p3, g3, 128);
-  if ((rc = C(6, u->p3)) || (rc = act(u, 6, u->bt, 128, 0))) return rc;
-  hipLaunchKernelGGL(k_up, dim3(blocks(g2.voxels() * 128)), dim3(256), 0, u->st, u->bt, u->c2, g2, 128, 256, 0);
-  if ((rc = C(7, u->c2)) || (rc = act(u, 7, u->d2, 64, 0))) return rc;
-  hipLaunchKernelGGL(k_up, dim3(blocks(g1.voxels() * 64)), dim3(256), 0, u->st, u->d2, u->c1, g1, 64, 128, 0);
-  if ((rc = C(8, u->c1)) || (rc = act(u, 8, u->d1, 32, 0))) return rc;
-  hipLaunchKernelGGL(k_up, dim3(blocks(g0.voxels() * 32)), dim3(256), 0, u->st, u->d1, u->c0, g0, 32, 64, 0);
-  if ((rc = C(9, u->c0)) || (rc = act(u, 9, u->d0, 32, 0))) return rc;
-  if ((rc = C(10, u->d0))) return rc;
+  auto up = [&](int li, bf16* a, int Ct) {
+    return EpiAct<true>{a, u->p + u->layers[li].boff, Ct, 0, u->vol(u->layers[li].level)};
+  };
+  auto pool = [&](const bf16* x, bf16* o, const Vol& go, int C) {
+    hipLaunchKernelGGL(k_pool, dim3(blocks(go.voxels() * (C / 4))), dim3(256), 0, u->st, x, o, go, C, 2 * C, C);
+  };
+  int rc;
+  if ((rc = conv(u, 0, u->x0, act(0, u->a0a, 32, 0)))) return rc;
+  if ((rc = conv(u, 1, u->a0a, act(1, u->c0, 64, 32)))) return rc;
+  pool(u->c0, u->p1, g1, 32);
+  if ((rc = conv(u, 2, u->p1, act(2, u->a1a, 64, 0)))) return rc;
+  if ((rc = conv(u, 3, u->a1a, act(3, u->c1, 128, 64)))) return rc;
+  pool(u->c1, u->p2, g2, 64);
+  if ((rc = conv(u, 4, u->p2, act(4, u->a2a, 128, 0)))) return rc;
+  if ((rc = conv(u, 5, u->a2a, act(5, u->c2, 256, 128)))) return rc;
+  pool(u->c2, u->p3, g3, 128);
+  if ((rc = conv(u, 6, u->p3, up(6, u->c2, 256)))) return rc;
+  if ((rc = conv(u, 7, u->c2, up(7, u->c1, 128)))) return rc;
+  if ((rc = conv(u, 8, u->c1, up(8, u->c0, 64)))) return rc;
+  if ((rc = conv(u, 9, u->c0, act(9, u->d0, 32, 0)))) return rc;
+  if ((rc = conv(u, 10, u->d0, EpiOut{u->y, u->p + u->layers[10].boff}))) return rc;
   UCHK(hipGetLastError());
   return WLC_OK;
 }
 
-// gradients of all parameters for the loss mse(y10[:, :3], target); *loss on the host
+// gradients of all parameters for the loss mse(y, target); *loss on the host
 int backward(wlc_unet* u, float* loss) {
-  auto& Ls = u->layers;
   const Vol g0 = u->vol(0), g1 = u->vol(1), g2 = u->vol(2), g3 = u->vol(3);
   const long long V0 = g0.voxels();
   int rc;
-  // zero the accumulated activation gradients
-  auto Z = [&](float* q, long long n) { return hipMemsetAsync(q, 0, sizeof(float) * (size_t)n, u->st); };
-  UCHK(Z(u->gs0, V0 * 32));
-  UCHK(Z(u->gs1, g1.voxels() * 64));
-  UCHK(Z(u->gs2, g2.voxels() * 128));
-  UCHK(Z(u->gbt, g3.voxels() * 128));
-  UCHK(Z(u->gd2, g2.voxels() * 64));
-  UCHK(Z(u->gd1, g1.voxels() * 32));
-  const int nparts = 256;
-  hipLaunchKernelGGL(k_mse, dim3(nparts), dim3(256), 0, u->st, u->y[10], u->target, u->dy[10], u->lpart, V0, 16, 3,
+  auto mask = [&](int li, const bf16* a) { return EpiMask{a, u->dy[li], u->dyb[li], u->layers[li].cout}; };
+  auto f32 = [&](float* q, int C) { return EpiF32{q, nullptr, C}; };
+  auto up_back = [&](int li, const float* gc, const bf16* c, const Vol& g, int C, int Ct) {
+    hipLaunchKernelGGL(k_up_back, dim3(blocks(g.voxels() * (C / 4))), dim3(256), 0, u->st, gc, c, u->dy[li], u->dyb[li],
+                       g, C, Ct);
+  };
+  auto skip_back = [&](int li, const float* gc, const float* gp, const bf16* c, const Vol& g, int C) {
+    hipLaunchKernelGGL(k_skip_back, dim3(blocks(g.voxels() * (C / 4))), dim3(256), 0, u->st, gc, gp, c, u->dy[li],
+                       u->dyb[li], g, C, 2 * C, C);
+  };
+  hipLaunchKernelGGL(k_mse, dim3(256), dim3(256), 0, u->st, u->y, u->target, u->dy[10], u->dyb[10], u->lpart, V0, 16, 3,
                      1.0f / (float)(V0 * 3));
-  hipLaunchKernelGGL(k_to_bf16, dim3(blocks(V0 * 16)), dim3(256), 0, u->st, u->dy[10], u->dyb[10], V0 * 16);
-  if ((rc = conv_backward(u, Ls[10], u->d0, u->gd0))) return rc;
-  if ((rc = relu_back(u, 9, u->gd0, 32, 0)) || (rc = conv_backward(u, Ls[9], u->c0, u->gc0))) return rc;
-  hipLaunchKernelGGL(k_up_back, dim3(blocks(g1.voxels() * 32)), dim3(256), 0, u->st, u->gc0, u->gd1, g1, 32, 64, 0);
-  hipLaunchKernelGGL(k_slice_add, dim3(blocks(V0 * 32)), dim3(256), 0, u->st, u->gc0, u->gs0, V0, 32, 64, 32);
-  if ((rc = relu_back(u, 8, u->gd1, 32, 0)) || (rc = conv_backward(u, Ls[8], u->c1, u->gc1))) return rc;
-  hipLaunchKernelGGL(k_up_back, dim3(blocks(g2.voxels() * 64)), dim3(256), 0, u->st, u->gc1, u->gd2, g2, 64, 128, 0);
-  hipLaunchKernelGGL(k_slice_add, dim3(blocks(g1.voxels() * 64)), dim3(256), 0, u->st, u->gc1, u->gs1, g1.voxels(), 64, 128, 64);
-  if ((rc = relu_back(u, 7, u->gd2, 64, 0)) || (rc = conv_backward(u, Ls[7], u->c2, u->gc2))) return rc;
-  hipLaunchKernelGGL(k_up_back, dim3(blocks(g3.voxels() * 128)), dim3(256), 0, u->st, u->gc2, u->gbt, g3, 128, 256, 0);
-  hipLaunchKernelGGL(k_slice_add, dim3(blocks(g2.voxels() * 128)), dim3(256), 0, u->st, u->gc2, u->gs2, g2.voxels(), 128, 256, 128);
-  if ((rc = relu_back(u, 6, u->gbt, 128, 0)) || (rc = conv_backward(u, Ls[6], u->p3, u->gp3))) return rc;
-  hipLaunchKernelGGL(k_pool_back, dim3(blocks(g2.voxels() * 128)), dim3(256), 0, u->st, u->gp3, u->gs2, g2, 128, 128, 0);
-  if ((rc = relu_back(u, 5, u->gs2, 128, 0)) || (rc = conv_backward(u, Ls[5], u->a2a, u->ga2a))) return rc;
-  if ((rc = relu_back(u, 4, u->ga2a, 128, 0)) || (rc = conv_backward(u, Ls[4], u->p2, u->gp2))) return rc;
-  hipLaunchKernelGGL(k_pool_back, dim3(blocks(g1.voxels() * 64)), dim3(256), 0, u->st, u->gp2, u->gs1, g1, 64, 64, 0);
-  if ((rc = relu_back(u, 3, u->gs1, 64, 0)) || (rc = conv_backward(u, Ls[3], u->a1a, u->ga1a))) return rc;
-  if ((rc = relu_back(u, 2, u->ga1a, 64, 0)) || (rc = conv_backward(u, Ls[2], u->p1, u->gp1))) return rc;
-  hipLaunchKernelGGL(k_pool_back, dim3(blocks(V0 * 32)), dim3(256), 0, u->st, u->gp1, u->gs0, g0, 32, 32, 0);
-  if ((rc = relu_back(u, 1, u->gs0, 32, 0)) || (rc = conv_backward(u, Ls[1], u->a0a, u->ga0a))) return rc;
-  if ((rc = relu_back(u, 0, u->ga0a, 32, 0)) || (rc = conv_backward(u, Ls[0], u->x0, nullptr))) return rc;
-  UCHK(hipGetLastError());
+  if ((rc = conv_back(u, 10, mask(9, u->d0)))) return rc;
+  if ((rc = conv_back(u, 9, f32(u->gc0, 64)))) return rc;
+  up_back(8, u->gc0, u->c0, g1, 32, 64);
+  if ((rc = conv_back(u, 8, f32(u->gc1, 128)))) return rc;
+  up_back(7, u->gc1, u->c1, g2, 64, 128);
+  if ((rc = conv_back(u, 7, f32(u->gc2, 256)))) return rc;
+  up_back(6, u->gc2, u->c2, g3, 128, 256);
+  if ((rc = conv_back(u, 6, f32(u->gp3, 128)))) return rc;
+  skip_back(5, u->gc2, u->gp3, u->c2, g2, 128);
+  if ((rc = conv_back(u, 5, mask(4, u->a2a)))) return rc;
+  if ((rc = conv_back(u, 4, f32(u->gp2, 64)))) return rc;
+  skip_back(3, u->gc1, u->gp2, u->c1, g1, 64);
+  if ((rc = conv_back(u, 3, mask(2, u->a1a)))) return rc;
+  if ((rc = conv_back(u, 2, f32(u->gp1, 32)))) return rc;
+  skip_back(1, u->gc0, u->gp1, u->c0, g0, 32);
+  if ((rc = conv_back(u, 1, mask(0, u->a0a)))) return rc;
+  if ((rc = launch_grads(u->st, u->dall, u->djobs, !u->jobs.empty(), u->odd, u->grid))) return rc;
   float lp[256];
   UCHK(hipMemcpyAsync(lp, u->lpart, sizeof(lp), hipMemcpyDeviceToHost, u->st));
   UCHK(hipStreamSynchronize(u->st));
@@ -918,20 +1021,22 @@ int backward(wlc_unet* u, float* loss) {
   return WLC_OK;
 }
 
-// input [B][n^3][11] (host FP32) -> bf16 [B n^3][16]; targets [B][n^3][3]
+// input [B][n^3][11] (host FP32), converted on the device; targets [B][n^3][3].  The caller waits
+// for the stream before it returns (the host arrays are read until then).
 int upload(wlc_unet* u, const float* x, const float* t) {
   const long long V = u->vol(0).voxels();
-  if (x) {
-    std::vector<bf16> h((size_t)V * 16, 0);
-    for (long long v = 0; v < V; ++v)
-      for (int c = 0; c < 11; ++c) h[(size_t)v * 16 + c] = f2bf(x[v * 11 + c]);
-    UCHK(hipMemcpyAsync(u->x0, h.data(), sizeof(bf16) * h.size(), hipMemcpyHostToDevice, u->st));
-    UCHK(hipStreamSynchronize(u->st));
-  }
-  if (t) {
-    UCHK(hipMemcpyAsync(u->target, t, sizeof(float) * (size_t)V * 3, hipMemcpyHostToDevice, u->st));
-    UCHK(hipStreamSynchronize(u->st));
-  }
+  UCHK(hipMemcpyAsync(u->xin, x, sizeof(float) * (size_t)V * 11, hipMemcpyHostToDevice, u->st));
+  hipLaunchKernelGGL(k_input, dim3(blocks(V * 16)), dim3(256), 0, u->st, u->xin, u->x0, V);
+  if (t) UCHK(hipMemcpyAsync(u->target, t, sizeof(float) * (size_t)V * 3, hipMemcpyHostToDevice, u->st));
+  UCHK(hipGetLastError());
+  return WLC_OK;
+}
+
+// the packed bf16 weights from the master copy
+int repack(wlc_unet* u) {
+  hipLaunchKernelGGL(k_pack, dim3(blocks(u->np)), dim3(256), 0, u->st, u->p, u->pack, u->wf, u->wb, u->np);
+  UCHK(hipGetLastError());
+  UCHK(hipStreamSynchronize(u->st));
   return WLC_OK;
 }
 
@@ -957,11 +1062,12 @@ int wlc_unet_create(int n, int batch, unsigned long long seed, wlc_unet** out) {
   u->np = last.boff + last.cout;
   int rc;
 #define UA(ptr, cnt) if ((rc = ualloc(u->allocs, &(ptr), (cnt)))) { unet_free(u); return rc; }
-  UA(u->p, u->np); UA(u->m, u->np); UA(u->v, u->np); UA(u->g, u->np); UA(u->pb, u->np); UA(u->mask, u->np);
-  long long maxw = 0;
-  for (const Layer& l : u->layers) maxw = std::max(maxw, (long long)l.cout * 27 * l.cin);
-  UA(u->wflip, maxw);
+  UA(u->p, u->np); UA(u->m, u->np); UA(u->v, u->np); UA(u->g, u->np); UA(u->mask, u->np);
+  UA(u->wf, u->np); UA(u->wb, u->np); UA(u->zrow, 64);
 #undef UA
+  u->pack.n = (int)u->layers.size();
+  for (size_t li = 0; li < u->layers.size(); ++li)
+    u->pack.l[li] = PackLayer{u->layers[li].woff, u->layers[li].cin, u->layers[li].cout};
   if ((rc = alloc_acts(u, n, batch))) {
     unet_free(u);
     return rc;
@@ -986,13 +1092,14 @@ int wlc_unet_create(int n, int batch, unsigned long long seed, wlc_unet** out) {
         }
     for (int co = 0; co < l.cout; ++co) hm[l.boff + co] = co < l.cout_real ? 1 : 0;
   }
-  std::vector<bf16> hb((size_t)u->np);
-  for (size_t i = 0; i < hb.size(); ++i) hb[i] = f2bf(hp[i]);
   if (hipMemcpy(u->p, hp.data(), sizeof(float) * hp.size(), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(u->pb, hb.data(), sizeof(bf16) * hb.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(u->mask, hm.data(), hm.size(), hipMemcpyHostToDevice) != hipSuccess) {
     unet_free(u);
     return ufail(WLC_EHIP, "parameter upload failed");
+  }
+  if ((rc = repack(u))) {
+    unet_free(u);
+    return rc;
   }
   *out = u;
   return WLC_OK;
@@ -1031,14 +1138,9 @@ int wlc_unet_forward(wlc_unet* u, const float* x, float* y) {
   UCHK(hipSetDevice(u->device));
   int rc = upload(u, x, nullptr);
   if (rc || (rc = forward(u))) return rc;
-  if (y) {
-    const long long V = u->vol(0).voxels();
-    std::vector<float> h((size_t)V * 16);
-    UCHK(hipMemcpyAsync(h.data(), u->y[10], sizeof(float) * h.size(), hipMemcpyDeviceToHost, u->st));
-    UCHK(hipStreamSynchronize(u->st));
-    for (long long v = 0; v < V; ++v)
-      for (int c = 0; c < 3; ++c) y[v * 3 + c] = h[(size_t)v * 16 + c];
-  }
+  if (y)
+    UCHK(hipMemcpyAsync(y, u->y, sizeof(float) * 3 * (size_t)u->vol(0).voxels(), hipMemcpyDeviceToHost, u->st));
+  UCHK(hipStreamSynchronize(u->st));
   return WLC_OK;
 }
 
@@ -1056,8 +1158,8 @@ int wlc_unet_adam(wlc_unet* u, float lr) {
   u->adam_t += 1;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.f - std::pow(b1, (float)u->adam_t), c2 = 1.f - std::pow(b2, (float)u->adam_t);
-  hipLaunchKernelGGL(k_adam, dim3(blocks(u->np)), dim3(256), 0, u->st, u->p, u->m, u->v, u->g, u->pb, u->mask,
-                     u->np, lr, b1, b2, eps, c1, c2);
+  hipLaunchKernelGGL(k_adam, dim3(blocks(u->np)), dim3(256), 0, u->st, u->p, u->m, u->v, u->g, u->pack,
+                     u->wf, u->wb, u->mask, u->np, lr, b1, b2, eps, c1, c2);
   UCHK(hipGetLastError());
   UCHK(hipStreamSynchronize(u->st));
   return WLC_OK;
@@ -1082,10 +1184,7 @@ int wlc_unet_set_params(wlc_unet* u, const float* in) {
   if (!u || !in) return ufail(WLC_EINVAL, "NULL argument");
   UCHK(hipSetDevice(u->device));
   UCHK(hipMemcpy(u->p, in, sizeof(float) * (size_t)u->np, hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_to_bf16, dim3(blocks(u->np)), dim3(256), 0, u->st, u->p, u->pb, u->np);
-  UCHK(hipGetLastError());
-  UCHK(hipStreamSynchronize(u->st));
-  return WLC_OK;
+  return repack(u);
 }
 
 // Test hook: one convolution and its gradients on host arrays (x [V][cin], w [cout][27][cin],
@@ -1099,45 +1198,59 @@ int wlc_test_conv3d(int B, int D, int H, int W, int cin, int cout, const float* 
   const Vol g{B, D, H, W};
   const long long V = g.voxels(), nw = (long long)cout * 27 * cin;
   if (V * std::max(cin, cout) >= (1LL << 31)) return ufail(WLC_EINVAL, "tensor too large");
-  const int nch = wgrad_chunks(V);
-  std::vector<bf16> hx((size_t)(V * cin)), hw((size_t)nw), hdy((size_t)(V * cout));
+  std::vector<bf16> hx((size_t)(V * cin)), hdy((size_t)(V * cout));
   for (size_t i = 0; i < hx.size(); ++i) hx[i] = f2bf(x[i]);
-  for (size_t i = 0; i < hw.size(); ++i) hw[i] = f2bf(w[i]);
   for (size_t i = 0; i < hdy.size(); ++i) hdy[i] = f2bf(dy[i]);
-  bf16 *dX = nullptr, *dW = nullptr, *dDY = nullptr, *dWf = nullptr, *dXT = nullptr, *dDYT = nullptr;
-  float *dB = nullptr, *dYo = nullptr, *dDX = nullptr, *dDW = nullptr, *dDB = nullptr, *dPart = nullptr,
-        *dDYf = nullptr, *dBpart = nullptr;
+  GradJob q = grad_job(g, cin, cout);
+  bf16 *dX = nullptr, *dDY = nullptr, *dF = nullptr, *dBk = nullptr, *dZ = nullptr;
+  float *dW = nullptr, *dB = nullptr, *dYo = nullptr, *dDX = nullptr, *dDYf = nullptr;
+  GradJobs* dJ = nullptr;
   hipError_t e = hipSuccess;
-  auto M = [&](void** q, size_t bytes) { if (e == hipSuccess) e = hipMalloc(q, bytes); };
-  M((void**)&dX, sizeof(bf16) * hx.size()); M((void**)&dW, sizeof(bf16) * nw); M((void**)&dDY, sizeof(bf16) * hdy.size());
-  M((void**)&dWf, sizeof(bf16) * nw); M((void**)&dB, sizeof(float) * cout); M((void**)&dYo, sizeof(float) * V * cout);
-  M((void**)&dDX, sizeof(float) * V * cin); M((void**)&dDW, sizeof(float) * nw); M((void**)&dDB, sizeof(float) * cout);
-  M((void**)&dPart, sizeof(float) * nw * nch); M((void**)&dDYf, sizeof(float) * V * cout);
-  M((void**)&dXT, sizeof(bf16) * hx.size()); M((void**)&dDYT, sizeof(bf16) * hdy.size());
-  M((void**)&dBpart, sizeof(float) * kBiasParts * cout);
+  auto M = [&](void** p, size_t bytes) { if (e == hipSuccess) e = hipMalloc(p, bytes); };
+  M((void**)&dX, sizeof(bf16) * hx.size()); M((void**)&dDY, sizeof(bf16) * hdy.size());
+  M((void**)&dF, sizeof(bf16) * nw); M((void**)&dBk, sizeof(bf16) * nw); M((void**)&dZ, 128);
+  M((void**)&dW, sizeof(float) * nw); M((void**)&dB, sizeof(float) * cout); M((void**)&dYo, sizeof(float) * V * cout);
+  M((void**)&dDX, sizeof(float) * V * cin); M((void**)&dDYf, sizeof(float) * V * cout); M((void**)&dJ, sizeof(GradJobs));
+  M((void**)&q.xt, sizeof(bf16) * hx.size()); M((void**)&q.dyt, sizeof(bf16) * hdy.size());
+  M((void**)&q.part, sizeof(float) * part_floats(q)); M((void**)&q.bpart, sizeof(float) * q.nbp * cout);
+  M((void**)&q.dW, sizeof(float) * nw); M((void**)&q.db, sizeof(float) * cout);
   if (e == hipSuccess) e = hipMemcpy(dX, hx.data(), sizeof(bf16) * hx.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(dW, hw.data(), sizeof(bf16) * nw, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(dW, w, sizeof(float) * nw, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dDY, hdy.data(), sizeof(bf16) * hdy.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dB, b, sizeof(float) * cout, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dDYf, dy, sizeof(float) * V * cout, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemset(dZ, 0, 128);
+  q.X = dX;
+  q.dYb = dDY;
+  q.dYf = dDYf;
+  std::vector<GradJob> one{q};
+  unsigned grid[6];
+  place_jobs(one, grid);
+  GradJobs J{};
+  J.n = 1;
+  J.j[0] = one[0];
+  if (e == hipSuccess) e = hipMemcpy(dJ, &J, sizeof(J), hipMemcpyHostToDevice);
   int rc = WLC_OK;
   if (e == hipSuccess) {
-    rc = launch_conv_fwd(nullptr, dX, dW, dB, dYo, g, cin, cout);
-    if (!rc) rc = launch_conv_wgrad(nullptr, dX, dDY, dDYf, g, cin, cout, dXT, dDYT, dPart, dBpart, dDW, dDB);
-    if (!rc) {
-      hipLaunchKernelGGL(k_flip_weights, dim3(blocks(nw)), dim3(256), 0, nullptr, dW, dWf, cin, cout);
-      rc = launch_conv_fwd(nullptr, dDY, dWf, nullptr, dDX, g, cout, cin);
-    }
+    PackTable T{};
+    T.n = 1;
+    T.l[0] = PackLayer{0, cin, cout};
+    hipLaunchKernelGGL(k_pack, dim3(blocks(nw)), dim3(256), 0, nullptr, dW, T, dF, dBk, nw);
+    rc = launch_conv(nullptr, dX, dF, dZ, g, cin, cout, EpiF32{dYo, dB, cout});
+    const bool rows = grad_rows(g);
+    if (!rc) rc = launch_grads(nullptr, dJ, dJ, rows, rows ? std::vector<GradJob>{} : one, grid);
+    if (!rc) rc = launch_conv(nullptr, dDY, dBk, dZ, g, cout, cin, EpiF32{dDX, nullptr, cin});
     if (!rc) e = hipGetLastError();
   }
   if (!rc && e == hipSuccess) e = hipDeviceSynchronize();
   if (!rc && e == hipSuccess) e = hipMemcpy(y, dYo, sizeof(float) * V * cout, hipMemcpyDeviceToHost);
   if (!rc && e == hipSuccess) e = hipMemcpy(dx, dDX, sizeof(float) * V * cin, hipMemcpyDeviceToHost);
-  if (!rc && e == hipSuccess) e = hipMemcpy(dw, dDW, sizeof(float) * nw, hipMemcpyDeviceToHost);
-  if (!rc && e == hipSuccess) e = hipMemcpy(db, dDB, sizeof(float) * cout, hipMemcpyDeviceToHost);
-  for (void* q : {(void*)dX, (void*)dW, (void*)dDY, (void*)dWf, (void*)dB, (void*)dYo, (void*)dDX, (void*)dDW,
-                  (void*)dDB, (void*)dPart, (void*)dDYf, (void*)dXT, (void*)dDYT, (void*)dBpart})
-    if (q) (void)hipFree(q);
+  if (!rc && e == hipSuccess) e = hipMemcpy(dw, q.dW, sizeof(float) * nw, hipMemcpyDeviceToHost);
+  if (!rc && e == hipSuccess) e = hipMemcpy(db, q.db, sizeof(float) * cout, hipMemcpyDeviceToHost);
+  for (void* p : {(void*)dX, (void*)dDY, (void*)dF, (void*)dBk, (void*)dZ, (void*)dW, (void*)dB, (void*)dYo, (void*)dDX,
+                  (void*)dDYf, (void*)dJ, (void*)q.xt, (void*)q.dyt, (void*)q.part, (void*)q.bpart, (void*)q.dW,
+                  (void*)q.db})
+    if (p) (void)hipFree(p);
   if (rc) return rc;
   if (e != hipSuccess) return ufail(WLC_EHIP, std::string("test conv3d: ") + hipGetErrorString(e));
   return WLC_OK;
