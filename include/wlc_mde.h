@@ -134,7 +134,8 @@ int wlc_mde_set_spectrum_fp32(wlc_handle* h, int on);
  * itself (the density terms still overlap the backward sweep).  wlc_mde_get_timing returns,
  * for kernel k in {0: rhs+xy FFT, 1: z FFT+solve, 2: inverse xy FFT, 3: density
  * accumulation, 4: inverse xy FFT of one step fused with rhs+xy FFT of the next}, the
- * summed milliseconds and the launch count since enabling.
+ * summed milliseconds and the launch count since enabling (for kernel 3 the contour points
+ * added: one launch covers a run of them).
  * No counterpart in the reference (which times only the whole run, SCFT_main.f90:51-55). */
 int wlc_mde_set_timing(wlc_handle* h, int enable);
 int wlc_mde_get_timing(wlc_handle* h, double* ms, long long* count, int nkernels);
@@ -161,11 +162,12 @@ int wlc_mde_step(wlc_handle* h, int dir, int s, const double* const hist_dev[3],
  * reference; for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  The chain is described by p
  * (validated as in wlc_mde_create), the work is queued on `stream` (a hipStream_t, NULL =
- * the null stream).  The scratch (FFT twiddles, one zero field, the half spectrum of the
- * target's harmonics) lives in a fixed 128 MiB device array that each GPU the library runs
- * on holds until the process ends; a step whose zero field plus half spectrum exceeds it
- * (e.g. 64^3 with Lmax above 6) is rejected with WLC_EINVAL.  Every call on one GPU shares
- * that array, so calls that overlap on one GPU (different streams or threads) race. */
+ * the null stream).  The scratch (one zero field, the half spectrum of the target's
+ * harmonics) lives in a fixed 128 MiB device array that each GPU the library runs on holds
+ * until the process ends; the FFT twiddles of every accepted edge are compiled in; a step
+ * whose zero field plus half spectrum exceeds the array (e.g. 64^3 with Lmax above 6) is
+ * rejected with WLC_EINVAL.  Every call on one GPU shares that array, so calls that overlap
+ * on one GPU (different streams or threads) race. */
 int wlc_mde_step_noalloc(const wlc_params* p, int dir, int s, const double* const hist_dev[3],
                          const double* w_dev, double* out_dev, void* stream);
 

@@ -22,6 +22,7 @@ FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     # keep hipcc from emitting packed-FP32 instructions
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    f"-I{BUILD}",
 ]
 
 
@@ -68,7 +69,7 @@ def _compile(unit):
 
 
 def gen_tables():
-    """Regenerate csrc/wlc_tables.inc from the host set-up code (g++)."""
+    """Regenerate csrc/wlc_tables.inc and _build/wlc_twiddles.inc from the host set-up code (g++)."""
     exe = os.path.join(BUILD, "gen_tables")
     cxx = shutil.which("g++") or "g++"
     cmd = [cxx, "-O2", "-std=c++17", "-o", exe, os.path.join(CSRC, "gen_tables.cpp"),
@@ -77,9 +78,12 @@ def gen_tables():
     if r.returncode != 0:
         raise RuntimeError(f"gen_tables build failed:\n{r.stderr[-4000:]}")
     out = os.path.join(BUILD, "wlc_tables.inc")
-    r = subprocess.run([exe, out], capture_output=True, text=True)
+    tw = os.path.join(BUILD, "wlc_twiddles.inc")
+    r = subprocess.run([exe, out, tw + ".new"], capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"gen_tables failed:\n{r.stderr}")
+    if not os.path.exists(tw) or open(tw).read() != open(tw + ".new").read():
+        os.replace(tw + ".new", tw)
     dst = os.path.join(CSRC, "wlc_tables.inc")
     new = open(out).read()
     if not os.path.exists(dst) or open(dst).read() != new:

@@ -818,44 +818,56 @@ int ensure_tables(int device) {
 
 // ---------------------------------------------------------------------------------------
 // Scratch of wlc_mde_step_noalloc: a fixed device array, one copy per GPU, held until the
-// process ends.  Layout: FFT twiddles of the three axes at offset 0 (3 x 256 complex), one
-// zero field at kScrZero, the half spectrum at kScrZero + the zero field rounded up to
-// 256 bytes.  The host reaches each device's copy only through the address
+// process ends.  Layout: one zero field at kScrZero, the half spectrum at kScrZero + the zero
+// field rounded up to 256 bytes.  The FFT twiddles of every accepted edge are compiled in
+// (kTwiddles).  The host reaches each device's copies only through the addresses
 // hipGetSymbolAddress returns on that device.
 constexpr size_t kScratchBytes = size_t(128) << 20;
 constexpr size_t kScrZero = 64 << 10;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
+#include "wlc_twiddles.inc"
 
+struct DeviceArrays {
+  unsigned char* scr = nullptr;
+  const double2* tw = nullptr;
+};
 std::mutex g_scr_mu;
-std::vector<unsigned char*> g_scr_ptr;  // per device, nullptr until resolved
+std::vector<DeviceArrays> g_scr;  // per device, null until resolved
 
-int scratch_on(int device, unsigned char** out) {
+int scratch_on(int device, DeviceArrays* out) {
   std::lock_guard<std::mutex> lk(g_scr_mu);
-  if ((int)g_scr_ptr.size() <= device) g_scr_ptr.resize(device + 1, nullptr);
-  if (!g_scr_ptr[device]) {
-    void* ptr = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !ptr)
+  if ((int)g_scr.size() <= device) g_scr.resize(device + 1);
+  if (!g_scr[device].scr) {
+    void *ptr = nullptr, *tw = nullptr;
+    hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+    if (e == hipSuccess) e = hipGetSymbolAddress(&tw, HIP_SYMBOL(kTwiddles));
+    if (e != hipSuccess || !ptr || !tw)
       return fail(WLC_EHIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-    g_scr_ptr[device] = static_cast<unsigned char*>(ptr);
+    g_scr[device].scr = static_cast<unsigned char*>(ptr);
+    g_scr[device].tw = static_cast<const double2*>(tw);
   }
-  *out = g_scr_ptr[device];
+  *out = g_scr[device];
   return WLC_OK;
 }
 
-// host twiddle tables per edge, kept for the life of the process (the source of the
-// per-call upload stays valid however the runtime stages the copy)
-std::mutex g_tw_mu;
-std::vector<std::vector<double2>> g_tw_host(257);
-
-const double2* host_twiddles(const wlc::AxisPlan& pl) {
-  std::lock_guard<std::mutex> lk(g_tw_mu);
-  auto& v = g_tw_host[pl.n];
-  if (v.empty()) {
-    v.resize(pl.n);
-    for (int t = 0; t < pl.n; ++t) v[t] = make_double2(pl.tw[2 * t], pl.tw[2 * t + 1]);
-  }
-  return v.data();
+// radices of each edge and where its twiddles are (edges were validated)
+struct EdgePlan {
+  int npass = 0, radix[8] = {}, off = 0;
+};
+const EdgePlan& edge_plan(int n) {
+  static const std::vector<EdgePlan> plans = [] {
+    std::vector<EdgePlan> v(257);
+    for (size_t k = 0; k < sizeof(kTwEdge) / sizeof(kTwEdge[0]); ++k) {
+      wlc::AxisPlan pl;
+      (void)wlc::make_axis_plan(kTwEdge[k], &pl);
+      EdgePlan& e = v[kTwEdge[k]];
+      e.npass = pl.npass;
+      for (int i = 0; i < 8 && i < pl.npass; ++i) e.radix[i] = pl.radix[i];
+      e.off = kTwOff[k];
+    }
+    return v;
+  }();
+  return plans[n];
 }
 
 }  // namespace
@@ -1392,22 +1404,15 @@ int wlc_mde_step_noalloc(const wlc_params* p, int dir, int s, const double* cons
   if (kScrZero + zero_bytes + spec_bytes > kScratchBytes)
     return fail(WLC_EINVAL, "step too large for the fixed scratch (" + std::to_string(kScratchBytes >> 20) +
                                 " MiB: one zero field plus the half spectrum of the target's harmonics)");
-  wlc::AxisPlan plan[3];
   const int edges[3] = {p->nx, p->ny, p->nz};
-  for (int a = 0; a < 3; ++a) {
-    std::string err = wlc::make_axis_plan(edges[a], &plan[a]);
-    if (!err.empty()) return fail(WLC_EINVAL, err);
-    if (plan[a].npass > 8) return fail(WLC_EINVAL, "too many FFT passes");
-  }
   int device = 0;
   HIPCHK(hipGetDevice(&device));
   if ((rc = ensure_tables(device))) return rc;
-  unsigned char* scr = nullptr;
-  if ((rc = scratch_on(device, &scr))) return rc;
+  DeviceArrays da;
+  if ((rc = scratch_on(device, &da))) return rc;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  double2* tw = reinterpret_cast<double2*>(scr);
-  double* zero = reinterpret_cast<double*>(scr + kScrZero);
-  double2* spec = reinterpret_cast<double2*>(scr + kScrZero + zero_bytes);
+  double* zero = reinterpret_cast<double*>(da.scr + kScrZero);
+  double2* spec = reinterpret_cast<double2*>(da.scr + kScrZero + zero_bytes);
   wlc::Geom g{};
   g.nx = p->nx; g.ny = p->ny; g.nz = p->nz; g.nxh = nxh;
   g.nt = wlc::kx_tiles(nxh);
@@ -1416,15 +1421,20 @@ int wlc_mde_step_noalloc(const wlc_params* p, int dir, int s, const double* cons
   g.hs = (long long)p->nz * g.zs;
   wlc::AxisDev* ax[3] = {&g.ax, &g.ay, &g.az};
   for (int a = 0; a < 3; ++a) {
-    ax[a]->n = plan[a].n;
-    ax[a]->npass = plan[a].npass;
-    for (int i = 0; i < 8; ++i) ax[a]->radix[i] = i < plan[a].npass ? plan[a].radix[i] : 0;
-    ax[a]->tw = tw + 256 * a;
-    HIPCHK(hipMemcpyAsync(tw + 256 * a, host_twiddles(plan[a]), sizeof(double2) * plan[a].n,
-                          hipMemcpyHostToDevice, st));
+    const EdgePlan& e = edge_plan(edges[a]);
+    ax[a]->n = edges[a];
+    ax[a]->npass = e.npass;
+    for (int i = 0; i < 8; ++i) ax[a]->radix[i] = e.radix[i];
+    ax[a]->tw = da.tw + e.off;
   }
-  // the array keeps the previous call's contents: the zero field is cleared every call
-  HIPCHK(wlc::launch_fill(zero, 0.0, (long long)field, st));
+  // the zero field is read only where a history slice is missing or holds fewer harmonics than
+  // the target; the array keeps the previous call's contents, so it is cleared then
+  bool reads_zero = order < 3;
+  for (int j = 0; j < order; ++j) {
+    const int hl = p->Lmax[params_block_of(*p, s - dir * (j + 1))];
+    reads_zero = reads_zero || hl < p->Lmax[blk];
+  }
+  if (reads_zero) HIPCHK(wlc::launch_fill(zero, 0.0, (long long)field, st));
   return queue_dense_step(*p, g, dir, s, order, hist_dev, w_dev, out_dev, spec, zero, st);
 }
 
