@@ -50,27 +50,19 @@ __device__ __forceinline__ void plane_of_block(int nz, int& z, int& grp) {
 
 // x then y forward transform of the packed plane in LDS (sizes compile-time when
 // NX, NY are nonzero)
-// The compile-time planes are square and keep their twiddles in LDS behind the plane: a pass's
-// first read of the table in memory costs as long as the pass.
-template <int NX, int NY>
-__device__ __forceinline__ double2* ct_tw(double2* lds) {
-  static_assert(NX == NY, "one table for both axes");
-  constexpr int n = NY * (NX / 2 + 1);
-  return lds + n + n / 8 + 1;
-}
 template <int NX, int NY, int MAXE>
 __device__ __forceinline__ void plane_fft_x(double2* lds, const Geom& g) {
-  if constexpr (NX > 0) FftCt<-1, NX, NY / 2, 1, NX, kThreads, true>::run(lds, ct_tw<NX, NY>(lds));
+  if constexpr (NX > 0) FftCt<-1, NX, NY / 2, 1, NX, kThreads, true>::run(lds, g.ax.tw);
   else fft_axis<-1, MAXE>(lds, g.ax, g.ny / 2, 1, g.nx);
 }
 template <int NX, int NY, int MAXE, int DIR>
 __device__ __forceinline__ void plane_fft_y(double2* lds, const Geom& g) {
-  if constexpr (NX > 0) FftCt<DIR, NY, NX / 2 + 1, NX / 2 + 1, 1, kThreads, true>::run(lds, ct_tw<NX, NY>(lds));
+  if constexpr (NX > 0) FftCt<DIR, NY, NX / 2 + 1, NX / 2 + 1, 1, kThreads, true>::run(lds, g.ay.tw);
   else fft_axis<DIR, MAXE>(lds, g.ay, g.nxh, g.nxh, 1);
 }
 template <int NX, int NY, int MAXE>
 __device__ __forceinline__ void plane_ifft_x(double2* lds, const Geom& g) {
-  if constexpr (NX > 0) FftCt<+1, NX, NY / 2, 1, NX, kThreads, true>::run(lds, ct_tw<NX, NY>(lds));
+  if constexpr (NX > 0) FftCt<+1, NX, NY / 2, 1, NX, kThreads, true>::run(lds, g.ax.tw);
   else fft_axis<+1, MAXE>(lds, g.ax, g.ny / 2, 1, g.nx);
 }
 
@@ -210,43 +202,15 @@ __device__ __forceinline__ double bdf_rhs(double q1, double q2, double q3, doubl
   return __builtin_fma(-(ds * w), u, t);
 }
 
-// History and field values of up to kPairs x pairs per thread.
-struct HistPairs {
-  double2 v2[kPairs], v3[kPairs], w[kPairs];
-};
-
-// loads of history slices 1 and 2 and w for the pairs base + c kThreads + thread (a zero history
-// plane is read from the zero field, so the loads depend only on the pair being in the plane)
-template <int ORDER>
-__device__ __forceinline__ void load_pairs(HistPairs& h, const Geom& g, const RhsArgs& a, int i, long long plane,
-                                           int base, int tot2) {
-  const double2* w2 = reinterpret_cast<const double2*>(a.w + plane);
-  const bool u2 = ORDER >= 2 && i < a.hM[1], u3 = ORDER >= 3 && i < a.hM[2];
-  const double2* q2 = reinterpret_cast<const double2*>(u2 ? a.h[1] + i * g.hs + plane : a.zero + plane);
-  const double2* q3 = reinterpret_cast<const double2*>(u3 ? a.h[2] + i * g.hs + plane : a.zero + plane);
-#pragma unroll
-  for (int c = 0; c < kPairs; ++c) {
-    const int e = base + c * kThreads + threadIdx.x;
-    h.v2[c] = h.v3[c] = h.w[c] = make_double2(0.0, 0.0);
-    if (e < tot2) {
-      if (ORDER >= 2) h.v2[c] = q2[e];
-      if (ORDER >= 3) h.v3[c] = q3[e];
-      h.w[c] = w2[e];
-    }
-  }
-}
-
 // BDF right-hand side of harmonic i on z-plane `plane` into the packed LDS plane:
 //   P = a0 q1 + a1 q2 + a2 q3 - ds w (b0 q1 + b1 q2 + b2 q3)
 // q1 is read from history slice 0, or (FROM_LDS) taken from the packed LDS plane times
 // `scale` (the freshly inverted q(s), also stored to `out` when `store`).  have1 = 0
-// makes q1 zero; rhs = 0 skips the right-hand side (store only).  `pre`: the history and field
-// of the first kPairs pairs, loaded by the caller (nullptr: loaded here).
+// makes q1 zero; rhs = 0 skips the right-hand side (store only).
 template <int NX, int NY, int ORDER, bool FROM_LDS>
 __device__ __forceinline__ void rhs_to_lds(double* pk, const Geom& g, const RhsArgs& a, int i,
                                            long long plane, bool have1, double scale,
-                                           double* __restrict__ out, bool store, bool rhs,
-                                           const HistPairs* pre = nullptr) {
+                                           double* __restrict__ out, bool store, bool rhs) {
   const int nx = NX ? NX : g.nx, ny = NY ? NY : g.ny;
   const long long hs = g.hs;
   const int tot2 = (nx * ny) >> 1;  // nx is even: x pairs (2p, 2p+1) share a row
@@ -254,22 +218,31 @@ __device__ __forceinline__ void rhs_to_lds(double* pk, const Geom& g, const RhsA
   const double a0 = a.a[0], a1 = a.a[1], a2 = a.a[2];
   const double b0 = a.b[0], b1 = a.b[1], b2 = a.b[2];
   const bool u1 = have1 && (FROM_LDS || i < a.hM[0]);
+  const bool u2 = rhs && ORDER >= 2 && i < a.hM[1];
+  const bool u3 = rhs && ORDER >= 3 && i < a.hM[2];
+  // a zero history plane is read from the zero field: the loads depend only on `in`
+  const double2* w2 = reinterpret_cast<const double2*>(a.w + plane);
   const double2* q1 =
       reinterpret_cast<const double2*>(u1 && !FROM_LDS ? a.h[0] + i * hs + plane : a.zero + plane);
+  const double2* q2 = reinterpret_cast<const double2*>(u2 ? a.h[1] + i * hs + plane : a.zero + plane);
+  const double2* q3 = reinterpret_cast<const double2*>(u3 ? a.h[2] + i * hs + plane : a.zero + plane);
   double2* o2 = reinterpret_cast<double2*>(out);
   const double2 zero = make_double2(0.0, 0.0);
   for (int base = 0; base < tot2; base += kPairs * kThreads) {
-    double2 v1[kPairs];
-    HistPairs h;
+    double2 v1[kPairs], v2[kPairs], v3[kPairs], ww[kPairs];
 #pragma unroll
     for (int c = 0; c < kPairs; ++c) {
       const int e = base + c * kThreads + threadIdx.x;
-      v1[c] = zero;
-      if (!FROM_LDS && e < tot2) v1[c] = q1[e];
-    }
-    if (rhs) {
-      if (pre) h = *pre;
-      else load_pairs<ORDER>(h, g, a, i, plane, base, tot2);
+      const bool in = e < tot2;
+      v1[c] = v2[c] = v3[c] = ww[c] = zero;
+      if (in) {
+        if (!FROM_LDS) v1[c] = q1[e];
+        if (rhs) {
+          if (ORDER >= 2) v2[c] = q2[e];
+          if (ORDER >= 3) v3[c] = q3[e];
+          ww[c] = w2[e];
+        }
+      }
     }
 #pragma unroll
     for (int c = 0; c < kPairs; ++c) {
@@ -282,19 +255,11 @@ __device__ __forceinline__ void rhs_to_lds(double* pk, const Geom& g, const RhsA
           if (store) o2[e] = v1[c];
         }
         if (rhs) {
-          pk[p0] = bdf_rhs(v1[c].x, h.v2[c].x, h.v3[c].x, h.w[c].x, a0, a1, a2, b0, b1, b2, ds);
-          pk[p1] = bdf_rhs(v1[c].y, h.v2[c].y, h.v3[c].y, h.w[c].y, a0, a1, a2, b0, b1, b2, ds);
+          pk[p0] = bdf_rhs(v1[c].x, v2[c].x, v3[c].x, ww[c].x, a0, a1, a2, b0, b1, b2, ds);
+          pk[p1] = bdf_rhs(v1[c].y, v2[c].y, v3[c].y, ww[c].y, a0, a1, a2, b0, b1, b2, ds);
         }
       }
     }
-  }
-}
-
-// the compile-time plane's twiddles into LDS (visible after the next barrier)
-template <int NX, int NY>
-__device__ __forceinline__ void load_ct_tw(double2* lds, const Geom& g) {
-  if constexpr (NX > 0) {
-    if (threadIdx.x < NX) ct_tw<NX, NY>(lds)[threadIdx.x] = g.ax.tw[threadIdx.x];
   }
 }
 
@@ -306,7 +271,6 @@ __device__ __forceinline__ void k_rhs_fft_xy_body(const Geom& g, const RhsArgs& 
   int z, i;
   plane_of_block(g.nz, z, i);
   const long long plane = (long long)z * g.zs;
-  load_ct_tw<NX, NY>(lds, g);
   rhs_to_lds<NX, NY, ORDER, false>(reinterpret_cast<double*>(lds), g, a, i, plane, true, 1.0,
                                nullptr, false, true);
   forward_xy<NX, NY, MAXE>(lds, g, reinterpret_cast<S*>(a.spec), i, z);
@@ -332,7 +296,6 @@ __device__ __forceinline__ void k_ifft_xy_body(const Geom& g, const InvArgs& a) 
   int z, i;
   plane_of_block(g.nz, z, i);
   const int nx = NX ? NX : g.nx, ny = NY ? NY : g.ny;
-  load_ct_tw<NX, NY>(lds, g);
   inverse_xy<NX, NY, MAXE>(lds, g, reinterpret_cast<const S*>(a.spec), i, z);
   double* out = a.out + i * g.hs + (long long)z * g.zs;
   const double* pk = reinterpret_cast<const double*>(lds);
@@ -369,20 +332,9 @@ __device__ __forceinline__ void k_inv_rhs_body(const Geom& g, const InvArgs& c, 
   const long long plane = (long long)z * g.zs;
   const bool inv = i < c.M;
   const bool rhs = i < a.M;
-  load_ct_tw<NX, NY>(lds, g);
-  if constexpr (NX > 0) {
-    // a thread's pairs are few: their history is asked for before the inverse passes
-    static_assert(NX * NY / 2 <= kPairs * kThreads, "one batch of pairs per thread");
-    HistPairs h;
-    if (rhs) load_pairs<ORDER>(h, g, a, i, plane, 0, NX * NY / 2);
-    if (inv) inverse_xy<NX, NY, MAXE>(lds, g, reinterpret_cast<const S*>(c.spec), i, z);
-    rhs_to_lds<NX, NY, ORDER, true>(reinterpret_cast<double*>(lds), g, a, i, plane, inv, c.scale,
-                                    c.out + i * g.hs + plane, inv, rhs, &h);
-  } else {
-    if (inv) inverse_xy<NX, NY, MAXE>(lds, g, reinterpret_cast<const S*>(c.spec), i, z);
-    rhs_to_lds<NX, NY, ORDER, true>(reinterpret_cast<double*>(lds), g, a, i, plane, inv, c.scale,
-                                    c.out + i * g.hs + plane, inv, rhs);
-  }
+  if (inv) inverse_xy<NX, NY, MAXE>(lds, g, reinterpret_cast<const S*>(c.spec), i, z);
+  rhs_to_lds<NX, NY, ORDER, true>(reinterpret_cast<double*>(lds), g, a, i, plane, inv, c.scale,
+                              c.out + i * g.hs + plane, inv, rhs);
   if (rhs) forward_xy<NX, NY, MAXE>(lds, g, reinterpret_cast<S*>(a.spec), i, z);
 }
 
@@ -434,7 +386,9 @@ static void* inv_rhs_kernel(int order) {
 // 24 x 24 and 32 x 32 planes take compile-time Stockham passes on four waves: a sweep pair with
 // both directions in flight takes 3.81 and 3.77 ms at 24^3 / Lmax 6 and 32^3 / Lmax 4 against 4.08
 // and 3.94 with the two-pass kernels, whose plane is two waves; every larger plane is faster there
-// (48 x 48, Lmax 6 61.5 -> 51.2 us; 36 x 54, Lmax 4 46 -> 40).
+// (48 x 48, Lmax 6 61.5 -> 51.2 us; 36 x 54, Lmax 4 46 -> 40).  Loading the history before the
+// inverse passes and keeping the twiddles in LDS, which the two-pass kernels gain by, costs these
+// registers and time (24 x 24, Lmax 6 13.3 -> 14.1 us, 32 x 32, Lmax 4 14.2 -> 15.4).
 static bool specialised(const Geom& g) {
   return g.nx == g.ny && (g.nx == 24 || g.nx == 32);
 }
@@ -443,7 +397,7 @@ static bool two_pass_plane(const Geom& g) { return !specialised(g) && p2::takes(
 
 static size_t plane_lds_bytes(const Geom& g) {
   const size_t n = (size_t)g.ny * g.nxh;
-  return sizeof(double2) * (specialised(g) ? n + n / 8 + 1 + g.nx : n);
+  return sizeof(double2) * (specialised(g) ? n + n / 8 + 1 : n);
 }
 
 bool plane_supported(int nx, int ny) {
