@@ -6,7 +6,7 @@ each step kernel with the GPU to itself) on a cubic grid of edge nz, and the fas
 written to csrc/wlc_tune.inc, the table the library compiles in (wlc_tune.cpp).  Variants:
 the one-wave nz = 64 kernel at one or two waves per SIMD, the degree-split two-column and
 whole-tile nz = 64 kernels (Lmax 5-7), the column kernel of the short axes (nz = 24, 32, 48),
-the nz = 128 kernels, and the generic kernel with
+the nz = 128 kernels (whole columns; three degree parts at Lmax 5-8), and the generic kernel with
 every admissible number of kx columns per workgroup, with and without the degree split
 (Lmax 4-7).  Candidates are selected through the library's measurement switches
 (WLC_GENERIC_ZSOLVE, WLC_ZSOLVE_SPLIT, WLC_ZSOLVE_OCC, WLC_ZSOLVE_TX).

@@ -41,6 +41,10 @@ def _units():
     for L in range(MAX_L + 1):
         units.append(("wlc_zsolve.hip", f"wlc_zsolve_L{L}.o", [f"-DWLC_L={L}"]))
         units.append(("wlc_zcol.hip", f"wlc_zcol_L{L}.o", [f"-DWLC_L={L}"]))
+        if L >= 5:
+            # (literals hoisted out of its loop over the column pairs would take the registers)
+            units.append(("wlc_z128.hip", f"wlc_z128_L{L}.o",
+                          [f"-DWLC_L={L}", "-mllvm", "-disable-machine-licm"]))
     return units
 
 

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "wlc_kernels.h"
+#include "wlc_z128.h"
 #include "wlc_zcol.h"
 
 namespace wlc {
@@ -17,12 +18,21 @@ namespace wlc {
 
 WLC_DECL(0) WLC_DECL(1) WLC_DECL(2) WLC_DECL(3) WLC_DECL(4) WLC_DECL(5) WLC_DECL(6) WLC_DECL(7) WLC_DECL(8)
 #undef WLC_DECL
+const void* z128_kernel_L5(bool, bool);
+const void* z128_kernel_L6(bool, bool);
+const void* z128_kernel_L7(bool, bool);
+const void* z128_kernel_L8(bool, bool);
 
 namespace {
 // short z axes take the column kernel unless the generic kernel or its degree split (1) is asked
 // for
 bool use_zcol(const Geom& g, const SolveArgs& a) {
   return zcol_nz(g.nz) && !a.generic && a.split >= 2 && a.M == (a.L + 1) * (a.L + 1);
+}
+
+// nz = 128 with a degree split asked for: the three-part kernel
+bool use_z128(const Geom& g, const SolveArgs& a) {
+  return g.nz == 128 && a.L >= kZ128MinL && !a.generic && a.split && a.M == (a.L + 1) * (a.L + 1);
 }
 
 const void* zcol_kernel(const Geom& g, const SolveArgs& a, bool batch) {
@@ -34,13 +44,30 @@ const void* zcol_kernel(const Geom& g, const SolveArgs& a, bool batch) {
   }
   return nullptr;
 }
+const void* z128_kernel(const Geom& g, const SolveArgs& a, bool batch) {
+  switch (a.L) {
+#define WLC_CASE(L) \
+  case L: return z128_kernel_L##L(g.spec32 != 0, batch);
+    WLC_CASE(5) WLC_CASE(6) WLC_CASE(7) WLC_CASE(8)
+#undef WLC_CASE
+  }
+  return nullptr;
+}
 
-hipError_t zcol_launch(const Geom& g, const SolveArgs& a, const ZJob* jobs, int n, hipStream_t st) {
-  const void* k = zcol_kernel(g, a, jobs != nullptr);
-  if (!k) return hipErrorInvalidValue;
-  const size_t lds = zcol_lds_bytes(g.nz, a.M);
-  if (lds > 64 * 1024) {
-    hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+bool own_file(const Geom& g, const SolveArgs& a) { return use_zcol(g, a) || use_z128(g, a); }
+
+LaunchKey own_key(const Geom& g, const SolveArgs& a, bool batch) {
+  if (use_z128(g, a))
+    return LaunchKey{z128_kernel(g, a, batch), z128_grid(g), 1u, (unsigned)kZ128Threads, z128_lds_bytes()};
+  return LaunchKey{zcol_kernel(g, a, batch), zcol_grid(g), 1u, (unsigned)zcol_threads(g.nz),
+                   zcol_lds_bytes(g.nz, a.M)};
+}
+
+hipError_t own_launch(const Geom& g, const SolveArgs& a, const ZJob* jobs, int n, hipStream_t st) {
+  const LaunchKey key = own_key(g, a, jobs != nullptr);
+  if (!key.k) return hipErrorInvalidValue;
+  if (key.lds > 64 * 1024) {
+    hipError_t e = hipFuncSetAttribute(key.k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)key.lds);
     if (e != hipSuccess) return e;
   }
   Geom gg = g;
@@ -48,13 +75,12 @@ hipError_t zcol_launch(const Geom& g, const SolveArgs& a, const ZJob* jobs, int 
   const ZJob* jp = jobs;
   void* one[] = {&gg, &aa};
   void* many[] = {&jp};
-  return hipLaunchKernel(k, dim3(zcol_grid(g), 1, n),
-                         dim3(zcol_threads(g.nz)), jobs ? many : one, lds, st);
+  return hipLaunchKernel(key.k, dim3(key.gx, 1, n), dim3(key.threads), jobs ? many : one, key.lds, st);
 }
 }  // namespace
 
 hipError_t launch_zsolve(const Geom& g, const SolveArgs& a, hipStream_t st) {
-  if (use_zcol(g, a)) return zcol_launch(g, a, nullptr, 1, st);
+  if (own_file(g, a)) return own_launch(g, a, nullptr, 1, st);
   switch (a.L) {
 #define WLC_CASE(L) \
   case L: return zsolve_launch_L##L(g, a, st);
@@ -66,7 +92,7 @@ hipError_t launch_zsolve(const Geom& g, const SolveArgs& a, hipStream_t st) {
 
 hipError_t launch_zsolve_batch(const ZJob& rep, const ZJob* jobs, int n, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  if (use_zcol(rep.g, rep.a)) return zcol_launch(rep.g, rep.a, jobs, n, st);
+  if (own_file(rep.g, rep.a)) return own_launch(rep.g, rep.a, jobs, n, st);
   switch (rep.a.L) {
 #define WLC_CASE(L) \
   case L: return zsolve_batch_L##L(rep, jobs, n, st);
@@ -77,9 +103,7 @@ hipError_t launch_zsolve_batch(const ZJob& rep, const ZJob* jobs, int n, hipStre
 }
 
 LaunchKey zsolve_key(const Geom& g, const SolveArgs& a) {
-  if (use_zcol(g, a))
-    return LaunchKey{zcol_kernel(g, a, false), zcol_grid(g), 1u,
-                     (unsigned)zcol_threads(g.nz), zcol_lds_bytes(g.nz, a.M)};
+  if (own_file(g, a)) return own_key(g, a, false);
   switch (a.L) {
 #define WLC_CASE(L) \
   case L: return zsolve_key_L##L(g, a);

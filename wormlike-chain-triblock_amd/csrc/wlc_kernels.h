@@ -70,8 +70,9 @@ struct SolveArgs {
                        // 2, 3 the column kernel.  nz = 64 (Lmax 5-7; else 0): 0 one wave per
                        // column, else two by degree: 1 two columns per workgroup, loaded
                        // directly, 2 a whole 4-kx tile per workgroup, 3 half a tile, both
-                       // through LDS (2 and 3: FP64 spectrum; FP32 runs as 1).  nz = 128 (Lmax
-                       // 5-8) and other nz (Lmax 4-7): any nonzero value splits by degree
+                       // through LDS (2 and 3: FP64 spectrum; FP32 runs as 1).  nz = 128, Lmax
+                       // 5-8: 0 whole columns per wave pair, else the three-part kernel
+                       // (wlc_z128.h).  Other nz, Lmax 4-7: any nonzero value splits by degree
 };
 
 // Kernel C: inverse y and x (C2R) passes, scaling by 1/N, store of q(s).
