@@ -12,9 +12,9 @@
 // goes through its pairs in a loop and asks for the next pair while it transforms this one back,
 // in the registers that its harmonics leave, eight harmonics of each part at a time.  A pair, not
 // a column: 32-byte pieces of the tiles move at the full rate (a bare copy of the spectrum in
-// place 594 us, in 16-byte pieces 863 to 1279).  Per launch on 128^3: Lmax 8 1853 -> 1201 us (of
-// them 565 for the bare copy), with the FP32 spectrum 1537 -> 953; Lmax 7 1275 -> 895, Lmax 6
-// 820 -> 613.
+// place 594 us, in 16-byte pieces 863 to 1279).  Per launch on 128^3: Lmax 8 1853 -> 1085 us (of
+// them 565 for the bare copy), with the FP32 spectrum 1537 -> 875; Lmax 7 1275 -> 818, Lmax 6
+// 820 -> 594.
 #include <hip/hip_runtime.h>
 
 #include "wlc_device.h"
@@ -201,12 +201,14 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// A wave's LDS rows hold 64 points of eight harmonics.  Natural order: point z of harmonic q at
-// 64 q + (z ^ 8 (q & 1)).  Between the two radix-8 passes: element m of row k, swizzled so that
-// the passes over the rows and along them both meet all banks equally often; the solve takes the
-// points as they lie there.
-__device__ __forceinline__ int place(int q, int z) { return 64 * q + (z ^ (8 * (q & 1))); }
-__device__ __forceinline__ int slot(int q, int k, int m) { return 64 * q + 8 * (k ^ (q & 1)) + (m ^ k); }
+// A wave's LDS rows hold 64 points of eight harmonics, 72 places apart.  Natural order: point z at
+// place z.  Between the two radix-8 passes: element m of row k at 9 k + m, the order in which the
+// solve takes the points (lane 8 k + m).  All three ways of going over them meet every bank equally
+// often and differ from a lane's first place by constants, which cost no registers (with places that
+// were turned by the row instead, Lmax 8 took 1201 us, not 1098).
+__device__ __forceinline__ int place(int q, int z) { return 72 * q + z; }
+__device__ __forceinline__ int slot(int q, int k, int m) { return 72 * q + 9 * k + m; }
+__device__ __forceinline__ int point(int q, int lane) { return slot(q, lane >> 3, lane & 7); }
 
 // The column pairs of a workgroup.  The tiles are dealt to the XCDs and the pairs of an XCD's
 // tiles to its workgroups in turn, so the two pairs of a tile, which share cache lines, are at
@@ -254,10 +256,14 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
   constexpr int NH = P::NH;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wc = (wv >> 1) & 1, wh = wv & 1;  // this wave's column and half
-  double2* rows = lds + PART * 4 * 512;       // of (column, half): 512 (2 c + h)
-  double2* own = rows + 512 * (2 * wc + wh);
-  const double2* tw = lds + 12 * 512 + 4 * kZ128Chains * 64;  // exp(-2 pi i t / 128)
-  double2* frame = lds + 12 * 512 + 4 * kZ128Chains * 64 + 128 + (2 * wc + wh) * kZ128Frame;
+  // rows of (column, half): kZ128Col (2 c + h); those of part 0 are the chains' rows too, during
+  // the solve
+  double2* rows = lds + (PART == 0 ? 0 : kZ128Chains * 64 + kZ128Rows * (PART - 1));
+  double2* own = rows + kZ128Col * (2 * wc + wh);
+  double2* chain = lds + kZ128Col * (2 * wc + wh);
+  const double2* tw = lds + 4 * kZ128Col;  // exp(-2 pi i t / 128)
+  const double2* tw64 = tw + 128;          // exp(-2 pi i j n / 64) at 8 n + j
+  double2* frame = lds + 4 * kZ128Col + 192 + (2 * wc + wh) * kZ128Frame;
   Pairs<S> w(g, a.spec);
   double2 v[NH];
   if (w.ky >= 0 && w.kx0 + (int)(threadIdx.x & 1) < w.nxh) {
@@ -281,9 +287,9 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
       const int lane = tid & 63;
       if (PART == 0 && real) {
         const int hq = lane >> 3, j = lane & 7;
-        // lane = 8 k1 + (k2 ^ k1) holds kz = 2 (k1 + 8 k2) + half
+        // lane = 8 k1 + k2 holds kz = 2 (k1 + 8 k2) + half
         const KFrame kf(signed_k(w.kx0 + wc, g.nx) * a.kfac[0], signed_k(w.ky, g.ny) * a.kfac[1],
-                        signed_k(2 * (hq + 8 * (j ^ hq)) + wh, 128) * a.kfac[2], a.sigma, a.ds);
+                        signed_k(2 * (hq + 8 * j) + wh, 128) * a.kfac[2], a.sigma, a.ds);
         if (lane == 0) frame[0] = make_double2(kf.cq, kf.sq);
         frame[2 + lane] = make_double2(kf.ct, kf.st);
         reinterpret_cast<double*>(frame + 66)[lane] = kf.gk;
@@ -296,12 +302,12 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
         __syncthreads();  // the rows are free (first round of all: the twiddles are in LDS)
 #pragma unroll
         for (int q = 0; q < 8; ++q)
-          if (8 * k + q < NH) rows[512 * (2 * tc + (tz >> 6)) + place(q, tm)] = v[8 * k + q];
+          if (8 * k + q < NH) rows[kZ128Col * (2 * tc + (tz >> 6)) + place(q, tm)] = v[8 * k + q];
         __syncthreads();
         double2 u[8];
         if (8 * k < NH && real) {
           // radix-2 step: the even kz have x(m) + x(m + 64), the odd ones (x(m) - x(m + 64)) W128^m
-          const double2 *lo = rows + 512 * (2 * wc), *hi = lo + 512;
+          const double2 *lo = rows + kZ128Col * (2 * wc), *hi = lo + kZ128Col;
           if (wh == 0) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) u[r] = cadd(lo[place(hq, j + 8 * r)], hi[place(hq, j + 8 * r)]);
@@ -315,7 +321,7 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
         if (8 * k < NH && real) {
           Dft<8, -1>::run(u);
 #pragma unroll
-          for (int n = 1; n < 8; ++n) u[n] = twiddle<-1>(u[n], tw[2 * j * n]);
+          for (int n = 1; n < 8; ++n) u[n] = twiddle<-1>(u[n], tw64[8 * n + j]);
 #pragma unroll
           for (int n = 0; n < 8; ++n) own[slot(hq, n, j)] = u[n];
           wave_sync();
@@ -327,12 +333,12 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
           wave_sync();
 #pragma unroll
           for (int q = 0; q < 8; ++q)
-            if (8 * k + q < NH) v[8 * k + q] = own[place(q, lane)];
+            if (8 * k + q < NH) v[8 * k + q] = own[point(q, lane)];
         } else {
           clear8(v, 8 * k);  // (nothing is kept across the round: registers)
         }
       }
-      double2* x = lds + 12 * 512 + (2 * wc + wh) * (kZ128Chains * 64) + lane;
+      double2* x = chain + lane;
       const double* gk = reinterpret_cast<const double*>(frame + 66) + lane;
       if (act) rotate<PART, true>(v, frame, lane);
       if (PART == 0 && act) chains_up<0>(v, cdelta, dslam, *gk, x);
@@ -364,7 +370,7 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
       if (8 * k < NH && real) {
 #pragma unroll
         for (int q = 0; q < 8; ++q)
-          if (8 * k + q < NH) own[place(q, lane)] = v[8 * k + q];
+          if (8 * k + q < NH) own[point(q, lane)] = v[8 * k + q];
         wave_sync();
       }
       // the next pair's harmonics take the registers of the round before
@@ -380,7 +386,7 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
         for (int m = 0; m < 8; ++m) u[m] = own[slot(hq, j, m)];
         Dft<8, +1>::run(u);
 #pragma unroll
-        for (int m = 1; m < 8; ++m) u[m] = twiddle<+1>(u[m], tw[2 * j * m]);
+        for (int m = 1; m < 8; ++m) u[m] = twiddle<+1>(u[m], tw64[8 * m + j]);
 #pragma unroll
         for (int m = 0; m < 8; ++m) own[slot(hq, j, m)] = u[m];
         wave_sync();
@@ -404,7 +410,7 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
         clear8(v, 8 * k);
       }
       if (io) {
-        const double2 *even = rows + 512 * (2 * tc), *odd = even + 512;
+        const double2 *even = rows + kZ128Col * (2 * tc), *odd = even + kZ128Col;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           if (8 * k + q < NH) {
@@ -421,7 +427,9 @@ __device__ __forceinline__ void column_pairs(const Geom& g, const SolveArgs& a, 
 template <class S>
 __device__ __forceinline__ void k_z128_body(const Geom& g, const SolveArgs& a) {
   extern __shared__ double2 lds[];
-  if (threadIdx.x < 128) lds[12 * 512 + 4 * kZ128Chains * 64 + threadIdx.x] = g.az.tw[threadIdx.x];
+  if (threadIdx.x < 128) lds[4 * kZ128Col + threadIdx.x] = g.az.tw[threadIdx.x];
+  else if (threadIdx.x < 192)
+    lds[4 * kZ128Col + threadIdx.x] = g.az.tw[2 * ((threadIdx.x & 63) >> 3) * (threadIdx.x & 7)];
   // wave 4 part + 2 column + half: every SIMD gets one wave of each part
   const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   if (part == 0) column_pairs<0, S>(g, a, lds);
