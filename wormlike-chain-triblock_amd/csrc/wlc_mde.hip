@@ -126,8 +126,8 @@ struct wlc_handle {
   hipEvent_t ev_pre = nullptr, ev_join[2] = {nullptr, nullptr};
   bool pre_recorded = false;
   // Forward-store checkpointing (ck > 0, when the full store does not fit or on request):
-  // the forward sweep keeps a 4-slot ring `fr` and copies slices jK-2, jK-1, jK of every
-  // segment boundary jK (j = 1 .. nseg-1) to `ckpt` and q(Ns) to `qlast`.  The backward
+  // the forward sweep keeps a 4-slot ring `fr` and writes slices jK-2, jK-1, jK of every
+  // segment boundary jK (j = 1 .. nseg-1) to `ckpt` instead and q(Ns) to `qlast`.  The backward
   // sweep recomputes segment j = (jK, (j+1)K] (segment 0 = [0, K]) from its checkpoint into
   // segment buffer j % 2 on stream `str` with its own spectrum `specr`, one segment ahead
   // of the densities that read it: ev_seg_ready[b] marks a buffer filled, ev_seg_free[b]
@@ -180,12 +180,34 @@ struct SweepCtx {
 
 long long slot_size(const wlc_handle* h) { return (long long)h->Mmax * h->hs; }
 
+// first segment restarted from a checkpoint (segment nstored restarts from the store)
+int first_ckpt_segment(const wlc_handle* h) { return h->nstored > 0 ? h->nstored + 1 : 1; }
+
+double* ckpt_slot(const wlc_handle* h, int j, int t) {
+  return h->ckpt + ((long long)(j - first_ckpt_segment(h)) * 3 + t) * slot_size(h);
+}
+
+// The slices that the checkpoints keep (the restart history of every segment boundary, q(Ns)) are
+// written where they are kept and read there by the steps that need them; a copy of each took
+// 0.64 ms of a 128^3 / Lmax 8 sweep, 22 of them in a sweep pair of 24 steps.
 double* fwd_slice(const wlc_handle* h, const FwdLoc& fl, int s) {
+  const int K = h->ck;
   if (fl.mode == 1) {
-    if (h->nstored > 0 && s <= h->nstored * h->ck) return h->store + (long long)s * slot_size(h);
+    if (s == h->Ns) return h->qlast;
+    if (h->nstored > 0 && s <= h->nstored * K) return h->store + (long long)s * slot_size(h);
+    // j = floor((s + 2) / K) gives jK - 2 <= s < (j + 1)K - 2: only s <= jK is a restart slice
+    const int j = (s + 2) / K;
+    if (j >= first_ckpt_segment(h) && j <= h->nseg - 1 && s <= j * K) return ckpt_slot(h, j, s - (j * K - 2));
     return h->fr + (long long)(s & 3) * slot_size(h);
   }
-  if (fl.mode == 2) return fl.base + (long long)(s - fl.lo) * slot_size(h);
+  if (fl.mode == 2) {
+    // segment j >= 1 starts from slices jK - 2, jK - 1, jK
+    if (fl.lo > 0 && s <= fl.lo + 2) {
+      const int j = (fl.lo + 2) / K;
+      return j == h->nstored ? h->store + (long long)s * slot_size(h) : ckpt_slot(h, j, s - fl.lo);
+    }
+    return fl.base + (long long)(s - fl.lo) * slot_size(h);
+  }
   return h->q + h->off[s];
 }
 
@@ -398,8 +420,6 @@ int density_at(wlc_handle* h, int s);
 
 // the steps of one sweep, targets first .. last (inclusive, in direction dir); after
 // each target the optional density accumulation
-int save_checkpoint(wlc_handle* h, const SweepCtx& sw, int s);
-
 int sweep(wlc_handle* h, const SweepCtx& sw, int first, int last, bool dens) {
   const int dir = sw.dir;
   int rc = step_rhs(h, sw, first);
@@ -412,40 +432,10 @@ int sweep(wlc_handle* h, const SweepCtx& sw, int first, int last, bool dens) {
     } else {
       if ((rc = step_inverse(h, sw, s, false))) return rc;
     }
-    if (dir > 0 && sw.fl.mode == 1 && (rc = save_checkpoint(h, sw, s))) return rc;
     if (dens && (rc = density_at(h, s))) return rc;
     if (!more) break;
     if (!h->fuse && (rc = step_rhs(h, sw, s + dir))) return rc;
   }
-  return WLC_OK;
-}
-
-// first segment restarted from a checkpoint (segment nstored restarts from the store)
-int first_ckpt_segment(const wlc_handle* h) { return h->nstored > 0 ? h->nstored + 1 : 1; }
-
-double* ckpt_slot(const wlc_handle* h, int j, int t) {
-  return h->ckpt + ((long long)(j - first_ckpt_segment(h)) * 3 + t) * slot_size(h);
-}
-
-// restart slice jK - 2 + t of segment j >= 1
-const double* restart_slice(const wlc_handle* h, int j, int t) {
-  if (h->nstored > 0 && j == h->nstored)
-    return h->store + (long long)(j * h->ck - 2 + t) * slot_size(h);
-  return ckpt_slot(h, j, t);
-}
-
-// after forward slice s on the ring: keep the restart history of every segment boundary
-// and the last slice
-int save_checkpoint(wlc_handle* h, const SweepCtx& sw, int s) {
-  const int K = h->ck;
-  const size_t bytes = sizeof(double) * (size_t)h->Mb[block_of(h, s)] * h->hs;
-  // j = floor((s + 2) / K) gives jK - 2 <= s < (j + 1)K - 2: only s <= jK is a restart slice
-  const int j = (s + 2) / K;
-  if (j >= first_ckpt_segment(h) && j <= h->nseg - 1 && s <= j * K)
-    HIPCHK(hipMemcpyAsync(ckpt_slot(h, j, s - (j * K - 2)), fwd_slice(h, sw.fl, s), bytes,
-                          hipMemcpyDeviceToDevice, sw.st));
-  if (s == h->Ns)
-    HIPCHK(hipMemcpyAsync(h->qlast, fwd_slice(h, sw.fl, s), bytes, hipMemcpyDeviceToDevice, sw.st));
   return WLC_OK;
 }
 
@@ -464,16 +454,8 @@ int recompute_segment(wlc_handle* h, int j) {
   const int b = j & 1, K = h->ck;
   if (h->seg_busy[b]) HIPCHK(hipStreamWaitEvent(h->str, h->ev_seg_free[b], 0));
   SweepCtx sw{+1, h->str, h->specr, seg_loc(h, j)};
-  if (j == 0) {
+  if (j == 0)
     HIPCHK(wlc::launch_set_delta(h->geom, fwd_slice(h, sw.fl, 0), h->Mb[block_of(h, 0)], h->str));
-  } else {
-    for (int t = 0; t < 3; ++t) {
-      const int s = j * K - 2 + t;
-      const size_t bytes = sizeof(double) * (size_t)h->Mb[block_of(h, s)] * h->hs;
-      HIPCHK(hipMemcpyAsync(fwd_slice(h, sw.fl, s), restart_slice(h, j, t), bytes,
-                            hipMemcpyDeviceToDevice, h->str));
-    }
-  }
   int rc = sweep(h, sw, j == 0 ? 1 : j * K + 1, std::min((j + 1) * K, h->Ns), false);
   if (rc) return rc;
   HIPCHK(hipEventRecord(h->ev_seg_ready[b], h->str));
