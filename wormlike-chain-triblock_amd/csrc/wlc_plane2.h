@@ -37,7 +37,7 @@ inline size_t lds_bytes(int nx, int ny) {
 inline bool takes(int nx, int ny) { return two_pass(nx).R > 0 && two_pass(ny).R > 0; }
 
 // kind 0: A, 1: C, 2: fused C + A
-const void* kernel(int nx, int ny, int kind, bool spec32, bool batch);
+const void* kernel(int nx, int ny, int kind, bool batch);
 
 }  // namespace p2
 }  // namespace wlc

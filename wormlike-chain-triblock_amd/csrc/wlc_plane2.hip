@@ -624,8 +624,8 @@ const void* pick_edges(int nx, int ny, int kind, bool batch) {
 
 }  // namespace
 
-const void* kernel(int nx, int ny, int kind, bool spec32, bool batch) {
-  return spec32 ? pick_edges<float2>(nx, ny, kind, batch) : pick_edges<double2>(nx, ny, kind, batch);
+const void* kernel(int nx, int ny, int kind, bool batch) {
+  return pick_edges<double2>(nx, ny, kind, batch);
 }
 
 }  // namespace p2

@@ -363,9 +363,8 @@ __global__ void __launch_bounds__(512, kWaves) k_zcol_b(const ZJob* __restrict__
 
 using namespace WLC_CAT(zcol_l_, WLC_L);
 
-const void* WLC_CAT(zcol_kernel_L, WLC_L)(bool spec32, bool batch) {
-  if (batch) return spec32 ? (const void*)k_zcol_b<float2> : (const void*)k_zcol_b<double2>;
-  return spec32 ? (const void*)k_zcol<float2> : (const void*)k_zcol<double2>;
+const void* WLC_CAT(zcol_kernel_L, WLC_L)(bool batch) {
+  return batch ? (const void*)k_zcol_b<double2> : (const void*)k_zcol<double2>;
 }
 
 }  // namespace wlc
