@@ -20,11 +20,11 @@ import sys
 
 # bench.py kernel keys -> substrings of the HIP kernel names
 KEYS = [
-    ("inv_rhs_fft_xy", ("k_inv_rhs64", "k_inv_rhs128", "k_inv_rhs<")),
-    ("rhs_fft_xy", ("k_rhs64", "k_rhs128", "k_rhs_fft_xy")),
-    ("ifft_xy", ("k_inv64", "k_inv128", "k_ifft_xy")),
-    ("zsolve", ("k_zsolve",)),
-    ("density_acc", ("k_density_acc",)),
+    ("inv_rhs_fft_xy", ("k_inv_rhs64", "k_inv_rhs128", "k_inv_rhs<", "k2_inv_rhs<")),
+    ("rhs_fft_xy", ("k_rhs64", "k_rhs128", "k_rhs_fft_xy", "k2_rhs<")),
+    ("ifft_xy", ("k_inv64", "k_inv128", "k_ifft_xy", "k2_inv<")),
+    ("zsolve", ("k_zsolve", "k_zcol", "k_z128")),
+    ("density_acc", ("k_density_acc", "k_density_run")),
 ]
 COPY_BYTES = 256 * 1024 * 1024
 
