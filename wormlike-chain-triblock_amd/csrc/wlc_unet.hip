@@ -30,6 +30,7 @@
 #include <cstring>
 #include <random>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/wlc_mde.h"
@@ -853,39 +854,55 @@ int alloc_acts(wlc_unet* u, int n, int B) {
   free_acts(u);
   u->n = n;
   u->B = B;
-  int rc;
-#define UA(ptr, cnt) if ((rc = ualloc(u->acts, &(ptr), (cnt)))) { free_acts(u); return rc; }
-  const long long V0 = u->vol(0).voxels(), V1 = u->vol(1).voxels(), V2 = u->vol(2).voxels(), V3 = u->vol(3).voxels();
-  UA(u->lpart, 256);
-  UA(u->x0, V0 * 16); UA(u->a0a, V0 * 32); UA(u->p1, V1 * 32); UA(u->a1a, V1 * 64);
-  UA(u->p2, V2 * 64); UA(u->a2a, V2 * 128); UA(u->p3, V3 * 128);
-  UA(u->c2, V2 * 256); UA(u->c1, V1 * 128); UA(u->c0, V0 * 64); UA(u->d0, V0 * 32);
-  UA(u->gp1, V1 * 32); UA(u->gp2, V2 * 64); UA(u->gp3, V3 * 128);
-  UA(u->gc2, V2 * 256); UA(u->gc1, V1 * 128); UA(u->gc0, V0 * 64);
-  UA(u->y, V0 * 3); UA(u->xin, V0 * 11); UA(u->target, V0 * 3);
-  const bf16* X[11] = {u->x0, u->a0a, u->p1, u->a1a, u->p2, u->a2a, u->p3, u->c2, u->c1, u->c0, u->d0};
+  // one allocation for all of them, cleared at once (a hundred of them one by one took 50 ms):
+  // laid out without a base to learn the size, then with it
+  std::vector<GradJob> all;
+  size_t bytes = 0;
+  auto lay = [&](uintptr_t base) {
+    bytes = 0;
+    auto take = [&](auto*& ptr, long long count) {
+      ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(base + bytes);
+      bytes += (sizeof(*ptr) * (size_t)std::max<long long>(count, 1) + 255) / 256 * 256;
+    };
+#define UA(ptr, cnt) take(ptr, cnt)
+    const long long V0 = u->vol(0).voxels(), V1 = u->vol(1).voxels(), V2 = u->vol(2).voxels(), V3 = u->vol(3).voxels();
+    UA(u->lpart, 256);
+    UA(u->x0, V0 * 16); UA(u->a0a, V0 * 32); UA(u->p1, V1 * 32); UA(u->a1a, V1 * 64);
+    UA(u->p2, V2 * 64); UA(u->a2a, V2 * 128); UA(u->p3, V3 * 128);
+    UA(u->c2, V2 * 256); UA(u->c1, V1 * 128); UA(u->c0, V0 * 64); UA(u->d0, V0 * 32);
+    UA(u->gp1, V1 * 32); UA(u->gp2, V2 * 64); UA(u->gp3, V3 * 128);
+    UA(u->gc2, V2 * 256); UA(u->gc1, V1 * 128); UA(u->gc0, V0 * 64);
+    UA(u->y, V0 * 3); UA(u->xin, V0 * 11); UA(u->target, V0 * 3);
+    const bf16* X[11] = {u->x0, u->a0a, u->p1, u->a1a, u->p2, u->a2a, u->p3, u->c2, u->c1, u->c0, u->d0};
+    all.clear();
+    for (int li = 0; li < 11; ++li) {
+      const Layer& l = u->layers[li];
+      const Vol g = u->vol(l.level);
+      const long long V = g.voxels();
+      UA(u->dy[li], V * l.cout); UA(u->dyb[li], V * l.cout);
+      GradJob q = grad_job(g, l.cin, l.cout);
+      q.X = X[li];
+      q.dYb = u->dyb[li];
+      q.dYf = u->dy[li];
+      q.dW = u->g + l.woff;
+      q.db = u->g + l.boff;
+      UA(q.part, part_floats(q));
+      UA(q.bpart, (long long)q.nbp * l.cout);
+      if (grad_rows(g)) {
+        UA(q.xt, V * l.cin);
+        UA(q.dyt, V * l.cout);
+      }
+      all.push_back(q);
+    }
+    UA(u->djobs, 1); UA(u->dall, 1);
+#undef UA
+  };
+  lay(0);
+  char* block = nullptr;
+  if (const int rc = ualloc(u->acts, &block, (long long)bytes)) return rc;
+  lay(reinterpret_cast<uintptr_t>(block));
   u->jobs.clear();
   u->odd.clear();
-  std::vector<GradJob> all;
-  for (int li = 0; li < 11; ++li) {
-    const Layer& l = u->layers[li];
-    const Vol g = u->vol(l.level);
-    const long long V = g.voxels();
-    UA(u->dy[li], V * l.cout); UA(u->dyb[li], V * l.cout);
-    GradJob q = grad_job(g, l.cin, l.cout);
-    q.X = X[li];
-    q.dYb = u->dyb[li];
-    q.dYf = u->dy[li];
-    q.dW = u->g + l.woff;
-    q.db = u->g + l.boff;
-    UA(q.part, part_floats(q));
-    UA(q.bpart, (long long)q.nbp * l.cout);
-    if (grad_rows(g)) {
-      UA(q.xt, V * l.cin);
-      UA(q.dyt, V * l.cout);
-    }
-    all.push_back(q);
-  }
   // launches 0 .. 2 run over the layers of the transposed kernel, 3 .. 5 over all of them
   for (const GradJob& q : all) (grad_rows(q.g) ? u->jobs : u->odd).push_back(q);
   unsigned gr[6] = {}, ga[6] = {};
@@ -893,8 +910,6 @@ int alloc_acts(wlc_unet* u, int n, int B) {
   place_jobs(all, ga);
   for (int k = 0; k < 6; ++k) u->grid[k] = k <= kDw ? gr[k] : ga[k];
   GradJobs t{};
-  UA(u->djobs, 1); UA(u->dall, 1);
-#undef UA
   t.n = (int)u->jobs.size();
   std::copy(u->jobs.begin(), u->jobs.end(), t.j);
   hipError_t e = hipMemcpy(u->djobs, &t, sizeof(t), hipMemcpyHostToDevice);
