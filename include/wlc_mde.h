@@ -259,7 +259,8 @@ void wlc_batch_destroy(wlc_batch* b);
 typedef struct wlc_unet wlc_unet;
 int wlc_unet_create(int n, int batch, unsigned long long seed, wlc_unet** out);
 /* new grid edge (multiple of 8) and batch for the next calls; parameters and Adam state kept
- * (the network is fully convolutional) */
+ * (the network is fully convolutional).  After WLC_ENOMEM the network has no buffers: forward and
+ * gradients return WLC_ESTATE until a resize succeeds */
 int wlc_unet_resize(wlc_unet* u, int n, int batch);
 /* trainable parameters (padded = 1: the flat layout's length, including zero padding) */
 long long wlc_unet_num_params(const wlc_unet* u, int padded);

@@ -717,7 +717,7 @@ using namespace wlc::nn;
 struct wlc_unet {
   int device = 0;
   hipStream_t st = nullptr;
-  int n = 0, B = 0;
+  int n = 0, B = 0;       // 0: no buffers (a resize failed)
   std::vector<Layer> layers;
   PackTable pack{};
   long long np = 0;       // flat parameter count (padded)
@@ -761,9 +761,9 @@ int ualloc(std::vector<void*>& list, T** ptr, long long count) {
   void* q = nullptr;
   if (hipMalloc(&q, sizeof(T) * (size_t)std::max<long long>(count, 1)) != hipSuccess)
     return ufail(WLC_ENOMEM, "device allocation failed (warm-start network)");
+  list.push_back(q);
   if (hipMemset(q, 0, sizeof(T) * (size_t)std::max<long long>(count, 1)) != hipSuccess)
     return ufail(WLC_EHIP, "device initialisation failed (warm-start network)");
-  list.push_back(q);
   *ptr = static_cast<T*>(q);
   return WLC_OK;
 }
@@ -771,6 +771,7 @@ int ualloc(std::vector<void*>& list, T** ptr, long long count) {
 void free_acts(wlc_unet* u) {
   for (void* q : u->acts) (void)hipFree(q);
   u->acts.clear();
+  u->n = u->B = 0;
 }
 
 void unet_free(wlc_unet* u) {
@@ -849,58 +850,68 @@ int launch_grads(hipStream_t st, const GradJobs* all, const GradJobs* rows, bool
   return WLC_OK;
 }
 
-// activation, gradient and scratch buffers for grid edge n and batch B
+// places of the activation, gradient and scratch buffers of u's grid edge and batch from `base`
+// on, the gradient jobs of all layers into `all`; the bytes they take
+size_t lay_acts(wlc_unet* u, uintptr_t base, std::vector<GradJob>& all) {
+  size_t bytes = 0;
+  auto take = [&](auto*& ptr, long long count) {
+    ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(base + bytes);
+    bytes += (sizeof(*ptr) * (size_t)std::max<long long>(count, 1) + 255) / 256 * 256;
+  };
+#define UA(ptr, cnt) take(ptr, cnt)
+  const long long V0 = u->vol(0).voxels(), V1 = u->vol(1).voxels(), V2 = u->vol(2).voxels(), V3 = u->vol(3).voxels();
+  UA(u->lpart, 256);
+  UA(u->x0, V0 * 16); UA(u->a0a, V0 * 32); UA(u->p1, V1 * 32); UA(u->a1a, V1 * 64);
+  UA(u->p2, V2 * 64); UA(u->a2a, V2 * 128); UA(u->p3, V3 * 128);
+  UA(u->c2, V2 * 256); UA(u->c1, V1 * 128); UA(u->c0, V0 * 64); UA(u->d0, V0 * 32);
+  UA(u->gp1, V1 * 32); UA(u->gp2, V2 * 64); UA(u->gp3, V3 * 128);
+  UA(u->gc2, V2 * 256); UA(u->gc1, V1 * 128); UA(u->gc0, V0 * 64);
+  UA(u->y, V0 * 3); UA(u->xin, V0 * 11); UA(u->target, V0 * 3);
+  const bf16* X[11] = {u->x0, u->a0a, u->p1, u->a1a, u->p2, u->a2a, u->p3, u->c2, u->c1, u->c0, u->d0};
+  all.clear();
+  for (int li = 0; li < 11; ++li) {
+    const Layer& l = u->layers[li];
+    const Vol g = u->vol(l.level);
+    const long long V = g.voxels();
+    UA(u->dy[li], V * l.cout); UA(u->dyb[li], V * l.cout);
+    GradJob q = grad_job(g, l.cin, l.cout);
+    q.X = X[li];
+    q.dYb = u->dyb[li];
+    q.dYf = u->dy[li];
+    q.dW = u->g + l.woff;
+    q.db = u->g + l.boff;
+    UA(q.part, part_floats(q));
+    UA(q.bpart, (long long)q.nbp * l.cout);
+    if (grad_rows(g)) {
+      UA(q.xt, V * l.cin);
+      UA(q.dyt, V * l.cout);
+    }
+    all.push_back(q);
+  }
+  UA(u->djobs, 1); UA(u->dall, 1);
+#undef UA
+  return bytes;
+}
+
+// activation, gradient and scratch buffers for grid edge n and batch B: one allocation for all of
+// them, cleared at once (a hundred of them one by one took 50 ms), its size learned from a copy of
+// the network.  Both sizes need not fit at once, so the old buffers go first; without new ones the
+// network has none (n = B = 0) and refuses to run until a resize succeeds.
 int alloc_acts(wlc_unet* u, int n, int B) {
   free_acts(u);
+  std::vector<GradJob> all;
+  wlc_unet dry = *u;
+  dry.n = n;
+  dry.B = B;
+  const size_t bytes = lay_acts(&dry, 0, all);
+  char* block = nullptr;
+  if (const int rc = ualloc(u->acts, &block, (long long)bytes)) {
+    free_acts(u);
+    return rc;
+  }
   u->n = n;
   u->B = B;
-  // one allocation for all of them, cleared at once (a hundred of them one by one took 50 ms):
-  // laid out without a base to learn the size, then with it
-  std::vector<GradJob> all;
-  size_t bytes = 0;
-  auto lay = [&](uintptr_t base) {
-    bytes = 0;
-    auto take = [&](auto*& ptr, long long count) {
-      ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(base + bytes);
-      bytes += (sizeof(*ptr) * (size_t)std::max<long long>(count, 1) + 255) / 256 * 256;
-    };
-#define UA(ptr, cnt) take(ptr, cnt)
-    const long long V0 = u->vol(0).voxels(), V1 = u->vol(1).voxels(), V2 = u->vol(2).voxels(), V3 = u->vol(3).voxels();
-    UA(u->lpart, 256);
-    UA(u->x0, V0 * 16); UA(u->a0a, V0 * 32); UA(u->p1, V1 * 32); UA(u->a1a, V1 * 64);
-    UA(u->p2, V2 * 64); UA(u->a2a, V2 * 128); UA(u->p3, V3 * 128);
-    UA(u->c2, V2 * 256); UA(u->c1, V1 * 128); UA(u->c0, V0 * 64); UA(u->d0, V0 * 32);
-    UA(u->gp1, V1 * 32); UA(u->gp2, V2 * 64); UA(u->gp3, V3 * 128);
-    UA(u->gc2, V2 * 256); UA(u->gc1, V1 * 128); UA(u->gc0, V0 * 64);
-    UA(u->y, V0 * 3); UA(u->xin, V0 * 11); UA(u->target, V0 * 3);
-    const bf16* X[11] = {u->x0, u->a0a, u->p1, u->a1a, u->p2, u->a2a, u->p3, u->c2, u->c1, u->c0, u->d0};
-    all.clear();
-    for (int li = 0; li < 11; ++li) {
-      const Layer& l = u->layers[li];
-      const Vol g = u->vol(l.level);
-      const long long V = g.voxels();
-      UA(u->dy[li], V * l.cout); UA(u->dyb[li], V * l.cout);
-      GradJob q = grad_job(g, l.cin, l.cout);
-      q.X = X[li];
-      q.dYb = u->dyb[li];
-      q.dYf = u->dy[li];
-      q.dW = u->g + l.woff;
-      q.db = u->g + l.boff;
-      UA(q.part, part_floats(q));
-      UA(q.bpart, (long long)q.nbp * l.cout);
-      if (grad_rows(g)) {
-        UA(q.xt, V * l.cin);
-        UA(q.dyt, V * l.cout);
-      }
-      all.push_back(q);
-    }
-    UA(u->djobs, 1); UA(u->dall, 1);
-#undef UA
-  };
-  lay(0);
-  char* block = nullptr;
-  if (const int rc = ualloc(u->acts, &block, (long long)bytes)) return rc;
-  lay(reinterpret_cast<uintptr_t>(block));
+  lay_acts(u, reinterpret_cast<uintptr_t>(block), all);
   u->jobs.clear();
   u->odd.clear();
   // launches 0 .. 2 run over the layers of the transposed kernel, 3 .. 5 over all of them
@@ -1039,6 +1050,7 @@ int backward(wlc_unet* u, float* loss) {
 // input [B][n^3][11] (host FP32), converted on the device; targets [B][n^3][3].  The caller waits
 // for the stream before it returns (the host arrays are read until then).
 int upload(wlc_unet* u, const float* x, const float* t) {
+  if (!u->B) return ufail(WLC_ESTATE, "the network has no buffers: its last resize failed");
   const long long V = u->vol(0).voxels();
   UCHK(hipMemcpyAsync(u->xin, x, sizeof(float) * (size_t)V * 11, hipMemcpyHostToDevice, u->st));
   hipLaunchKernelGGL(k_input, dim3(blocks(V * 16)), dim3(256), 0, u->st, u->xin, u->x0, V);
@@ -1066,8 +1078,6 @@ int wlc_unet_create(int n, int batch, unsigned long long seed, wlc_unet** out) {
   if ((long long)batch * n * n * n * 256 >= (1LL << 31))
     return ufail(WLC_EINVAL, "batch x grid too large (the kernels index an activation tensor with 32 bits)");
   wlc_unet* u = new wlc_unet();
-  u->n = n;
-  u->B = batch;
   if (hipGetDevice(&u->device) != hipSuccess || hipStreamCreateWithFlags(&u->st, hipStreamNonBlocking) != hipSuccess) {
     delete u;
     return ufail(WLC_EHIP, "no HIP device / stream");
