@@ -138,7 +138,8 @@ struct EpiAct {
     }
   }
 };
-// gradient of a pre-activation: the sum where the activation is positive, FP32 and bf16
+// gradient of a pre-activation: the sum where the activation is positive (not where it is NaN),
+// FP32 and bf16
 struct EpiMask {
   const bf16* act;
   float* dy;
@@ -150,7 +151,7 @@ struct EpiMask {
     us4 h;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      s[r] = m[r] ? s[r] : 0.f;  // an activation is never negative
+      s[r] = bf2f(m[r]) > 0.f ? s[r] : 0.f;
       h[r] = f2bf(s[r]);
     }
     *reinterpret_cast<f32x4*>(dy + at) = s;
@@ -586,7 +587,7 @@ __global__ void k_up_back(const float* __restrict__ dfine, const bf16* __restric
   us4 h;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    s[r] = m[r] ? s[r] : 0.f;
+    s[r] = bf2f(m[r]) > 0.f ? s[r] : 0.f;
     h[r] = f2bf(s[r]);
   }
   *reinterpret_cast<f32x4*>(dy + vo * C + c) = s;
@@ -616,7 +617,7 @@ __global__ void k_skip_back(const float* __restrict__ dcat, const float* __restr
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     s[r] += p[r] * 0.125f;
-    s[r] = m[r] ? s[r] : 0.f;
+    s[r] = bf2f(m[r]) > 0.f ? s[r] : 0.f;
     h[r] = f2bf(s[r]);
   }
   *reinterpret_cast<f32x4*>(dy + v * C + c) = s;
