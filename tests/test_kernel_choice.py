@@ -1,0 +1,64 @@
+"""Where the library changes from one kernel to another by the size of a launch: which kernel runs on
+either side of the line (on the host, launches recorded), and both sides against the oracle."""
+import numpy as np
+import pytest
+
+import host_hip
+
+TOL = 1e-10  # the repository's parity bound (FP64 path)
+
+SWEEP = """
+    shape, Nblk, L, sp = {shape}, {Nblk}, {L}, {sp}
+    g = W.WormlikeMDE(shape, (3.0, 3.5, 4.0), Nblk, L, (1.0,) * len(L), spectrum_fp32=sp)
+    g.set_w(np.zeros((len(L),) + shape))
+    H.host_hip_forget()
+    g.MDE_q()
+    print("\\n".join(launches()))
+"""
+
+
+@pytest.fixture(scope="module")
+def so(tmp_path_factory):
+    return host_hip.build(tmp_path_factory.mktemp("host_hip"))
+
+
+def _launches(so, shape, Nblk, L, sp=False):
+    return host_hip.run(so, SWEEP.format(shape=shape, Nblk=Nblk, L=L, sp=sp))
+
+
+def _matches_oracle(wlc, oracle, shape, Nblk, L):
+    box, lam = tuple(0.12 * e + 0.5 for e in shape[::-1]), (1.0, 0.5, 2.0)[:len(L)]
+    w = 1.5 * np.random.default_rng(sum(shape)).standard_normal((len(L),) + shape)
+    orc = oracle.Oracle(shape, box, Nblk, L, lam)
+    g = wlc.WormlikeMDE(shape, box, Nblk, L, lam, keep_qstar=True)
+    g.set_w(w)
+    g.MDE_q()
+    g.MDE_qstar()
+    for d, ref in ((1, orc.forward(w)), (-1, orc.backward(w))):
+        for s in range(sum(Nblk) + 1):
+            a, b = g.get_q(d, s), orc.slice(ref, s)
+            assert np.abs(a - b).max() < TOL * np.abs(b).max(), (d, s)
+    g.close()
+    orc.close()
+
+
+# 48 x 72 planes: two-pass kernels up to 512 planes of a launch, the run-time kernels above; a chain
+# whose Lmax changes crosses the line
+def test_planes_of_five_waves(so):
+    for ny, nx in ((48, 72), (72, 48)):
+        for nz, L, two in ((32, (3,), True), (36, (3,), False), (18, (4,), True), (24, (4,), False)):
+            k = [x for x in _launches(so, (nz, ny, nx), (4,), L) if "k2_" in x or "rhs" in x or "ifft" in x]
+            assert len(k) == 5 and all(("k2_" in x) == two for x in k), (ny, nx, nz, L)
+    k = [x for x in _launches(so, (36, 48, 72), (3, 3), (2, 3)) if "k2_" in x or "rhs" in x or "ifft" in x]
+    assert [("k2_" in x) for x in k] == [True, True, True, False, False, False, False]
+    # other planes keep the two-pass kernels at any number
+    for ny, nx in ((54, 72), (64, 72), (72, 72), (36, 72)):
+        k = _launches(so, (72, ny, nx), (4,), (4,))
+        assert sum("k2_" in x for x in k) == 5, (ny, nx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ny,nx", [(48, 72), (72, 48)])
+def test_planes_of_five_waves_match_oracle(wlc, oracle, ny, nx):
+    # 324 planes, then 576
+    _matches_oracle(wlc, oracle, (36, ny, nx), (3, 3), (2, 3))

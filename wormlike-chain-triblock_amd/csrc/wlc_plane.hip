@@ -396,7 +396,17 @@ static bool specialised(const Geom& g) {
 // FP64 spectrum only: with the FP32 one another order of the same operations rounds some stored
 // values the other way, which after 40 to 100 steps moves phi by 1e-9 to 1e-7 of itself, as far as
 // the storage type itself does, so that mode keeps the kernels and with them its results
-static bool two_pass_plane(const Geom& g) { return !g.spec32 && !specialised(g) && p2::takes(g.nx, g.ny); }
+static bool two_pass_plane(const Geom& g, int planes) {
+  if (g.spec32 || specialised(g) || !p2::takes(g.nx, g.ny)) return false;
+  // 48 x 72 and 72 x 48: a two-pass plane is five waves, and a CU holds one at a time (two waves per
+  // SIMD), while the run-time kernel keeps these planes in eight slots a thread.  From about two
+  // planes per CU on that one is faster: C + A of 72 x 48 with 400 planes 37.3 us against 31.2 us of
+  // the two-pass kernel, with 576 44.4 against 45.3, 1024 52.2 against 61.4, 3136 152 against 187.
+  // (72 x 64, 64 x 72 and 72 x 72, five and six waves, need sixteen slots there: 0.94 to 1.00 of
+  // its time.)
+  const bool one_per_cu = p2::shape_of(g.nx, g.ny).waves > 4;
+  return !(one_per_cu && pick_maxe((long long)g.ny * g.nxh, kThreads) == 8 && planes > 512);
+}
 
 static size_t plane_lds_bytes(const Geom& g) {
   const size_t n = (size_t)g.ny * g.nxh;
@@ -429,10 +439,10 @@ static void* p128_kernel(int kind) {
   return kind == 0 ? (void*)p128::k_rhs128<ORDER, S> : (void*)p128::k_inv_rhs128<ORDER, S>;
 }
 
-// kind 0: A (order), 1: C, 2: fused C + A (order of the next step); *threads = workgroup
-// size; S = storage type of the half spectrum; B: the batched twin
+// kind 0: A (order), 1: C, 2: fused C + A (order of the next step); planes: of the launch (nz times
+// harmonics); *threads = workgroup size; S = storage type of the half spectrum; B: the batched twin
 template <class S, bool B>
-static void* pick_plane_kernel_t(const Geom& g, int kind, int order, size_t* lds, int* threads) {
+static void* pick_plane_kernel_t(const Geom& g, int kind, int order, int planes, size_t* lds, int* threads) {
   *lds = plane_lds_bytes(g);
   *threads = kThreads;
   if (g.nx == 64 && g.ny == 64) {  // static 32 KB plane
@@ -456,7 +466,7 @@ static void* pick_plane_kernel_t(const Geom& g, int kind, int order, size_t* lds
     }
     return nullptr;
   }
-  if (two_pass_plane(g)) {
+  if (two_pass_plane(g, planes)) {
     *lds = p2::lds_bytes(g.nx, g.ny);
     *threads = 64 * p2::shape_of(g.nx, g.ny).waves;
     return const_cast<void*>(p2::kernel(g.nx, g.ny, kind, B));
@@ -479,20 +489,20 @@ static void* pick_plane_kernel_t(const Geom& g, int kind, int order, size_t* lds
   return nullptr;
 }
 
-static void* pick_plane_kernel(const Geom& g, int kind, int order, size_t* lds, int* threads,
+static void* pick_plane_kernel(const Geom& g, int kind, int order, int planes, size_t* lds, int* threads,
                                bool batch = false) {
   if (batch)
-    return g.spec32 ? pick_plane_kernel_t<float2, true>(g, kind, order, lds, threads)
-                    : pick_plane_kernel_t<double2, true>(g, kind, order, lds, threads);
-  return g.spec32 ? pick_plane_kernel_t<float2, false>(g, kind, order, lds, threads)
-                  : pick_plane_kernel_t<double2, false>(g, kind, order, lds, threads);
+    return g.spec32 ? pick_plane_kernel_t<float2, true>(g, kind, order, planes, lds, threads)
+                    : pick_plane_kernel_t<double2, true>(g, kind, order, planes, lds, threads);
+  return g.spec32 ? pick_plane_kernel_t<float2, false>(g, kind, order, planes, lds, threads)
+                  : pick_plane_kernel_t<double2, false>(g, kind, order, planes, lds, threads);
 }
 
 static hipError_t launch_plane(const Geom& g, int kind, int order, int planes, void** args,
                                hipStream_t st) {
   size_t lds = 0;
   int threads = kThreads;
-  void* k = pick_plane_kernel(g, kind, order, &lds, &threads);
+  void* k = pick_plane_kernel(g, kind, order, g.nz * planes, &lds, &threads);
   if (!k) return hipErrorInvalidValue;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -527,7 +537,7 @@ hipError_t launch_inv_rhs(const Geom& g, const InvArgs& c, const RhsArgs& a, int
 LaunchKey plane_key(const Geom& g, int kind, int order, int planes) {
   size_t lds = 0;
   int threads = kThreads;
-  const void* k = pick_plane_kernel(g, kind, order, &lds, &threads);
+  const void* k = pick_plane_kernel(g, kind, order, g.nz * planes, &lds, &threads);
   return LaunchKey{k, (unsigned)(g.nz * planes), 1u, (unsigned)threads, lds};
 }
 
@@ -536,7 +546,7 @@ static hipError_t launch_plane_batch(const Geom& g, int kind, int order, int pla
   if (n <= 0) return hipSuccess;
   size_t lds = 0;
   int threads = kThreads;
-  void* k = pick_plane_kernel(g, kind, order, &lds, &threads, true);
+  void* k = pick_plane_kernel(g, kind, order, g.nz * planes, &lds, &threads, true);
   if (!k) return hipErrorInvalidValue;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
