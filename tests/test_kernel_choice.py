@@ -62,3 +62,30 @@ def test_planes_of_five_waves(so):
 def test_planes_of_five_waves_match_oracle(wlc, oracle, ny, nx):
     # 324 planes, then 576
     _matches_oracle(wlc, oracle, (36, ny, nx), (3, 3), (2, 3))
+
+
+# short z axes at Lmax 0, 1 (and 2 at nz = 8): the column kernel up to a number of column groups (four
+# columns to nz = 16, else two), the generic kernel above
+@pytest.mark.parametrize("nz,L,line,few,many", [
+    (8, 0, 1024, (72, 108), (108, 72)), (12, 0, 1024, (72, 108), (108, 72)), (16, 1, 1024, (72, 108), (108, 72)),
+    (24, 0, 1024, (72, 54), (64, 64)), (32, 1, 1024, (72, 54), (64, 64)), (48, 0, 640, (48, 48), (54, 48)),
+    (36, 0, 640, (48, 48), (54, 48)), (48, 1, 1024, (72, 54), (64, 64)), (18, 1, 3072, (108, 108), (128, 96)),
+    (54, 1, 1536, (72, 72), (108, 64)), (8, 2, 2048, (144, 108), (128, 128)), (36, 2, 4096, (128, 96), (128, 128)),
+    (48, 2, 2048, (72, 72), (96, 96)),
+])
+def test_few_harmonics_many_columns(so, nz, L, line, few, many):
+    cols = 4 if nz <= 16 else 2
+    for (ny, nx), col in ((few, True), (many, False)):
+        assert (-(-(nx // 2 + 1) // cols) * ny <= line) == col
+        k = [x for x in _launches(so, (nz, ny, nx), (4,), (L,)) if "zcol" in x or "zsolve" in x]
+        assert len(k) == 4 and all(("zcol" in x) == col for x in k), (ny, nx)
+    # more harmonics: the column kernel at any number of columns
+    k = [x for x in _launches(so, (nz, *many), (4,), (3,)) if "zcol" in x or "zsolve" in x]
+    assert len(k) == 4 and all("zcol" in x for x in k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,L", [((24, 64, 64), (0, 1)), ((8, 108, 72), (1, 0)), ((18, 128, 96), (1, 2)),
+                                     ((8, 128, 128), (2, 3))])
+def test_few_harmonics_many_columns_match_oracle(wlc, oracle, shape, L):
+    _matches_oracle(wlc, oracle, shape, (3, 2), L)

@@ -24,12 +24,35 @@ const void* z128_kernel_L7(bool, bool);
 const void* z128_kernel_L8(bool, bool);
 
 namespace {
+// Column groups up to which the column kernel is the faster one for short z axes.  It spreads the
+// harmonics of a group over a workgroup: with one to four of them most of its threads idle, which
+// costs nothing while the groups fit the GPU together and the most where they take many rounds, and
+// there the generic kernel's thread per k-point is faster.  Per launch, generic / column kernel:
+// Lmax 0, 48^2 x 48 (624 groups) 10.1 / 10.0 us, 72 x 54 x 48 (1008) 10.5 / 12.6, 128^2 x 48 19.7 /
+// 31.5, 54^2 x 24 (756) 8.1 / 7.3, 64^2 x 24 (1088) 8.1 / 9.2, 108 x 72 x 8 (1080) and on 7.5 / 9.2;
+// Lmax 1, 48^2 x 36 13.7 / 12.5, 64^2 x 36 16.3 / 16.8, 128^2 x 48 32.2 / 44.2.  The generic
+// transform of 18 and 54 has the most radix-3 passes: Lmax 1, 64^2 x 54 20.9 / 18.4, 108 x 72 x 54
+// (2016) 24.8 / 26.4; 96^2 x 18 (2352) 16.5 / 16.7, 128^2 x 18 22.3 / 22.0.  At Lmax 2 the column
+// kernel is behind only with very many groups: 128^2 x 8 (2176) 15.8 / 17.2; where the two sweeps
+// run at once, its LDS beside the planes' of 96^2 and 128^2 costs more than it gains: pair of sweeps
+// of 60 steps on 96^2 x 48 (2400) 12.7 / 13.3 ms, of 160 on 128^2 x 48 (4224) 38.9 / 40.4, of 80 on
+// 128^2 x 36 16.2 / 16.7, but 96^2 x 36 11.0 / 10.8.  Above that nowhere.
+unsigned zcol_groups(int nz, int L) {
+  const bool slow3 = nz == 18 || nz == 54, wide = nz == 36 || nz == 48;
+  if (L == 0) return wide ? 640 : 1024;
+  if (L == 1) return slow3 ? (nz == 18 ? 3072 : 1536) : 1024;
+  if (L == 2) return nz == 8 || nz == 48 ? 2048 : nz == 36 ? 4096 : ~0u;
+  return ~0u;
+}
+
 // short z axes with the FP64 spectrum take the column kernel unless the generic kernel or its
 // degree split (1) is asked for; with the FP32 spectrum the generic ones, as before the column
 // kernel: another order of the same operations rounds some stored values the other way, which
 // moves phi by up to 1e-7 of itself after 40 to 100 steps
 bool use_zcol(const Geom& g, const SolveArgs& a) {
-  return zcol_nz(g.nz) && !g.spec32 && !a.generic && a.split >= 2 && a.M == (a.L + 1) * (a.L + 1);
+  if (!zcol_nz(g.nz) || g.spec32 || a.generic || a.split < 2 || a.M != (a.L + 1) * (a.L + 1)) return false;
+  const int cols = 1 << zcol_log2_cols(g.nz);
+  return unsigned((g.nxh + cols - 1) / cols * g.ny) <= zcol_groups(g.nz, a.L);
 }
 
 // nz = 128 with a degree split asked for: the three-part kernel
