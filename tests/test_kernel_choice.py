@@ -89,3 +89,47 @@ def test_few_harmonics_many_columns(so, nz, L, line, few, many):
                                      ((8, 128, 128), (2, 3))])
 def test_few_harmonics_many_columns_match_oracle(wlc, oracle, shape, L):
     _matches_oracle(wlc, oracle, shape, (3, 2), L)
+
+
+# nz = 48, Lmax 7: the column kernel up to 960 column groups, a half-tile kernel above
+def test_nz48_lmax7(so):
+    for (ny, nx), col in (((54, 54), True), ((48, 72), True), ((72, 54), False), ((64, 64), False)):
+        k = [x for x in _launches(so, (48, ny, nx), (4,), (7,)) if "zcol" in x or "zsolve" in x]
+        assert len(k) == 4 and all(("zcol" in x) == col and ("zsolve48" in x) != col for x in k), (ny, nx)
+    # other Lmax, and the FP32 spectrum: as at any number of columns
+    for L, sp in ((6, False), (8, False), (7, True)):
+        k = [x for x in _launches(so, (48, 64, 64), (4,), (L,), sp) if "zcol" in x or "zsolve" in x]
+        assert len(k) == 4 and all("zsolve48" not in x and ("zcol" in x) != sp for x in k), (L, sp)
+
+
+@pytest.mark.gpu
+def test_nz48_lmax7_matches_oracle(wlc, oracle):
+    # nxh = 33 and 37: a tile of one real column; blocks of the other Lmax take the column kernel
+    for shape, L in (((48, 64, 64), (7,)), ((48, 64, 72), (7, 2))):
+        _matches_oracle(wlc, oracle, shape, (3, 2)[:len(L)], L)
+
+
+@pytest.mark.gpu
+def test_nz48_lmax7_batched(wlc):
+    # rows of half tiles in and out of the XCD order (2 nt ny a multiple of 16 or not)
+    cases = []
+    for shape in ((48, 64, 64), (48, 64, 64), (48, 54, 72)):
+        w = 1.5 * np.random.default_rng(len(cases)).standard_normal((1,) + shape)
+        cases.append(dict(shape=shape, box=(4.0, 3.5, 3.0), Nblk=(3,), L=(7,), lam=(1.0,), w=w,
+                          chi=np.array([[0, 15, 0], [15, 0, 0], [0, 0, 0]], float)))
+    b = wlc.Batch(cases)
+    for i, c in enumerate(cases):
+        b.set_w(i, c["w"])
+    b.sweep()
+    for i, c in enumerate(cases):
+        g = wlc.WormlikeMDE(c["shape"], c["box"], c["Nblk"], c["L"], c["lam"])
+        g.set_w(c["w"])
+        g.MDE_q()
+        g.MDE_qstar()
+        phi, Q, td = g.density()
+        bphi, bQ, btd = b.density(i)
+        # the twins run the same operations; contraction may differ
+        assert np.abs(bphi - phi).max() < 1e-13 * np.abs(phi).max()
+        assert abs(bQ - Q) / Q < 1e-13 and abs(btd - td) / td < 1e-13
+        g.close()
+    b.close()

@@ -36,11 +36,13 @@ namespace {
 // kernel is behind only with very many groups: 128^2 x 8 (2176) 15.8 / 17.2; where the two sweeps
 // run at once, its LDS beside the planes' of 96^2 and 128^2 costs more than it gains: pair of sweeps
 // of 60 steps on 96^2 x 48 (2400) 12.7 / 13.3 ms, of 160 on 128^2 x 48 (4224) 38.9 / 40.4, of 80 on
-// 128^2 x 36 16.2 / 16.7, but 96^2 x 36 11.0 / 10.8.  Above that nowhere.
+// 128^2 x 36 16.2 / 16.7, but 96^2 x 36 11.0 / 10.8.  Above that nowhere, but at Lmax 7 nz = 48 has a
+// kernel of its own for many columns (k_zsolve48 in wlc_zsolve.hip).
 unsigned zcol_groups(int nz, int L) {
   const bool slow3 = nz == 18 || nz == 54, wide = nz == 36 || nz == 48;
   if (L == 0) return wide ? 640 : 1024;
   if (L == 1) return slow3 ? (nz == 18 ? 3072 : 1536) : 1024;
+  if (L == 7 && nz == 48) return 960;
   if (L == 2) return nz == 8 || nz == 48 ? 2048 : nz == 36 ? 4096 : ~0u;
   return ~0u;
 }

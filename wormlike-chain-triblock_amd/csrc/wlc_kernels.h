@@ -67,12 +67,14 @@ struct SolveArgs {
   int occ;             // nz = 64 kernel: target waves per SIMD (1 or 2)
   int split;           // how the work of a k-point is split.  nz of the column kernel (wlc_zcol.h):
                        // 0 one thread per k-point and 1 two, by degree (Lmax 4-7), both generic;
-                       // 2, 3 the column kernel.  nz = 64 (Lmax 5-7; else 0): 0 one wave per
-                       // column, else two by degree: 1 two columns per workgroup, loaded
-                       // directly, 2 a whole 4-kx tile per workgroup, 3 half a tile, both
-                       // through LDS (2 and 3: FP64 spectrum; FP32 runs as 1).  nz = 128, Lmax
-                       // 5-8: 0 whole columns per wave pair, else the three-part kernel
-                       // (wlc_z128.h).  Other nz, Lmax 4-7: any nonzero value splits by degree
+                       // 2, 3 the column kernel (with few harmonics on many columns the generic
+                       // one, at nz = 48 and Lmax 7 on many columns k_zsolve48).  nz = 64 (Lmax
+                       // 5-7; else 0): 0 one wave per column, else two by degree: 1 two columns
+                       // per workgroup, loaded directly, 2 a whole 4-kx tile per workgroup, 3
+                       // half a tile, both through LDS (2 and 3: FP64 spectrum; FP32 runs as 1).
+                       // nz = 128, Lmax 5-8: 0 whole columns per wave pair, else the three-part
+                       // kernel (wlc_z128.h).  Other nz, Lmax 4-7: any nonzero value splits by
+                       // degree
 };
 
 // Kernel C: inverse y and x (C2R) passes, scaling by 1/N, store of q(s).

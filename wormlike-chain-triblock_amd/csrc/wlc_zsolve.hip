@@ -11,7 +11,7 @@
 
 #include <type_traits>
 
-#include "wlc_device.h"
+#include "wlc_dft.h"
 
 #ifndef WLC_L
 #error "compile with -DWLC_L=<Lmax>"
@@ -698,6 +698,178 @@ __global__ void __launch_bounds__(256, 2) k_zsolve64p_b(const ZJob* __restrict__
 }
 
 // ---------------------------------------------------------------------------
+// nz = 48, Lmax 7, many columns: the half-tile split kernel with a wave-local transform
+// ---------------------------------------------------------------------------
+// Same workgroup shape as k_zsolve64p (four waves: two columns x two degree parts, two
+// workgroups per CU; the halves of a tile are blocks b and b + 8 on one XCD), lane = z for
+// lanes 0..47 (the others hold zeros through the solve).  The 48-point transform of a batch of
+// eight harmonics is a four-step 6 x 8 in the wave's LDS region: with n = j + 6 m and
+// k = k1 + 8 k2, a DFT-8 over m for each (harmonic, j) (48 lanes), the twiddle W48^(j k1), then
+// a DFT-6 over j for each (harmonic, k1) (64 lanes).
+// The column kernel of the short axes (wlc_zcol.hip) needs 98 KB of LDS here, one workgroup per
+// CU; where the columns take several rounds this one is faster (72^2 x 48 102.7 against 120.7 us,
+// 128^2 x 48 356 against 406, 72 x 54 x 48 88 against 93; with fewer, 54^2 72.4 against 61.4).  FP64 spectrum.
+#if WLC_L == 7
+constexpr int kN48 = 48;
+constexpr int kPad48 = kN48 + kN48 / 8;  // padded units per harmonic (pad8(47) < kPad48)
+constexpr int kRegion48 = (kHB * kPad48 + 2) > (kXch + 2) ? (kHB * kPad48 + 2) : (kXch + 2);
+
+// the 48-point transforms of the eight harmonics in region wl (element z of slot h at
+// wl[h kPad48 + pad8(z)]), in place; DIR < 0 forward, DIR > 0 inverse (unnormalised)
+template <int DIR>
+__device__ __forceinline__ void z48_batch(double2* wl, int lane, const double2* __restrict__ twz) {
+  constexpr int N1 = kN48 / 8, P = kPad48;
+  if (lane < kN48) {
+    const int h = lane / N1, j = lane - N1 * (lane / N1);
+    double2 u[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) u[m] = wl[h * P + pad8(j + N1 * m)];
+    Dft<8, DIR>::run(u);
+#pragma unroll
+    for (int k1 = 1; k1 < 8; ++k1) u[k1] = twiddle<DIR>(u[k1], twz[j * k1]);
+    // the positions j + N1 k1 this lane writes are the ones it read
+#pragma unroll
+    for (int k1 = 0; k1 < 8; ++k1) wl[h * P + pad8(j + N1 * k1)] = u[k1];
+  }
+  wave_sync();
+  {
+    const int h = lane >> 3, k1 = lane & 7;
+    double2 u[N1];
+#pragma unroll
+    for (int j = 0; j < N1; ++j) u[j] = wl[h * P + pad8(j + N1 * k1)];
+    Dft<N1, DIR>::run(u);
+    wave_sync();  // every lane has read its inputs before any output overwrites them
+#pragma unroll
+    for (int k2 = 0; k2 < N1; ++k2) wl[h * P + pad8(k1 + 8 * k2)] = u[k2];
+  }
+  wave_sync();
+}
+
+__device__ __forceinline__ void k_zsolve48_body(const Geom& g, const SolveArgs& a) {
+  extern __shared__ double2 lds[];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int part = wv >> 1, c = wv & 1, gi = threadIdx.x & 127;
+  const int ny = g.ny, nxh = g.nxh, nt = g.nt;
+  const int nb = gridDim.x, b = blockIdx.x;
+  int tl, half;
+  if ((nb & 15) == 0) {
+    const int t = b >> 3;
+    half = t & 1;
+    tl = (t >> 1) * 8 + (b & 7);
+  } else {
+    half = b & 1;
+    tl = b >> 1;
+  }
+  const int t4 = tl % nt, ky = tl / nt;
+  if (t4 * kKxTile + 2 * half >= nxh) return;  // both columns are padding (uniform)
+  const int kx = t4 * kKxTile + 2 * half + c;
+  const bool real_col = kx < nxh;  // wave-uniform
+  // thread gi of a part moves element (z = gi / 2, column gi % 2) of each harmonic
+  const int tz = gi >> 1, tc = gi & 1;
+  const bool io = tz < kN48 && t4 * kKxTile + 2 * half + tc < nxh;
+  const int go = kKxTile * tz + tc;
+  const bool active = a.solve && real_col;
+  const long long istride = spec_index(1, 0, 0, 0, ny, nt, kN48);
+  const int nh = part ? PartHi::NH : PartLo::NH;
+  const int hb0 = part ? PartHi::B0 : PartLo::B0;
+  double2* hp = reinterpret_cast<double2*>(a.spec) + spec_index(0, ky, t4 * kKxTile, 0, ny, nt, kN48) + 2 * half +
+          (long long)hb0 * istride;
+  double2* glds = lds + part * (2 * kRegion48);
+  double2* wl = glds + c * kRegion48;
+  double2* xch = lds + c * kRegion48;  // the Lo wave's region of column c
+  const double2* twz = g.az.tw;        // exp(-2 pi i t / 48)
+  const int zl = lane < kN48 ? lane : 0;
+  const KFrame f(signed_k(kx, g.nx) * a.kfac[0], signed_k(ky, ny) * a.kfac[1],
+                 signed_k(zl, kN48) * a.kfac[2], a.sigma, a.ds);
+  double2 v[kNV];
+#pragma unroll
+  for (int q = 0; q < kNV; ++q) v[q] = make_double2(0.0, 0.0);
+  // forward: per batch of eight harmonics, the part's tiles into LDS (the next batch's loads
+  // in flight), the 48-point transforms, lane = kz back into registers
+  double2 nxt[kHB];
+#pragma unroll
+  for (int q = 0; q < kHB; ++q)
+    nxt[q] = (io && q < nh) ? spec_ld(hp + (long long)q * istride + go) : make_double2(0.0, 0.0);
+#pragma unroll
+  for (int bb = 0; bb < kNBt; ++bb) {
+    const int b0 = bb * kHB;
+    __syncthreads();  // every wave of the part has read the previous batch out of its region
+    if (tz < kN48) {
+#pragma unroll
+      for (int q = 0; q < kHB; ++q)
+        if (b0 + q < nh) glds[tc * kRegion48 + q * kPad48 + pad8(tz)] = nxt[q];
+    }
+    if (bb + 1 < kNBt) {
+#pragma unroll
+      for (int q = 0; q < kHB; ++q) {
+        const int hq = b0 + kHB + q;
+        nxt[q] = (io && hq < nh) ? spec_ld(hp + (long long)hq * istride + go) : make_double2(0.0, 0.0);
+      }
+    }
+    __syncthreads();
+    if (real_col && b0 < nh) {
+      z48_batch<-1>(wl, lane, twz);
+      if (lane < kN48) {
+#pragma unroll
+        for (int q = 0; q < kHB; ++q)
+          if (b0 + q < kNV && b0 + q < nh) v[b0 + q] = wl[q * kPad48 + pad8(lane)];
+      }
+    }
+  }
+  if (active) {
+    if (part == 0) {
+      PartLo::to_frame(v, f);
+      tri_lower_forward<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
+    } else {
+      PartHi::to_frame(v, f);
+    }
+  }
+  __syncthreads();
+  if (part == 1 && active) tri_upper<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
+  __syncthreads();
+  if (active) {
+    if (part == 0) {
+      tri_lower_back<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
+      PartLo::from_frame(v, f);
+    } else {
+      PartHi::from_frame(v, f);
+    }
+  }
+  // inverse: per batch, lane = kz into LDS, the inverse transforms, the tiles out
+#pragma unroll
+  for (int bb = 0; bb < kNBt; ++bb) {
+    const int b0 = bb * kHB;
+    __syncthreads();  // the previous batch's tiles (and the crossing chains) have been read
+    if (real_col && b0 < nh) {
+      if (lane < kN48) {
+#pragma unroll
+        for (int q = 0; q < kHB; ++q)
+          if (b0 + q < kNV && b0 + q < nh) wl[q * kPad48 + pad8(lane)] = v[b0 + q];
+      }
+      wave_sync();
+      z48_batch<+1>(wl, lane, twz);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kHB; ++q)
+      if (io && b0 + q < nh)
+        spec_st(hp + (long long)(b0 + q) * istride + go, glds[tc * kRegion48 + q * kPad48 + pad8(tz)]);
+  }
+}
+
+__global__ void __launch_bounds__(256, 2) k_zsolve48(Geom g, SolveArgs a) {
+  k_zsolve48_body(g, a);
+}
+
+// the same for one instance of a batch per blockIdx.z
+__global__ void __launch_bounds__(256, 2) k_zsolve48_b(const ZJob* __restrict__ jobs) {
+  const ZJob& j = jobs[blockIdx.z];
+  if (j.skip && *j.skip) return;
+  k_zsolve48_body(j.g, j.a);
+}
+#endif
+
+// ---------------------------------------------------------------------------
 // nz = 128: two waves per (kx, ky) column
 // ---------------------------------------------------------------------------
 // Wave p of a column works on z = m + 64 p (lane m).  Forward: one radix-2 decimation-
@@ -1020,6 +1192,18 @@ struct ZPlan {
 template <class S>
 hipError_t zsolve_plan(const Geom& g, const SolveArgs& a, ZPlan* z) {
   if (a.M != kM) return hipErrorInvalidValue;
+#if WLC_L == 7
+  if (g.nz == kN48 && !g.spec32 && !a.generic && a.split >= 2) {
+    // two workgroups of four waves per 4-kx tile; the grids with fewer columns took the column
+    // kernel before they came here
+    z->k1 = (const void*)k_zsolve48;
+    z->kb = (const void*)k_zsolve48_b;
+    z->grid = dim3(2 * g.nt * g.ny);
+    z->block = dim3(256);
+    z->lds = sizeof(double2) * (size_t)(2 * 2 * kRegion48);
+    return hipSuccess;
+  }
+#endif
   if constexpr (std::is_same<S, double2>::value) {
     // one workgroup of eight waves per 4-kx tile; FP64 spectrum only: with the FP32 half
     // spectrum (2 KB tiles) the two-column kernel below is faster (64^3/L6: 69 vs 93 us)
