@@ -5,7 +5,8 @@ import pytest
 
 import host_hip
 
-TOL = 1e-10  # the repository's parity bound (FP64 path)
+# the repository's parity bound (FP64 path) and its FP32-spectrum bound on short chains
+TOL, TOL32 = 1e-10, 2e-6
 
 SWEEP = """
     shape, Nblk, L, sp = {shape}, {Nblk}, {L}, {sp}
@@ -26,20 +27,44 @@ def _launches(so, shape, Nblk, L, sp=False):
     return host_hip.run(so, SWEEP.format(shape=shape, Nblk=Nblk, L=L, sp=sp))
 
 
-def _matches_oracle(wlc, oracle, shape, Nblk, L):
+def _matches_oracle(wlc, oracle, shape, Nblk, L, spec32=False):
     box, lam = tuple(0.12 * e + 0.5 for e in shape[::-1]), (1.0, 0.5, 2.0)[:len(L)]
     w = 1.5 * np.random.default_rng(sum(shape)).standard_normal((len(L),) + shape)
     orc = oracle.Oracle(shape, box, Nblk, L, lam)
-    g = wlc.WormlikeMDE(shape, box, Nblk, L, lam, keep_qstar=True)
+    g = wlc.WormlikeMDE(shape, box, Nblk, L, lam, keep_qstar=True, spectrum_fp32=spec32)
     g.set_w(w)
     g.MDE_q()
     g.MDE_qstar()
     for d, ref in ((1, orc.forward(w)), (-1, orc.backward(w))):
         for s in range(sum(Nblk) + 1):
             a, b = g.get_q(d, s), orc.slice(ref, s)
-            assert np.abs(a - b).max() < TOL * np.abs(b).max(), (d, s)
+            assert np.abs(a - b).max() < (TOL32 if spec32 else TOL) * np.abs(b).max(), (d, s)
     g.close()
     orc.close()
+
+
+def _batch_matches_handles(wlc, instances):
+    cases = []
+    for shape, L in instances:
+        w = 1.5 * np.random.default_rng(len(cases)).standard_normal((1,) + shape)
+        cases.append(dict(shape=shape, box=(4.0, 3.5, 3.0), Nblk=(3,), L=(L,), lam=(1.0,), w=w,
+                          chi=np.array([[0, 15, 0], [15, 0, 0], [0, 0, 0]], float)))
+    b = wlc.Batch(cases)
+    for i, c in enumerate(cases):
+        b.set_w(i, c["w"])
+    b.sweep()
+    for i, c in enumerate(cases):
+        g = wlc.WormlikeMDE(c["shape"], c["box"], c["Nblk"], c["L"], c["lam"])
+        g.set_w(c["w"])
+        g.MDE_q()
+        g.MDE_qstar()
+        phi, Q, td = g.density()
+        bphi, bQ, btd = b.density(i)
+        # the twins run the same operations; contraction may differ
+        assert np.abs(bphi - phi).max() < 1e-13 * np.abs(phi).max()
+        assert abs(bQ - Q) / Q < 1e-13 and abs(btd - td) / td < 1e-13
+        g.close()
+    b.close()
 
 
 # 48 x 72 planes: two-pass kernels up to 512 planes of a launch, the run-time kernels above; a chain
@@ -112,24 +137,30 @@ def test_nz48_lmax7_matches_oracle(wlc, oracle):
 @pytest.mark.gpu
 def test_nz48_lmax7_batched(wlc):
     # rows of half tiles in and out of the XCD order (2 nt ny a multiple of 16 or not)
-    cases = []
-    for shape in ((48, 64, 64), (48, 64, 64), (48, 54, 72)):
-        w = 1.5 * np.random.default_rng(len(cases)).standard_normal((1,) + shape)
-        cases.append(dict(shape=shape, box=(4.0, 3.5, 3.0), Nblk=(3,), L=(7,), lam=(1.0,), w=w,
-                          chi=np.array([[0, 15, 0], [15, 0, 0], [0, 0, 0]], float)))
-    b = wlc.Batch(cases)
-    for i, c in enumerate(cases):
-        b.set_w(i, c["w"])
-    b.sweep()
-    for i, c in enumerate(cases):
-        g = wlc.WormlikeMDE(c["shape"], c["box"], c["Nblk"], c["L"], c["lam"])
-        g.set_w(c["w"])
-        g.MDE_q()
-        g.MDE_qstar()
-        phi, Q, td = g.density()
-        bphi, bQ, btd = b.density(i)
-        # the twins run the same operations; contraction may differ
-        assert np.abs(bphi - phi).max() < 1e-13 * np.abs(phi).max()
-        assert abs(bQ - Q) / Q < 1e-13 and abs(btd - td) / td < 1e-13
-        g.close()
-    b.close()
+    _batch_matches_handles(wlc, [((48, 64, 64), 7), ((48, 64, 64), 7), ((48, 54, 72), 7)])
+
+
+# nz = 128: a column to each CU (Lmax 5, 6, with the FP32 spectrum to 8) up to 256 columns, the
+# three-part kernel above
+@pytest.mark.parametrize("L,sp,thin", [(5, False, True), (6, False, True), (7, False, False), (8, False, False),
+                                       (5, True, True), (6, True, True), (7, True, True), (8, True, True)])
+def test_nz128_thin(so, L, sp, thin):
+    for (ny, nx), few in (((64, 6), True), ((16, 24), True), ((72, 6), False), ((24, 24), False)):
+        assert (ny * (nx // 2 + 1) <= 256) == few
+        k = [x for x in _launches(so, (128, ny, nx), (4,), (L,), sp) if "z128" in x or "zsolve" in x]
+        one = thin and few
+        assert len(k) == 4 and all(("k_zsolve128s" in x) == one and ("k_z128" in x) != one for x in k), (ny, nx)
+
+
+# beyond 256 columns: a pair with one real column, a padding pair, whole tiles; Lmax changing at a
+# junction; the FP32 spectrum at the bound of the short chains' tests
+@pytest.mark.gpu
+@pytest.mark.parametrize("ny,nx,L,spec32", [(72, 6, (5, 8), False), (54, 8, (6, 7), False), (48, 12, (8, 6), False),
+                                            (54, 8, (7, 8), True), (48, 12, (5, 6), True)])
+def test_nz128_three_parts_match_oracle(wlc, oracle, ny, nx, L, spec32):
+    _matches_oracle(wlc, oracle, (128, ny, nx), (2, 3), L, spec32)
+
+
+@pytest.mark.gpu
+def test_nz128_batched(wlc):
+    _batch_matches_handles(wlc, [((128, 48, 12), 6), ((128, 48, 12), 6), ((128, 4, 12), 6), ((128, 4, 12), 5)])

@@ -57,9 +57,10 @@ bool use_zcol(const Geom& g, const SolveArgs& a) {
   return unsigned((g.nxh + cols - 1) / cols * g.ny) <= zcol_groups(g.nz, a.L);
 }
 
-// nz = 128 with a degree split asked for: the three-part kernel
+// nz = 128 with a degree split asked for: the three-part kernel where there are columns for it
 bool use_z128(const Geom& g, const SolveArgs& a) {
-  return g.nz == 128 && a.L >= kZ128MinL && !a.generic && a.split && a.M == (a.L + 1) * (a.L + 1);
+  return g.nz == 128 && a.L >= kZ128MinL && !a.generic && a.split && !z128_thin(g, a.L) &&
+         a.M == (a.L + 1) * (a.L + 1);
 }
 
 const void* zcol_kernel(const SolveArgs& a, bool batch) {

@@ -15,6 +15,14 @@ constexpr int kZ128Rows = 8 * 72;  // a wave's LDS: eight harmonics
 constexpr int kZ128Col = kZ128Chains * 64 + 2 * kZ128Rows;
 static_assert(kZ128Chains * 64 >= kZ128Rows, "the chains' rows hold the first part's");
 
+// Grids of at most one column per CU, where a kernel that takes one column to a workgroup
+// (k_zsolve128s, two degree parts) is the faster one.  Per launch, that kernel / the three-part one,
+// on 24 x 16 (208 columns): Lmax 5 26.1 / 29.2 us, Lmax 6 31.6 / 35.4, with the FP32 spectrum Lmax 5
+// 21.8 / 26.2, 6 27.2 / 31.6, 7 37.3 / 41.3, 8 42.1 / 52.5; on 24 x 24 (312): 32.6 / 30.6, 41.7 /
+// 37.2, 27.3 / 26.7, 35.5 / 33.2, 48.2 / 42.4, 73.5 / 54.2.  With the FP64 spectrum of Lmax 7 and 8 it
+// has no advantage (24 x 16: whole columns 55.2 and 83.4, three parts 45.4 and 58.8).
+inline bool z128_thin(const Geom& g, int L) { return g.nxh * g.ny <= 256 && (g.spec32 || L <= 6); }
+
 // one workgroup per CU (LDS admits no second one) goes through the column pairs of its XCD's
 // tiles; fewer where there are fewer pairs
 inline unsigned z128_grid(const Geom& g) {

@@ -12,6 +12,7 @@
 #include <type_traits>
 
 #include "wlc_dft.h"
+#include "wlc_z128.h"
 
 #ifndef WLC_L
 #error "compile with -DWLC_L=<Lmax>"
@@ -881,18 +882,21 @@ __global__ void __launch_bounds__(256, 2) k_zsolve48_b(const ZJob* __restrict__ 
 // columns between HBM and LDS with coalesced accesses and forms the radix-2 step from LDS
 // (z128_load_dif, z128_dit_store); with the FP32 spectrum each wave loads its half directly and
 // the halves are exchanged through LDS (z128_exchange).  Lmax 5-8 run the three-part kernel of
-// wlc_z128.hip unless the split is switched off.
+// wlc_z128.hip, or k_zsolve128s on a few columns, unless the split is switched off.
 constexpr int kXB = 16;  // harmonics per cross-wave exchange
 constexpr int kRegion128 = kRegion > kXB * 64 ? kRegion : kXB * 64;
 
 // exchange with the partner wave of the column: own values in, partner's values out,
 // kXB harmonics at a time; every wave of the workgroup takes part in the barriers
-template <int DIR, int NH, int XB = kXB, int N>
+// NLOOP >= NH sets the number of batches, so that waves exchanging different numbers of
+// harmonics in one workgroup still pass the same number of barriers
+template <int DIR, int NH, int NLOOP = NH, int XB = kXB, int N>
 __device__ __forceinline__ void z128_exchange(double2 (&v)[N], double2* own, const double2* other,
                                               int lane, int p, double2 t, bool real_col) {
   static_assert(XB <= kXB, "exchange batch fits a wave region");
+  static_assert(NLOOP >= NH, "every harmonic is exchanged");
 #pragma unroll
-  for (int b0 = 0; b0 < NH; b0 += XB) {
+  for (int b0 = 0; b0 < NLOOP; b0 += XB) {
     __syncthreads();  // the partner has read the previous batch
     if (real_col) {
 #pragma unroll
@@ -1079,6 +1083,130 @@ __global__ void __launch_bounds__(256, OCC) k_zsolve128_b(const ZJob* __restrict
   k_zsolve128_body<OCC, S>(j.g, j.a);
 }
 
+// nz = 128 with the degree split of k_zsolve64s: workgroup = one column, four waves
+// wv = 2 part + p (part 0: l <= kLS, part 1: l > kLS; p: z half).  The radix-2 step pairs
+// wv with wv ^ 1, the crossing tridiagonal chains pair wv with wv ^ 2 through the region of
+// the part-0 wave of the same z half.  For grids of so few columns that each has a CU
+// (z128_thin in wlc_z128.h): the three-part kernel takes two columns to a CU and hands the
+// chains on once more.
+template <int OCC, class S>
+__device__ __forceinline__ void k_zsolve128s_body(const Geom& g, const SolveArgs& a) {
+  __shared__ double2 lds[4 * kRegion128];
+  static_assert(kXch + 2 <= kRegion128, "crossing chains fit a wave region");
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int p = wv & 1, part = wv >> 1;
+  const int ny = g.ny, nxh = g.nxh, nt = g.nt;
+  // block -> column: the four columns of a 4-kx tile run on one XCD (blocks b, b + 8,
+  // b + 16, b + 24), so each tile's cache lines are fetched once
+  const int nb = gridDim.x, b = blockIdx.x;
+  int tl, kxl;
+  if ((nb & 31) == 0) {
+    const int t = b >> 3;
+    kxl = t & 3;
+    tl = (t >> 2) * 8 + (b & 7);
+  } else {
+    kxl = b & 3;
+    tl = b >> 2;
+  }
+  const int t4 = tl % nt, ky = tl / nt;
+  const int kx = t4 * kKxTile + kxl;
+  if (kx >= nxh) return;  // a padding column (uniform over the workgroup)
+  const long long istride = spec_index(1, 0, 0, 0, ny, nt, 128);
+  S* col = reinterpret_cast<S*>(a.spec) + spec_index(0, ky, t4 * kKxTile, 64 * p, ny, nt, 128) + kxl;
+  double2* wl = lds + wv * kRegion128;
+  const double2* partner = lds + (wv ^ 1) * kRegion128;
+  double2* xch = lds + p * kRegion128;  // region of the part-0 wave of this z half
+  // the twiddles are reloaded (cache hits) around each transform instead of being held
+  // through the solve, where the registers are needed for the harmonics
+  const double2* twz = g.az.tw;  // exp(-2 pi i m / 128); exp(-2 pi i j k2 / 64) = twz[2 j k2]
+  const bool active = a.solve;
+  const KFrame f(signed_k(kx, g.nx) * a.kfac[0], signed_k(ky, ny) * a.kfac[1],
+                 signed_k(2 * lane + p, 128) * a.kfac[2], a.sigma, a.ds);
+  double2 v[kNV];
+  {
+    const double2 t = g.az.tw[lane];  // exp(-2 pi i m / 128)
+    if (part == 0) {
+#pragma unroll
+      for (int h = 0; h < PartLo::NH; ++h) v[h] = spec_ld(col + (long long)(PartLo::B0 + h) * istride + 4 * lane);
+      z128_exchange<-1, PartLo::NH, kNV>(v, wl, partner, lane, p, t, true);
+    } else {
+#pragma unroll
+      for (int h = 0; h < PartHi::NH; ++h) v[h] = spec_ld(col + (long long)(PartHi::B0 + h) * istride + 4 * lane);
+      z128_exchange<-1, PartHi::NH, kNV>(v, wl, partner, lane, p, t, true);
+    }
+  }
+  __syncthreads();  // the exchange regions are reused by the transforms and the chains
+  {
+    double2 tw[8];
+#pragma unroll
+    for (int k2 = 0; k2 < 8; ++k2) tw[k2] = twz[2 * (lane & 7) * k2];
+    if (part == 0) {
+      z64_fwd_regs<PartLo::NH>(v, wl, lane, tw);
+    } else {
+      z64_fwd_regs<PartHi::NH>(v, wl, lane, tw);
+    }
+  }
+  // xch is the part-0 wave's own region: its transform is done (program order), and the
+  // part-1 wave reads xch only after the next barrier
+  if (part == 0) {
+    if (active) {
+      PartLo::to_frame(v, f);
+      tri_lower_forward<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
+    }
+  } else {
+    if (active) PartHi::to_frame(v, f);
+  }
+  __syncthreads();
+  if (part == 1 && active) tri_upper<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
+  __syncthreads();
+  if (part == 0) {
+    if (active) {
+      tri_lower_back<kL, kLS>(v, a.cdelta, a.dslam, f.gk, xch, lane);
+      PartLo::from_frame(v, f);
+    }
+  } else {
+    if (active) PartHi::from_frame(v, f);
+  }
+  // after the last barrier only the part-0 wave reads xch (its own region), so the
+  // transforms below need no further barrier
+  double2 tw[8];
+#pragma unroll
+  for (int k2 = 0; k2 < 8; ++k2) tw[k2] = twz[2 * (lane & 7) * k2];
+  const double2 t = g.az.tw[lane];
+  if (part == 0) {
+    z64_inv_regs<PartLo::NH>(v, wl, lane, tw);
+    if (p == 1) {
+#pragma unroll
+      for (int h = 0; h < PartLo::NH; ++h) v[h] = twiddle<+1>(v[h], t);
+    }
+    z128_exchange<+1, PartLo::NH, kNV>(v, wl, partner, lane, p, t, true);
+#pragma unroll
+    for (int h = 0; h < PartLo::NH; ++h) spec_st(col + (long long)(PartLo::B0 + h) * istride + 4 * lane, v[h]);
+  } else {
+    z64_inv_regs<PartHi::NH>(v, wl, lane, tw);
+    if (p == 1) {
+#pragma unroll
+      for (int h = 0; h < PartHi::NH; ++h) v[h] = twiddle<+1>(v[h], t);
+    }
+    z128_exchange<+1, PartHi::NH, kNV>(v, wl, partner, lane, p, t, true);
+#pragma unroll
+    for (int h = 0; h < PartHi::NH; ++h) spec_st(col + (long long)(PartHi::B0 + h) * istride + 4 * lane, v[h]);
+  }
+}
+
+template <int OCC, class S>
+__global__ void __launch_bounds__(256, OCC) k_zsolve128s(Geom g, SolveArgs a) {
+  k_zsolve128s_body<OCC, S>(g, a);
+}
+
+// the same for one instance of a batch per blockIdx.z
+template <int OCC, class S>
+__global__ void __launch_bounds__(256, OCC) k_zsolve128s_b(const ZJob* __restrict__ jobs) {
+  const ZJob& j = jobs[blockIdx.z];
+  if (j.skip && *j.skip) return;
+  k_zsolve128s_body<OCC, S>(j.g, j.a);
+}
+
 // generic kernel B (nz other than 64 and 128, or any nz with the generic kernel forced),
 // 4 <= Lmax <= 7, with the harmonics of each
 // k-point split by degree over two threads: thread t < TX nz holds l <= kLS of k-point
@@ -1232,6 +1360,18 @@ hipError_t zsolve_plan(const Geom& g, const SolveArgs& a, ZPlan* z) {
     z->grid = dim3(2 * g.nt * g.ny);
     z->block = dim3(256);
     return hipSuccess;
+  }
+  if constexpr (kL >= kZ128MinL && (kL <= 6 || std::is_same<S, float2>::value)) {
+    if (g.nz == 128 && !a.generic && a.split && z128_thin(g, kL)) {
+      // one workgroup (one column, harmonics split over two waves per z half) per column; two
+      // waves per SIMD up to Lmax 7, one at Lmax 8 (the 45 harmonics of l = 6..8 need more than
+      // half the register file)
+      z->k1 = (const void*)k_zsolve128s<(kL >= 8 ? 1 : 2), S>;
+      z->kb = (const void*)k_zsolve128s_b<(kL >= 8 ? 1 : 2), S>;
+      z->grid = dim3(4 * g.nt * g.ny);
+      z->block = dim3(256);
+      return hipSuccess;
+    }
   }
   if (g.nz == 128 && !a.generic) {
     // two workgroups (two columns each) per 4-kx tile
