@@ -140,8 +140,6 @@ LaunchKey zsolve_key(const Geom& g, const SolveArgs& a);
 // small elementwise/reduction kernels
 hipError_t launch_set_delta(const Geom& g, double* slice, int M, hipStream_t st);
 hipError_t launch_fill(double* dst, double v, long long n, hipStream_t st);
-// y += a x over n doubles
-hipError_t launch_axpy(double* y, double a, const double* x, long long n, hipStream_t st);
 // rho_t += wgt_t * sum_{i < lim_t} q_i qs_i for up to two targets (t = 0, 1)
 hipError_t launch_density_acc(const Geom& g, const double* q, const double* qs, double* rho0,
                               int lim0, double w0, double* rho1, int lim1, double w1,
@@ -149,9 +147,6 @@ hipError_t launch_density_acc(const Geom& g, const double* q, const double* qs, 
 // partial[b] = sum over a chunk of r of W_r * f(r), f = sum_{t<nf} src[t*N + r]
 hipError_t launch_weighted_sum(const Geom& g, const double* src, int nf, double dV,
                                double* partial, int nparts, double* result, hipStream_t st);
-// phi_b = V * rho_b / totden (totden read from device)
-hipError_t launch_phi(const Geom& g, const double* rho, int nblk, double V, const double* totden,
-                      double* phi, hipStream_t st);
 
 hipError_t upload_orientation_tables(const OrientTables& t);
 
