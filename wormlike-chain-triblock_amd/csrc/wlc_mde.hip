@@ -165,7 +165,7 @@ namespace {
 
 // where forward slice s of the sweep being queued lives
 struct FwdLoc {
-  int mode = 0;  // 0: full store, 1: 4-slot ring, 2: segment buffer starting at slice lo
+  int mode = 0;  // 0: full store, 1: 4-slot ring, 2: segment buffer, lo its first computed slice
   double* base = nullptr;
   int lo = 0;
 };
@@ -202,9 +202,9 @@ double* fwd_slice(const wlc_handle* h, const FwdLoc& fl, int s) {
   }
   if (fl.mode == 2) {
     // segment j >= 1 starts from slices jK - 2, jK - 1, jK
-    if (fl.lo > 0 && s <= fl.lo + 2) {
-      const int j = (fl.lo + 2) / K;
-      return j == h->nstored ? h->store + (long long)s * slot_size(h) : ckpt_slot(h, j, s - fl.lo);
+    if (s < fl.lo) {
+      const int j = (fl.lo - 1) / K;
+      return j == h->nstored ? h->store + (long long)s * slot_size(h) : ckpt_slot(h, j, s - (j * K - 2));
     }
     return fl.base + (long long)(s - fl.lo) * slot_size(h);
   }
@@ -455,7 +455,7 @@ FwdLoc seg_loc(const wlc_handle* h, int j) {
   FwdLoc fl;
   fl.mode = 2;
   fl.base = h->segbuf[j & 1];
-  fl.lo = j == 0 ? 0 : j * h->ck - 2;
+  fl.lo = j == 0 ? 0 : j * h->ck + 1;
   return fl;
 }
 
@@ -970,7 +970,7 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
       // automatic mode: keep as many of the lowest segments whole as fit beside the
       // checkpoint buffers (the last segment is always recomputed); an explicit ckpt_every
       // checkpoints every segment unless WLC_STORED_SEGMENTS asks for a mix (tests)
-      const size_t ck_fixed = base + (size_t)(4 + 1 + 2 * (h->ck + 3)) * slot_bytes + spec_bytes;
+      const size_t ck_fixed = base + (size_t)(4 + 1 + 2 * (h->ck + 1)) * slot_bytes + spec_bytes;
       if (automatic) {
         for (int n = h->nseg - 1; n >= 1; --n) {
           const size_t need = ck_fixed + (size_t)(n * h->ck + 1) * slot_bytes +
@@ -992,7 +992,7 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
       const int nck = h->nseg - (h->nstored > 0 ? h->nstored + 1 : 1);
       if (nck > 0) ALLOC(h->ckpt, (size_t)nck * 3 * slot_bytes);
     }
-    for (int b = 0; b < 2; ++b) ALLOC(h->segbuf[b], (size_t)(h->ck + 3) * slot_bytes);
+    for (int b = 0; b < 2; ++b) ALLOC(h->segbuf[b], (size_t)(h->ck + 1) * slot_bytes);
     ALLOC(h->qlast, slot_bytes);
     ALLOC(h->specr, spec_bytes);
     if (hipStreamCreateWithFlags(&h->str, hipStreamNonBlocking) != hipSuccess) {
