@@ -64,15 +64,14 @@ struct Plane {
 };
 
 // workgroup-uniform base of spectrum plane (i, z) and 32-bit offsets
-template <class S>
 struct SpecPlane {
-  S* p;
+  double2* p;
   unsigned rs, ts;
-  __device__ __forceinline__ SpecPlane(S* spec, const Geom& g, int i, int z)
+  __device__ __forceinline__ SpecPlane(double2* spec, const Geom& g, int i, int z)
       : p(spec + spec_index(i, 0, 0, z, g.ny, g.nt, g.nz)),
         rs(unsigned(g.nt) * unsigned(g.nz) * kKxTile),
         ts(unsigned(g.nz) * kKxTile) {}
-  __device__ __forceinline__ S* at(int ky, int kx) const {
+  __device__ __forceinline__ double2* at(int ky, int kx) const {
     return p + (unsigned(ky) * rs + unsigned(kx >> 2) * ts + unsigned(kx & 3));
   }
 };
@@ -85,11 +84,11 @@ struct Start {
 
 // the spectrum (R, T of the y axis), then columns 0 and h and the twiddles into LDS; the caller's
 // own loads are issued by `more` before anything is waited for, and a barrier follows
-template <int RMAX, class S, class F>
-__device__ __forceinline__ void start(Start<RMAX>& st, const Plane& pl, int R, int T, const S* spec, const Geom& g,
+template <int RMAX, class F>
+__device__ __forceinline__ void start(Start<RMAX>& st, const Plane& pl, int R, int T, const double2* spec, const Geom& g,
                                       int i, int z, bool inv, F&& more) {
   const int tid = threadIdx.x, nthr = blockDim.x;
-  const SpecPlane<S> sp(const_cast<S*>(spec), g, i, z);
+  const SpecPlane sp(const_cast<double2*>(spec), g, i, z);
   if (inv) {
     const int jy = tid / pl.s.h, c = tid - jy * pl.s.h;
     if (jy < T && c) {
@@ -280,8 +279,8 @@ __device__ __forceinline__ int x_slot(int k) {
 // Unpack of the row pairs (A_k = (Z_k + conj Z_{n-k}) / 2 the even row slot, B_k = (Z_k -
 // conj Z_{n-k}) / 2i the odd one), forward y transform, store of the spectrum plane; pk and pn are
 // the slots of Z_c and Z_{n-c} (c = 0: of Z_0 and Z_h, the real values of the packed column).
-template <int NY, class S>
-__device__ __forceinline__ void y_forward(const Plane& pl, int pk, int pn, S* spec, const Geom& g, int i, int z) {
+template <int NY>
+__device__ __forceinline__ void y_forward(const Plane& pl, int pk, int pn, double2* spec, const Geom& g, int i, int z) {
   constexpr int R = two_pass(NY).R, T = two_pass(NY).T, Q = (R + T - 1) / T;
   static_assert(T % 2 == 0, "a thread unpacks whole row pairs");
   const int jy = threadIdx.x / pl.s.h, c = threadIdx.x - jy * pl.s.h;
@@ -315,7 +314,7 @@ __device__ __forceinline__ void y_forward(const Plane& pl, int pk, int pn, S* sp
     }
   }
   __syncthreads();
-  const SpecPlane<S> sp(spec, g, i, z);
+  const SpecPlane sp(spec, g, i, z);
   if (jy < T) {
     double2 v[R];
 #pragma unroll
@@ -357,8 +356,8 @@ __device__ __forceinline__ void x_inverse_any(const Plane& pl) {
 #undef X
   }
 }
-template <int NX, int NY, class S>
-__device__ __forceinline__ void forward_any(const Plane& pl, S* spec, const Geom& g, int i, int z) {
+template <int NX, int NY>
+__device__ __forceinline__ void forward_any(const Plane& pl, double2* spec, const Geom& g, int i, int z) {
   const int c = threadIdx.x % pl.s.h, cn = c ? pl.nx - c : pl.s.h;
   int pk = 0, pn = 0;
   if constexpr (NX > 0) {
@@ -483,7 +482,7 @@ struct YPlan {
 };
 
 // A: right-hand side from the history slices, forward x and y passes
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __device__ __forceinline__ void k_rhs_body(const Geom& g, const RhsArgs& a) {
   extern __shared__ double2 lds[];
   int z, i;
@@ -494,7 +493,7 @@ __device__ __forceinline__ void k_rhs_body(const Geom& g, const RhsArgs& a) {
   Start<YPlan<NY>::RMAX> st;
   Items<NX, NY> it;
   Hist<Items<NX, NY>::N> hv;
-  start(st, pl, py.R, py.T, reinterpret_cast<const S*>(a.spec), g, i, z, false, [&] {
+  start(st, pl, py.R, py.T, a.spec, g, i, z, false, [&] {
     it.set(pl);
     load_hist<NX, NY>(hv, it, g, a, i, plane);
   });
@@ -503,11 +502,11 @@ __device__ __forceinline__ void k_rhs_body(const Geom& g, const RhsArgs& a) {
   for (int m = 0; m < Items<NX, NY>::N; ++m)
     if (it.at[m] >= 0) put_rhs(lds, it.at[m], m, ld2(h0 + it.o0[m]), ld2(h0 + it.o1[m]), hv, a);
   wave_lds_sync();
-  forward_any<NX, NY>(pl, reinterpret_cast<S*>(a.spec), g, i, z);
+  forward_any<NX, NY>(pl, a.spec, g, i, z);
 }
 
 // C: inverse y and x passes, 1/N, store of q(s)
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __device__ __forceinline__ void k_inv_body(const Geom& g, const InvArgs& c) {
   extern __shared__ double2 lds[];
   int z, i;
@@ -516,7 +515,7 @@ __device__ __forceinline__ void k_inv_body(const Geom& g, const InvArgs& c) {
   const TwoPass py = two_pass(pl.ny);
   Start<YPlan<NY>::RMAX> st;
   Items<NX, NY> it;
-  start(st, pl, py.R, py.T, reinterpret_cast<const S*>(c.spec), g, i, z, true, [&] { it.set(pl); });
+  start(st, pl, py.R, py.T, c.spec, g, i, z, true, [&] { it.set(pl); });
   y_inverse_any<NY>(pl, st);
   x_inverse_any<NX>(pl);
   double* out = c.out + i * g.hs + (long long)z * g.zs;
@@ -532,7 +531,7 @@ __device__ __forceinline__ void k_inv_body(const Geom& g, const InvArgs& c) {
 // C of step s fused with A of the next: harmonic i < M(s) is inverted and stored and stays in LDS
 // as the newest history plane (zero beyond: a junction that grows the basis); for i < M(next) the
 // right-hand side is formed in place and transformed into the same spectrum plane.
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __device__ __forceinline__ void k_inv_rhs_body(const Geom& g, const InvArgs& c, const RhsArgs& a) {
   extern __shared__ double2 lds[];
   int z, i;
@@ -544,7 +543,7 @@ __device__ __forceinline__ void k_inv_rhs_body(const Geom& g, const InvArgs& c, 
   Start<YPlan<NY>::RMAX> st;
   Items<NX, NY> it;
   Hist<Items<NX, NY>::N> hv;
-  start(st, pl, py.R, py.T, reinterpret_cast<const S*>(c.spec), g, i, z, inv, [&] {
+  start(st, pl, py.R, py.T, c.spec, g, i, z, inv, [&] {
     it.set(pl);
     if (rhs) load_hist<NX, NY>(hv, it, g, a, i, plane);
   });
@@ -568,64 +567,59 @@ __device__ __forceinline__ void k_inv_rhs_body(const Geom& g, const InvArgs& c, 
     }
   if (!rhs) return;
   wave_lds_sync();
-  forward_any<NX, NY>(pl, reinterpret_cast<S*>(a.spec), g, i, z);
+  forward_any<NX, NY>(pl, a.spec, g, i, z);
 }
 
 // run-time edges: two waves per SIMD (220 registers); held to three they spill (36 x 54, Lmax 4
 // 41 -> 57 us)
 #define WLC_BOUNDS(NX, NY) __launch_bounds__(NX > 0 ? 64 * shape_of(NX > 0 ? NX : 8, NY > 0 ? NY : 8).waves : kMaxThreads, NX > 0 ? 1 : 2)
 
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __global__ void WLC_BOUNDS(NX, NY) k2_rhs(Geom g, RhsArgs a) {
-  k_rhs_body<NX, NY, S>(g, a);
+  k_rhs_body<NX, NY>(g, a);
 }
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __global__ void WLC_BOUNDS(NX, NY) k2_inv(Geom g, InvArgs c) {
-  k_inv_body<NX, NY, S>(g, c);
+  k_inv_body<NX, NY>(g, c);
 }
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __global__ void WLC_BOUNDS(NX, NY) k2_inv_rhs(Geom g, InvArgs c, RhsArgs a) {
-  k_inv_rhs_body<NX, NY, S>(g, c, a);
+  k_inv_rhs_body<NX, NY>(g, c, a);
 }
 
 // the same for one instance of a batch per blockIdx.z
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __global__ void WLC_BOUNDS(NX, NY) k2_rhs_b(const PlaneJob* __restrict__ jobs) {
   const PlaneJob& j = jobs[blockIdx.z];
   if (j.skip && *j.skip) return;
-  k_rhs_body<NX, NY, S>(j.g, j.a);
+  k_rhs_body<NX, NY>(j.g, j.a);
 }
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __global__ void WLC_BOUNDS(NX, NY) k2_inv_b(const PlaneJob* __restrict__ jobs) {
   const PlaneJob& j = jobs[blockIdx.z];
   if (j.skip && *j.skip) return;
-  k_inv_body<NX, NY, S>(j.g, j.c);
+  k_inv_body<NX, NY>(j.g, j.c);
 }
-template <int NX, int NY, class S>
+template <int NX, int NY>
 __global__ void WLC_BOUNDS(NX, NY) k2_inv_rhs_b(const PlaneJob* __restrict__ jobs) {
   const PlaneJob& j = jobs[blockIdx.z];
   if (j.skip && *j.skip) return;
-  k_inv_rhs_body<NX, NY, S>(j.g, j.c, j.a);
+  k_inv_rhs_body<NX, NY>(j.g, j.c, j.a);
 }
 
-template <int NX, int NY, class S>
+template <int NX, int NY>
 const void* pick(int kind, bool batch) {
-  if (kind == 0) return batch ? (const void*)k2_rhs_b<NX, NY, S> : (const void*)k2_rhs<NX, NY, S>;
-  if (kind == 1) return batch ? (const void*)k2_inv_b<NX, NY, S> : (const void*)k2_inv<NX, NY, S>;
-  return batch ? (const void*)k2_inv_rhs_b<NX, NY, S> : (const void*)k2_inv_rhs<NX, NY, S>;
-}
-
-template <class S>
-const void* pick_edges(int nx, int ny, int kind, bool batch) {
-  // 48 x 48 (the batching workload) with compile-time edges, any other pair without
-  if (nx == 48 && ny == 48) return pick<48, 48, S>(kind, batch);
-  return pick<0, 0, S>(kind, batch);
+  if (kind == 0) return batch ? (const void*)k2_rhs_b<NX, NY> : (const void*)k2_rhs<NX, NY>;
+  if (kind == 1) return batch ? (const void*)k2_inv_b<NX, NY> : (const void*)k2_inv<NX, NY>;
+  return batch ? (const void*)k2_inv_rhs_b<NX, NY> : (const void*)k2_inv_rhs<NX, NY>;
 }
 
 }  // namespace
 
 const void* kernel(int nx, int ny, int kind, bool batch) {
-  return pick_edges<double2>(nx, ny, kind, batch);
+  // 48 x 48 (the batching workload) with compile-time edges, any other pair without
+  if (nx == 48 && ny == 48) return pick<48, 48>(kind, batch);
+  return pick<0, 0>(kind, batch);
 }
 
 }  // namespace p2

@@ -131,9 +131,8 @@ __device__ __forceinline__ void chains_part(double2* at, int np, double cdelta, 
 // slots of 1 << lc columns: element m of row k at slot_of(k, m).  The rows are a power of two
 // of 16-byte units apart when T is, so the lanes of a pass over the rows would meet on one
 // bank group; the order within a row is turned by the row (48^3 / Lmax 6 47.0 -> 40.6 us).
-template <class S>
 struct Cols {
-  S* p;
+  double2* p;
   unsigned istride;
   int lc, nc, np;
 };
@@ -154,8 +153,8 @@ __device__ __forceinline__ int slot_of(int k, int m, int lc) {
 }
 
 // forward pass 1: DFT-R over z = j + T r, twiddle, from HBM into LDS
-template <int R, int T, class S>
-__device__ __forceinline__ void pass_in(double2* lds, const Cols<S>& w, const double2* __restrict__ tw) {
+template <int R, int T>
+__device__ __forceinline__ void pass_in(double2* lds, const Cols& w, const double2* __restrict__ tw) {
   constexpr int U = R <= 4 ? 4 : 2;  // butterflies in flight per thread
   const int total = (kM * T) << w.lc, nthr = blockDim.x;
   for (int base = threadIdx.x; base < total; base += U * nthr) {
@@ -166,7 +165,7 @@ __device__ __forceinline__ void pass_in(double2* lds, const Cols<S>& w, const do
       const int c = idx & ((1 << w.lc) - 1), r = idx >> w.lc;
       const int i = r / T, j = r - i * T;
       const bool ok = idx < total && c < w.nc;
-      const S* src = w.p + (unsigned(i) * w.istride + unsigned(kKxTile * j + c));
+      const double2* src = w.p + (unsigned(i) * w.istride + unsigned(kKxTile * j + c));
 #pragma unroll
       for (int k = 0; k < R; ++k) u[q][k] = ok ? spec_ld(src + kKxTile * T * k) : make_double2(0.0, 0.0);
     }
@@ -188,8 +187,8 @@ __device__ __forceinline__ void pass_in(double2* lds, const Cols<S>& w, const do
 
 // forward pass 2 (DIR = -1: DFT-T over row k1) and inverse pass 1 (DIR = +1: the same, then the
 // twiddle), in place in LDS
-template <int R, int T, int DIR, class S>
-__device__ __forceinline__ void pass_mid(double2* lds, const Cols<S>& w, const double2* __restrict__ tw) {
+template <int R, int T, int DIR>
+__device__ __forceinline__ void pass_mid(double2* lds, const Cols& w, const double2* __restrict__ tw) {
   constexpr int U = 2;
   const int total = (kM * R) << w.lc, nthr = blockDim.x;
   for (int base = threadIdx.x; base < total; base += U * nthr) {
@@ -223,8 +222,8 @@ __device__ __forceinline__ void pass_mid(double2* lds, const Cols<S>& w, const d
 }
 
 // inverse pass 2: DFT-R over the rows, from LDS to HBM
-template <int R, int T, class S>
-__device__ __forceinline__ void pass_out(const double2* lds, const Cols<S>& w) {
+template <int R, int T>
+__device__ __forceinline__ void pass_out(const double2* lds, const Cols& w) {
   constexpr int U = 2;
   const int total = (kM * T) << w.lc, nthr = blockDim.x;
   for (int base = threadIdx.x; base < total; base += U * nthr) {
@@ -246,7 +245,7 @@ __device__ __forceinline__ void pass_out(const double2* lds, const Cols<S>& w) {
       const int i = r / T, j = r - i * T;
       if (idx < total && c < w.nc) {
         Dft<R, +1>::run(u[q]);
-        S* dst = w.p + (unsigned(i) * w.istride + unsigned(kKxTile * j + c));
+        double2* dst = w.p + (unsigned(i) * w.istride + unsigned(kKxTile * j + c));
 #pragma unroll
         for (int k = 0; k < R; ++k) spec_st(dst + kKxTile * T * k, u[q][k]);
       }
@@ -258,15 +257,15 @@ __device__ __forceinline__ int turn_of(int T, int k, int lc) {
   return T == 2 ? turn<2>(k, lc) : T == 4 ? turn<4>(k, lc) : T == 8 ? turn<8>(k, lc) : 0;
 }
 
-template <int NZ, class S>
-__device__ __forceinline__ void transform_in(double2* lds, const Cols<S>& w, const double2* __restrict__ tw) {
+template <int NZ>
+__device__ __forceinline__ void transform_in(double2* lds, const Cols& w, const double2* __restrict__ tw) {
   constexpr int R = two_pass(NZ).R, T = two_pass(NZ).T;
   pass_in<R, T>(lds, w, tw);
   __syncthreads();
   pass_mid<R, T, -1>(lds, w, tw);
 }
-template <int NZ, class S>
-__device__ __forceinline__ void transform_out(double2* lds, const Cols<S>& w, const double2* __restrict__ tw) {
+template <int NZ>
+__device__ __forceinline__ void transform_out(double2* lds, const Cols& w, const double2* __restrict__ tw) {
   constexpr int R = two_pass(NZ).R, T = two_pass(NZ).T;
   pass_mid<R, T, +1>(lds, w, tw);
   __syncthreads();
@@ -275,7 +274,6 @@ __device__ __forceinline__ void transform_out(double2* lds, const Cols<S>& w, co
 
 #define WLC_EACH_NZ(X) X(8) X(12) X(16) X(18) X(24) X(32) X(36) X(48) X(54)
 
-template <class S>
 __device__ __forceinline__ void k_zcol_body(const Geom& g, const SolveArgs& a) {
   extern __shared__ double2 lds[];
   const int nz = g.nz, ny = g.ny, nt = g.nt;
@@ -287,13 +285,13 @@ __device__ __forceinline__ void k_zcol_body(const Geom& g, const SolveArgs& a) {
   if (tl >= nt * ny) return;  // (uniform)
   const int t4 = tl % nt, ky = tl / nt;
   const int kx0 = t4 * kKxTile + (grp << lc);
-  Cols<S> w;
+  Cols w;
   w.lc = lc;
   w.nc = min(1 << lc, g.nxh - kx0);
   if (w.nc <= 0) return;  // padding columns only (uniform)
   w.np = nz << lc;
   w.istride = (unsigned)spec_index(1, 0, 0, 0, ny, nt, nz);
-  w.p = reinterpret_cast<S*>(a.spec) + spec_index(0, ky, kx0, 0, ny, nt, nz);
+  w.p = a.spec + spec_index(0, ky, kx0, 0, ny, nt, nz);
   const double2* tw = g.az.tw;
   int R = 1, T = 1;
   switch (nz) {
@@ -346,17 +344,15 @@ __device__ __forceinline__ void k_zcol_body(const Geom& g, const SolveArgs& a) {
   }
 }
 
-template <class S>
 __global__ void __launch_bounds__(512, kWaves) k_zcol(Geom g, SolveArgs a) {
-  k_zcol_body<S>(g, a);
+  k_zcol_body(g, a);
 }
 
 // the same for one instance of a batch per blockIdx.z
-template <class S>
 __global__ void __launch_bounds__(512, kWaves) k_zcol_b(const ZJob* __restrict__ jobs) {
   const ZJob& j = jobs[blockIdx.z];
   if (j.skip && *j.skip) return;
-  k_zcol_body<S>(j.g, j.a);
+  k_zcol_body(j.g, j.a);
 }
 
 }  // namespace zcol_l_<L>
@@ -364,7 +360,7 @@ __global__ void __launch_bounds__(512, kWaves) k_zcol_b(const ZJob* __restrict__
 using namespace WLC_CAT(zcol_l_, WLC_L);
 
 const void* WLC_CAT(zcol_kernel_L, WLC_L)(bool batch) {
-  return batch ? (const void*)k_zcol_b<double2> : (const void*)k_zcol<double2>;
+  return batch ? (const void*)k_zcol_b : (const void*)k_zcol;
 }
 
 }  // namespace wlc
