@@ -140,15 +140,16 @@ def test_nz48_lmax7_batched(wlc):
     _batch_matches_handles(wlc, [((48, 64, 64), 7), ((48, 64, 64), 7), ((48, 54, 72), 7)])
 
 
-# nz = 128: a column to each CU (Lmax 5, 6, with the FP32 spectrum to 8) up to 256 columns, the
-# three-part kernel above
-@pytest.mark.parametrize("L,sp,thin", [(5, False, True), (6, False, True), (7, False, False), (8, False, False),
-                                       (5, True, True), (6, True, True), (7, True, True), (8, True, True)])
-def test_nz128_thin(so, L, sp, thin):
+# nz = 128: a column to each CU (Lmax 5, 6, with the FP32 spectrum to 8) up to 256 columns, with the
+# FP32 spectrum at Lmax 5 and 6 beyond them too; the three-part kernel for the rest
+@pytest.mark.parametrize("L,sp,few_cols,many_cols", [
+    (5, False, True, False), (6, False, True, False), (7, False, False, False), (8, False, False, False),
+    (5, True, True, True), (6, True, True, True), (7, True, True, False), (8, True, True, False)])
+def test_nz128_two_parts(so, L, sp, few_cols, many_cols):
     for (ny, nx), few in (((64, 6), True), ((16, 24), True), ((72, 6), False), ((24, 24), False)):
         assert (ny * (nx // 2 + 1) <= 256) == few
         k = [x for x in _launches(so, (128, ny, nx), (4,), (L,), sp) if "z128" in x or "zsolve" in x]
-        one = thin and few
+        one = few_cols if few else many_cols
         assert len(k) == 4 and all(("k_zsolve128s" in x) == one and ("k_z128" in x) != one for x in k), (ny, nx)
 
 
@@ -156,9 +157,16 @@ def test_nz128_thin(so, L, sp, thin):
 # junction; the FP32 spectrum at the bound of the short chains' tests
 @pytest.mark.gpu
 @pytest.mark.parametrize("ny,nx,L,spec32", [(72, 6, (5, 8), False), (54, 8, (6, 7), False), (48, 12, (8, 6), False),
-                                            (54, 8, (7, 8), True), (48, 12, (5, 6), True)])
+                                            (54, 8, (7, 8), True), (48, 12, (7, 7), True)])
 def test_nz128_three_parts_match_oracle(wlc, oracle, ny, nx, L, spec32):
     _matches_oracle(wlc, oracle, (128, ny, nx), (2, 3), L, spec32)
+
+
+@pytest.mark.gpu
+def test_nz128_two_parts_match_oracle(wlc, oracle):
+    # more columns than CUs, rows of four-column tiles in the XCD order and not
+    _matches_oracle(wlc, oracle, (128, 48, 12), (2, 3), (5, 6), spec32=True)
+    _matches_oracle(wlc, oracle, (128, 54, 8), (2, 3), (6, 5), spec32=True)
 
 
 @pytest.mark.gpu

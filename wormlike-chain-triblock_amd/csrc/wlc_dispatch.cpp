@@ -59,7 +59,7 @@ bool use_zcol(const Geom& g, const SolveArgs& a) {
 
 // nz = 128 with a degree split asked for: the three-part kernel where there are columns for it
 bool use_z128(const Geom& g, const SolveArgs& a) {
-  return g.nz == 128 && a.L >= kZ128MinL && !a.generic && a.split && !z128_thin(g, a.L) &&
+  return g.nz == 128 && a.L >= kZ128MinL && !a.generic && a.split && !z128_two_parts(g, a.L) &&
          a.M == (a.L + 1) * (a.L + 1);
 }
 

@@ -73,7 +73,7 @@ struct SolveArgs {
                        // per workgroup, loaded directly, 2 a whole 4-kx tile per workgroup, 3
                        // half a tile, both through LDS (2 and 3: FP64 spectrum; FP32 runs as 1).
                        // nz = 128, Lmax 5-8: 0 whole columns per wave pair, else the three-part
-                       // kernel (on a few columns k_zsolve128s, see wlc_z128.h).  Other nz,
+                       // kernel or k_zsolve128s (see wlc_z128.h).  Other nz,
                        // Lmax 4-7: any nonzero value splits by degree
 };
 

@@ -455,8 +455,14 @@ __global__ void __launch_bounds__(kZ128Threads, 3) k_z128_b(const ZJob* __restri
 using namespace WLC_CAT(z128_l_, WLC_L);
 
 const void* WLC_CAT(z128_kernel_L, WLC_L)(bool spec32, bool batch) {
-  if (batch) return spec32 ? (const void*)k_z128_b<float2> : (const void*)k_z128_b<double2>;
-  return spec32 ? (const void*)k_z128<float2> : (const void*)k_z128<double2>;
+  if (spec32) {
+#if WLC_L >= 7
+    return batch ? (const void*)k_z128_b<float2> : (const void*)k_z128<float2>;
+#else
+    return nullptr;  // runs in two parts (z128_two_parts)
+#endif
+  }
+  return batch ? (const void*)k_z128_b<double2> : (const void*)k_z128<double2>;
 }
 
 }  // namespace wlc

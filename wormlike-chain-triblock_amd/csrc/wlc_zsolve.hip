@@ -882,7 +882,7 @@ __global__ void __launch_bounds__(256, 2) k_zsolve48_b(const ZJob* __restrict__ 
 // columns between HBM and LDS with coalesced accesses and forms the radix-2 step from LDS
 // (z128_load_dif, z128_dit_store); with the FP32 spectrum each wave loads its half directly and
 // the halves are exchanged through LDS (z128_exchange).  Lmax 5-8 run the three-part kernel of
-// wlc_z128.hip, or k_zsolve128s on a few columns, unless the split is switched off.
+// wlc_z128.hip or k_zsolve128s unless the split is switched off.
 constexpr int kXB = 16;  // harmonics per cross-wave exchange
 constexpr int kRegion128 = kRegion > kXB * 64 ? kRegion : kXB * 64;
 
@@ -1086,9 +1086,8 @@ __global__ void __launch_bounds__(256, OCC) k_zsolve128_b(const ZJob* __restrict
 // nz = 128 with the degree split of k_zsolve64s: workgroup = one column, four waves
 // wv = 2 part + p (part 0: l <= kLS, part 1: l > kLS; p: z half).  The radix-2 step pairs
 // wv with wv ^ 1, the crossing tridiagonal chains pair wv with wv ^ 2 through the region of
-// the part-0 wave of the same z half.  For grids of so few columns that each has a CU
-// (z128_thin in wlc_z128.h): the three-part kernel takes two columns to a CU and hands the
-// chains on once more.
+// the part-0 wave of the same z half.  Where it is the faster one (z128_two_parts
+// in wlc_z128.h): the three-part kernel takes two columns to a CU and hands the chains on once more.
 template <int OCC, class S>
 __device__ __forceinline__ void k_zsolve128s_body(const Geom& g, const SolveArgs& a) {
   __shared__ double2 lds[4 * kRegion128];
@@ -1362,7 +1361,7 @@ hipError_t zsolve_plan(const Geom& g, const SolveArgs& a, ZPlan* z) {
     return hipSuccess;
   }
   if constexpr (kL >= kZ128MinL && (kL <= 6 || std::is_same<S, float2>::value)) {
-    if (g.nz == 128 && !a.generic && a.split && z128_thin(g, kL)) {
+    if (g.nz == 128 && !a.generic && a.split && z128_two_parts(g, kL)) {
       // one workgroup (one column, harmonics split over two waves per z half) per column; two
       // waves per SIMD up to Lmax 7, one at Lmax 8 (the 45 harmonics of l = 6..8 need more than
       // half the register file)
