@@ -82,6 +82,23 @@ def test_planes_of_five_waves(so):
         assert sum("k2_" in x for x in k) == 5, (ny, nx)
 
 
+# 72 x 12, 16 and 24 planes: C + A by the run-time kernels above 1280 planes, A and C alone not
+def test_thin_planes(so):
+    for ny, nx, thin in ((72, 12, True), (12, 72, True), (72, 16, True), (16, 72, True), (72, 24, True),
+                         (24, 72, True), (72, 18, False), (18, 72, False), (72, 32, False), (54, 12, False)):
+        for nz, L in ((48, 4), (54, 4)):
+            k = [x for x in _launches(so, (nz, ny, nx), (4,), (L,)) if "k2_" in x or "rhs" in x or "ifft" in x]
+            assert "k2_rhs" in k[0] and "k2_inv" in k[-1] and len(k) == 5
+            assert all(("k2_inv_rhs" in x) != (thin and nz == 54) for x in k[1:-1]), (ny, nx, nz)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ny,nx", [(72, 12), (12, 72), (72, 16), (24, 72)])
+def test_thin_planes_match_oracle(wlc, oracle, ny, nx):
+    # 1350 planes, then 486, across the junction
+    _matches_oracle(wlc, oracle, (54, ny, nx), (3, 3), (4, 2))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("ny,nx", [(48, 72), (72, 48)])
 def test_planes_of_five_waves_match_oracle(wlc, oracle, ny, nx):

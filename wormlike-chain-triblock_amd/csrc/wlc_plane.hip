@@ -396,8 +396,16 @@ static bool specialised(const Geom& g) {
 // FP64 spectrum only: with the FP32 one another order of the same operations rounds some stored
 // values the other way, which after 40 to 100 steps moves phi by 1e-9 to 1e-7 of itself, as far as
 // the storage type itself does, so that mode keeps the kernels and with them its results
-static bool two_pass_plane(const Geom& g, int planes) {
+static bool two_pass_plane(const Geom& g, int kind, int planes) {
   if (g.spec32 || specialised(g) || !p2::takes(g.nx, g.ny)) return false;
+  // 72 x 12, x 16 and x 24, either way round, C + A: three waves a plane, two planes per CU, and not
+  // enough rows or columns for the lanes of all three; beside the other sweep's kernels the four waves
+  // of the run-time kernel do better once there are many planes.  Pair of sweeps of 40 steps, run-time /
+  // two-pass: 72 x 12 with 600 planes 1.83 / 1.89 ms, 1176 2.73 / 2.95, 3136 5.50 / 6.11; 12 x 72, 3136
+  // 5.29 / 5.78; 72 x 16, 600 2.02 / 1.97, 1200 2.99 / 3.01, 2352 5.47 / 5.84; 24 x 72, 600 2.35 / 2.27,
+  // 2352 6.63 / 7.06.  A and C alone stay (a step on 72 x 12 x 64, Lmax 7, 108 / 99 us).
+  const int lo = std::min(g.nx, g.ny), hi = std::max(g.nx, g.ny);
+  if (kind == 2 && hi == 72 && (lo == 12 || lo == 16 || lo == 24) && planes > 1280) return false;
   // 48 x 72 and 72 x 48: a two-pass plane is five waves, and a CU holds one at a time (two waves per
   // SIMD), while the run-time kernel keeps these planes in eight slots a thread.  From about two
   // planes per CU on that one is faster: C + A of 72 x 48 with 400 planes 37.3 us against 31.2 us of
@@ -466,7 +474,7 @@ static void* pick_plane_kernel_t(const Geom& g, int kind, int order, int planes,
     }
     return nullptr;
   }
-  if (two_pass_plane(g, planes)) {
+  if (two_pass_plane(g, kind, planes)) {
     *lds = p2::lds_bytes(g.nx, g.ny);
     *threads = 64 * p2::shape_of(g.nx, g.ny).waves;
     return const_cast<void*>(p2::kernel(g.nx, g.ny, kind, B));
