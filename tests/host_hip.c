@@ -149,7 +149,8 @@ int hipDeviceSynchronize(void) { return kOk; }
 int hipGetLastError(void) { return kOk; }
 const char* hipGetErrorString(int e) { return e == kNoMemory ? "out of memory" : e ? "invalid argument" : "no error"; }
 static void* handle(void) { return malloc(8); }
-int hipStreamCreateWithFlags(void** s, unsigned f) { return (void)f, *s = handle(), kOk; }
+static int g_streams;
+int hipStreamCreateWithFlags(void** s, unsigned f) { return (void)f, ++g_streams, *s = handle(), kOk; }
 int hipStreamDestroy(void* s) { return free(s), kOk; }
 int hipStreamSynchronize(void* s) { return (void)s, kOk; }
 int hipStreamWaitEvent(void* s, void* e, unsigned f) { return (void)s, (void)e, (void)f, kOk; }
@@ -171,6 +172,7 @@ int hipGraphExecDestroy(void* x) { return free(x), kOk; }
 /* --- what the tests ask -------------------------------------------------------------------- */
 void host_hip_fail(int nth) { g_fail = nth; }  /* the nth hipMalloc from now fails (0: none) */
 int host_hip_bad(void) { return g_bad; }       /* copies, fills and frees outside live memory */
+int host_hip_streams(void) { return g_streams; }  /* created so far */
 int host_hip_allocs(void) { return g_allocs; }
 long long host_hip_alloc_bytes(int i) { return (long long)g_alloc[i].n; }
 int host_hip_alloc_live(int i) { return g_alloc[i].live; }

@@ -936,21 +936,6 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
       return fail(WLC_ENOMEM, std::string("device allocation failed: ") + #ptr); \
     }                                                                            \
   } while (0)
-  // the two sweeps' streams one after the other: the runtime gives a new stream the hardware
-  // queue with the fewest users, so the two land on different ones and can overlap (24^3 /
-  // Lmax 6: 3.8 ms a pair of sweeps, 5.7 ms when they share one)
-  if (hipStreamCreateWithFlags(&h->st, hipStreamNonBlocking) != hipSuccess ||
-      hipStreamCreateWithFlags(&h->stb, hipStreamNonBlocking) != hipSuccess ||
-      hipStreamCreateWithFlags(&h->st2, hipStreamNonBlocking) != hipSuccess) {
-    free_handle(h);
-    return fail(WLC_EHIP, "stream creation failed");
-  }
-  bool ev_ok = hipEventCreateWithFlags(&h->ev_step, hipEventDisableTiming) == hipSuccess;
-  for (auto& e : h->ev_dens) ev_ok = ev_ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-  if (!ev_ok) {
-    free_handle(h);
-    return fail(WLC_EHIP, "event creation failed");
-  }
   const size_t store_bytes = sizeof(double) * (size_t)h->off[h->Ns + 1];
   // sized for FP64 elements in either mode, so that wlc_mde_set_spectrum_fp32 can switch
   const size_t spec_bytes = sizeof(double2) * (size_t)h->Mmax * p->ny * wlc::kx_tiles(h->nxh) * wlc::kKxTile * p->nz;
@@ -985,6 +970,24 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
       }
     }
   }
+  // the streams that run at the same time one after the other, and no more than the handle needs:
+  // the runtime gives a new stream the hardware queue with the fewest users, of which a process has
+  // four, so these land on different ones and can overlap (24^3 / Lmax 6: 3.8 ms a pair of sweeps,
+  // 5.7 ms when the sweeps share one; with one more stream before its own the recomputation
+  // shared one: 24^3 / Lmax 4, Ns 60, checkpointed, 2.9 -> 3.9 ms)
+  hipStream_t* const second = h->ck ? &h->str : &h->stb;
+  if (hipStreamCreateWithFlags(&h->st, hipStreamNonBlocking) != hipSuccess ||
+      hipStreamCreateWithFlags(second, hipStreamNonBlocking) != hipSuccess ||
+      hipStreamCreateWithFlags(&h->st2, hipStreamNonBlocking) != hipSuccess) {
+    free_handle(h);
+    return fail(WLC_EHIP, "stream creation failed");
+  }
+  bool ev_ok = hipEventCreateWithFlags(&h->ev_step, hipEventDisableTiming) == hipSuccess;
+  for (auto& e : h->ev_dens) ev_ok = ev_ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  if (!ev_ok) {
+    free_handle(h);
+    return fail(WLC_EHIP, "event creation failed");
+  }
   if (h->ck) {
     ALLOC(h->fr, 4 * slot_bytes);
     if (h->nstored > 0) ALLOC(h->store, (size_t)(h->nstored * h->ck + 1) * slot_bytes);
@@ -995,10 +998,6 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
     for (int b = 0; b < 2; ++b) ALLOC(h->segbuf[b], (size_t)(h->ck + 1) * slot_bytes);
     ALLOC(h->qlast, slot_bytes);
     ALLOC(h->specr, spec_bytes);
-    if (hipStreamCreateWithFlags(&h->str, hipStreamNonBlocking) != hipSuccess) {
-      free_handle(h);
-      return fail(WLC_EHIP, "stream creation failed");
-    }
     bool ok = true;
     for (auto& e : h->ev_seg_ready) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     for (auto& e : h->ev_seg_free) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
@@ -1024,7 +1023,7 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
               free_b > extra + spec_bytes + (size_t(2) << 30);
     if (!h->conc) h->parts = 1;
   }
-  if (!h->conc) {
+  if (!h->conc && h->stb) {
     (void)hipStreamDestroy(h->stb);
     h->stb = nullptr;
   }
