@@ -77,9 +77,26 @@ def test_planes_of_five_waves(so):
     k = [x for x in _launches(so, (36, 48, 72), (3, 3), (2, 3)) if "k2_" in x or "rhs" in x or "ifft" in x]
     assert [("k2_" in x) for x in k] == [True, True, True, False, False, False, False]
     # other planes keep the two-pass kernels at any number
-    for ny, nx in ((54, 72), (64, 72), (72, 72), (36, 72)):
-        k = _launches(so, (72, ny, nx), (4,), (4,))
-        assert sum("k2_" in x for x in k) == 5, (ny, nx)
+    for nz, ny, nx in ((72, 54, 72), (64, 64, 72), (64, 72, 72), (72, 36, 72)):
+        k = _launches(so, (nz, ny, nx), (4,), (4,))
+        assert sum("k2_" in x for x in k) == 5, (nz, ny, nx)
+
+
+# 72 x 64, 64 x 72 and 72 x 72 planes on a z axis longer than 64: C + A by the run-time kernels between
+# 600 and 3300 planes
+def test_planes_of_more_waves(so):
+    for ny, nx in ((72, 64), (64, 72), (72, 72)):
+        for nz, L, two in ((72, 1, True), (72, 2, False), (64, 3, True), (96, 3, False), (72, 5, False), (72, 6, True)):
+            k = [x for x in _launches(so, (nz, ny, nx), (4,), (L,)) if "k2_" in x or "rhs" in x or "ifft" in x]
+            assert "k2_rhs" in k[0] and "k2_inv" in k[-1] and len(k) == 5
+            assert all(("k2_inv_rhs" in x) == two for x in k[1:-1]), (ny, nx, nz, L)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ny,nx", [(72, 64), (64, 72)])
+def test_planes_of_more_waves_match_oracle(wlc, oracle, ny, nx):
+    # 648 planes, then 288
+    _matches_oracle(wlc, oracle, (72, ny, nx), (2, 2), (2, 1))
 
 
 # 72 x 12, 16 and 24 planes: C + A by the run-time kernels above 1280 planes, A and C alone not

@@ -395,7 +395,9 @@ static bool specialised(const Geom& g) {
 
 // FP64 spectrum only: with the FP32 one another order of the same operations rounds some stored
 // values the other way, which after 40 to 100 steps moves phi by 1e-9 to 1e-7 of itself, as far as
-// the storage type itself does, so that mode keeps the kernels and with them its results
+// the storage type itself does, so that mode keeps the kernels and with them its results.  It costs
+// time: C + A of 48^3 / Lmax 6 59.6 us against 53.5 with the FP64 spectrum, of 36 x 54 x 48 / Lmax 4
+// 55.2 against 43.0 (launches timed by events).
 static bool two_pass_plane(const Geom& g, int kind, int planes) {
   if (g.spec32 || specialised(g) || !p2::takes(g.nx, g.ny)) return false;
   // 72 x 12, x 16 and x 24, either way round, C + A: three waves a plane, two planes per CU, and not
@@ -410,10 +412,14 @@ static bool two_pass_plane(const Geom& g, int kind, int planes) {
   // SIMD), while the run-time kernel keeps these planes in eight slots a thread.  From about two
   // planes per CU on that one is faster: C + A of 72 x 48 with 400 planes 37.3 us against 31.2 us of
   // the two-pass kernel, with 576 44.4 against 45.3, 1024 52.2 against 61.4, 3136 152 against 187.
-  // (72 x 64, 64 x 72 and 72 x 72, five and six waves, need sixteen slots there: 0.94 to 1.00 of
-  // its time.)
-  const bool one_per_cu = p2::shape_of(g.nx, g.ny).waves > 4;
-  return !(one_per_cu && pick_maxe((long long)g.ny * g.nxh, kThreads) == 8 && planes > 512);
+  // 72 x 64, 64 x 72 and 72 x 72, five and six waves, need sixteen slots there; alone, the two-pass C + A
+  // takes 0.94 to 1.00 of its time.  Beside the other sweep and the generic z solve of a long z axis it
+  // falls behind with some planes per CU and catches up with many: pair of sweeps of 40 steps on
+  // 72 x 64 x 72, run-time / two-pass, 648 planes 5.80 / 6.27 ms, 1152 9.74 / 11.2, 1800 17.6 / 17.8,
+  // 2592 27.6 / 27.7, 3528 38.9 / 37.2; on 72^2 x 96, 864 8.46 / 9.19, 1536 14.6 / 15.6, 3456 42.1 / 42.3.
+  if (p2::shape_of(g.nx, g.ny).waves <= 4) return true;
+  if (pick_maxe((long long)g.ny * g.nxh, kThreads) == 8) return planes <= 512;
+  return !(kind == 2 && g.nz > 64 && planes > 600 && planes <= 3300);
 }
 
 static size_t plane_lds_bytes(const Geom& g) {
