@@ -30,9 +30,10 @@ ZOpts zsolve_opts(int nz, int L, int spec32) {
   ZOpts o;
   o.generic = 0;
   o.occ = 1;
-  // short nz, FP64 spectrum: the column kernel at every Lmax (24^3 / Lmax 6 11.2 against 20.5 us of
-  // the half-tile kernel before it, 36^3 / Lmax 4 13.1 against 27 us of the generic one); Lmax 5-7
-  // at nz = 64: the whole-tile split kernel; elsewhere a degree split
+  // short nz, FP64 spectrum: the column kernel (24^3 / Lmax 6 12.8 us against 17.0 of the half-tile
+  // kernel before it, 36^3 / Lmax 4 14.1 against 28.9 of the generic one; zcol_groups in
+  // wlc_dispatch.cpp draws the line); Lmax 5-7 at nz = 64: the whole-tile split kernel; elsewhere a
+  // degree split
   o.split = 2;
   o.tx = zsolve_tx(nz);
   o.tuned = 0;

@@ -11,10 +11,12 @@
 // (four waves again).  The loads of the first radix pass and the stores of the last go straight
 // between HBM and registers.  The transform is two register passes (n = R T), both in place, so
 // kz index k1 + R k2 sits in row k1 (T slots) during the solve and nothing is reordered.
-// Measured per launch against the half-tile kernel it replaces (all harmonics of half a column
-// in the registers of one wave): 24^3 / Lmax 6 16.0 -> 11.2 us (of which 2.2 are launch and 2.4
-// the first loads), 32^3 / Lmax 4 13.5 -> 10.7, 48^3 / Lmax 6 51.6 -> 40.3 and Lmax 4 26 -> 23.5;
-// against the generic kernel, 36^3 / Lmax 4 27 -> 13.1.  It is bound by the latency of its phases.
+// Per launch in one kernel trace, against the half-tile kernel it replaces (all harmonics of half a
+// column in the registers of one wave): 24^3 / Lmax 6 17.0 -> 12.8 us (of which 2.2 are launch and 2.4
+// the first loads), Lmax 4 10.6 -> 8.6, 32^3 / Lmax 4 15.6 -> 12.7, 48^3 / Lmax 6 46.6 -> 40.7, but 48^3 /
+// Lmax 4 21.9 -> 24.7 and Lmax 5 28.7 -> 31.3 (its 624 groups are a second round of 512, a fifth full);
+// against the generic kernel, 36^3 / Lmax 4 28.9 -> 14.1, 54^3 / Lmax 4 64.7 -> 28.3.  It is bound by the
+// latency of its phases.  Where it is not taken: zcol_groups in wlc_dispatch.cpp.
 #include <hip/hip_runtime.h>
 
 #include "wlc_dft.h"
