@@ -67,59 +67,78 @@ def _batch_matches_handles(wlc, instances):
     b.close()
 
 
-# 48 x 72 planes: two-pass kernels up to 512 planes of a launch, the run-time kernels above; a chain
-# whose Lmax changes crosses the line
+# 48 x 72 planes: two-pass kernels up to 512 planes of the largest block's launches, the run-time kernels
+# above; all launches of a chain alike
 def test_planes_of_five_waves(so):
     for ny, nx in ((48, 72), (72, 48)):
         for nz, L, two in ((32, (3,), True), (36, (3,), False), (18, (4,), True), (24, (4,), False)):
             k = [x for x in _launches(so, (nz, ny, nx), (4,), L) if "k2_" in x or "rhs" in x or "ifft" in x]
             assert len(k) == 5 and all(("k2_" in x) == two for x in k), (ny, nx, nz, L)
-    k = [x for x in _launches(so, (36, 48, 72), (3, 3), (2, 3)) if "k2_" in x or "rhs" in x or "ifft" in x]
-    assert [("k2_" in x) for x in k] == [True, True, True, False, False, False, False]
+    for L in ((2, 3), (3, 2)):
+        k = [x for x in _launches(so, (36, 48, 72), (3, 3), L) if "k2_" in x or "rhs" in x or "ifft" in x]
+        assert len(k) == 7 and not any("k2_" in x for x in k), L
     # other planes keep the two-pass kernels at any number
     for nz, ny, nx in ((72, 54, 72), (64, 64, 72), (64, 72, 72), (72, 36, 72)):
         k = _launches(so, (nz, ny, nx), (4,), (4,))
         assert sum("k2_" in x for x in k) == 5, (nz, ny, nx)
 
 
-# 72 x 64, 64 x 72 and 72 x 72 planes on a z axis longer than 64: C + A by the run-time kernels between
-# 600 and 3300 planes
+# 72 x 64, 64 x 72 and 72 x 72 planes on a z axis longer than 64: run-time kernels between 600 and 3300
+# planes
 def test_planes_of_more_waves(so):
     for ny, nx in ((72, 64), (64, 72), (72, 72)):
         for nz, L, two in ((72, 1, True), (72, 2, False), (64, 3, True), (96, 3, False), (72, 5, False), (72, 6, True)):
             k = [x for x in _launches(so, (nz, ny, nx), (4,), (L,)) if "k2_" in x or "rhs" in x or "ifft" in x]
-            assert "k2_rhs" in k[0] and "k2_inv" in k[-1] and len(k) == 5
-            assert all(("k2_inv_rhs" in x) == two for x in k[1:-1]), (ny, nx, nz, L)
+            assert len(k) == 5 and all(("k2_" in x) == two for x in k), (ny, nx, nz, L)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("ny,nx", [(72, 64), (64, 72)])
 def test_planes_of_more_waves_match_oracle(wlc, oracle, ny, nx):
-    # 648 planes, then 288
+    # 648 planes and, after the junction, 288
     _matches_oracle(wlc, oracle, (72, ny, nx), (2, 2), (2, 1))
 
 
-# 72 x 12, 16 and 24 planes: C + A by the run-time kernels above 1280 planes, A and C alone not
+# 72 x 12, 16 and 24 planes: run-time kernels above 1280 planes
 def test_thin_planes(so):
     for ny, nx, thin in ((72, 12, True), (12, 72, True), (72, 16, True), (16, 72, True), (72, 24, True),
                          (24, 72, True), (72, 18, False), (18, 72, False), (72, 32, False), (54, 12, False)):
         for nz, L in ((48, 4), (54, 4)):
             k = [x for x in _launches(so, (nz, ny, nx), (4,), (L,)) if "k2_" in x or "rhs" in x or "ifft" in x]
-            assert "k2_rhs" in k[0] and "k2_inv" in k[-1] and len(k) == 5
-            assert all(("k2_inv_rhs" in x) != (thin and nz == 54) for x in k[1:-1]), (ny, nx, nz)
+            assert len(k) == 5 and all(("k2_" in x) != (thin and nz == 54) for x in k), (ny, nx, nz)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("ny,nx", [(72, 12), (12, 72), (72, 16), (24, 72)])
 def test_thin_planes_match_oracle(wlc, oracle, ny, nx):
-    # 1350 planes, then 486, across the junction
+    # 1350 planes and, after the junction, 486
     _matches_oracle(wlc, oracle, (54, ny, nx), (3, 3), (4, 2))
+
+
+# a checkpointed sweep restarts with the kernel that only forms the right-hand side, and ends a segment
+# with the one that only transforms back, where the first sweep ran the fused kernel: the recomputed slices
+# and all that comes of them keep their bits, at a junction too
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,L", [((54, 72, 12), (4, 2)), ((54, 24, 72), (2, 4)), ((72, 64, 72), (2, 1)),
+                                     ((36, 48, 72), (3, 2)), ((24, 36, 54), (3, 1))])
+def test_recomputed_slices_keep_their_bits(wlc, monkeypatch, shape, L):
+    monkeypatch.setenv("WLC_CONCURRENT", "0")
+    w = 1.5 * np.random.default_rng(5).standard_normal((2,) + shape)
+    res = []
+    for k in (0, 3):
+        g = wlc.WormlikeMDE(shape, (4.0, 3.5, 3.0), (6, 7), L, (1.0, 0.5), ckpt_every=k)
+        g.set_w(w)
+        g.MDE_q()
+        g.MDE_qstar()
+        res.append((*g.density(), g.get_q(+1, 13), g.get_q(-1, 0)))
+        g.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*res))
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("ny,nx", [(48, 72), (72, 48)])
 def test_planes_of_five_waves_match_oracle(wlc, oracle, ny, nx):
-    # 324 planes, then 576
+    # 324 planes and, after the junction, 576
     _matches_oracle(wlc, oracle, (36, ny, nx), (3, 3), (2, 3))
 
 

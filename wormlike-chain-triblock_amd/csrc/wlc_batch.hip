@@ -1275,6 +1275,7 @@ int wlc_batch_create(const wlc_params* params, const double* chi, int n, const w
     g.nx = p.nx; g.ny = p.ny; g.nz = p.nz; g.nxh = I.nxh;
     g.nt = kx_tiles(I.nxh);
     g.spec32 = p.spectrum_fp32;
+    g.mtop = I.Mmax;
     g.zs = I.zs;
     g.hs = I.hs;
     AxisDev* ax[3] = {&g.ax, &g.ay, &g.az};

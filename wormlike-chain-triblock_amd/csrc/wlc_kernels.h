@@ -38,6 +38,7 @@ struct Geom {
   int nx, ny, nz, nxh;
   int nt;          // kx tiles
   int spec32;      // 1: the half spectrum is stored as float2
+  int mtop;        // most harmonics of a slice of the chain
   long long zs;    // real-space z-plane stride (doubles): nx*ny + pad
   long long hs;    // real-space field / harmonic stride (doubles): nz*zs + pad
   AxisDev ax, ay, az;

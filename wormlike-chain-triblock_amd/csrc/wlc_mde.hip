@@ -1080,6 +1080,7 @@ int wlc_mde_create(const wlc_params* p, wlc_handle** out) {
   g.nx = p->nx; g.ny = p->ny; g.nz = p->nz; g.nxh = h->nxh;
   g.nt = wlc::kx_tiles(h->nxh);
   g.spec32 = p->spectrum_fp32;
+  g.mtop = h->Mmax;
   g.zs = h->zs;
   g.hs = h->hs;
   wlc::AxisDev* ax[3] = {&g.ax, &g.ay, &g.az};
@@ -1408,6 +1409,7 @@ int wlc_mde_step_noalloc(const wlc_params* p, int dir, int s, const double* cons
   g.nx = p->nx; g.ny = p->ny; g.nz = p->nz; g.nxh = nxh;
   g.nt = wlc::kx_tiles(nxh);
   g.spec32 = p->spectrum_fp32;
+  for (int b = 0; b < p->nblk; ++b) g.mtop = std::max(g.mtop, (p->Lmax[b] + 1) * (p->Lmax[b] + 1));
   g.zs = (long long)p->nx * p->ny;
   g.hs = (long long)p->nz * g.zs;
   wlc::AxisDev* ax[3] = {&g.ax, &g.ay, &g.az};

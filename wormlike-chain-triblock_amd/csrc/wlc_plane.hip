@@ -398,16 +398,21 @@ static bool specialised(const Geom& g) {
 // the storage type itself does, so that mode keeps the kernels and with them its results.  It costs
 // time: C + A of 48^3 / Lmax 6 59.6 us against 53.5 with the FP64 spectrum, of 36 x 54 x 48 / Lmax 4
 // 55.2 against 43.0 (launches timed by events).
-static bool two_pass_plane(const Geom& g, int kind, int planes) {
+//
+// All launches of a chain come from one family, by its largest block: a sweep that restarts from stored
+// slices begins with A and ends with C where the first one ran C + A (across a junction with the
+// harmonics of both blocks), and has to give the same bits.
+static bool two_pass_plane(const Geom& g) {
   if (g.spec32 || specialised(g) || !p2::takes(g.nx, g.ny)) return false;
-  // 72 x 12, x 16 and x 24, either way round, C + A: three waves a plane, two planes per CU, and not
+  const int planes = g.nz * g.mtop;
+  // 72 x 12, x 16 and x 24, either way round: three waves a plane, two planes per CU, and not
   // enough rows or columns for the lanes of all three; beside the other sweep's kernels the four waves
-  // of the run-time kernel do better once there are many planes.  Pair of sweeps of 40 steps, run-time /
-  // two-pass: 72 x 12 with 600 planes 1.83 / 1.89 ms, 1176 2.73 / 2.95, 3136 5.50 / 6.11; 12 x 72, 3136
-  // 5.29 / 5.78; 72 x 16, 600 2.02 / 1.97, 1200 2.99 / 3.01, 2352 5.47 / 5.84; 24 x 72, 600 2.35 / 2.27,
-  // 2352 6.63 / 7.06.  A and C alone stay (a step on 72 x 12 x 64, Lmax 7, 108 / 99 us).
+  // of the run-time kernel do better once there are many planes.  Pair of sweeps of 40 steps, C + A
+  // run-time / two-pass: 72 x 12 with 600 planes 1.83 / 1.89 ms, 1176 2.73 / 2.95, 3136 5.50 / 6.11;
+  // 12 x 72, 3136 5.29 / 5.78; 72 x 16, 600 2.02 / 1.97, 1200 2.99 / 3.01, 2352 5.47 / 5.84; 24 x 72, 600
+  // 2.35 / 2.27, 2352 6.63 / 7.06.  A step by itself is slower (72 x 12 x 64, Lmax 7, 108 / 99 us).
   const int lo = std::min(g.nx, g.ny), hi = std::max(g.nx, g.ny);
-  if (kind == 2 && hi == 72 && (lo == 12 || lo == 16 || lo == 24) && planes > 1280) return false;
+  if (hi == 72 && (lo == 12 || lo == 16 || lo == 24) && planes > 1280) return false;
   // 48 x 72 and 72 x 48: a two-pass plane is five waves, and a CU holds one at a time (two waves per
   // SIMD), while the run-time kernel keeps these planes in eight slots a thread.  From about two
   // planes per CU on that one is faster: C + A of 72 x 48 with 400 planes 37.3 us against 31.2 us of
@@ -415,11 +420,11 @@ static bool two_pass_plane(const Geom& g, int kind, int planes) {
   // 72 x 64, 64 x 72 and 72 x 72, five and six waves, need sixteen slots there; alone, the two-pass C + A
   // takes 0.94 to 1.00 of its time.  Beside the other sweep and the generic z solve of a long z axis it
   // falls behind with some planes per CU and catches up with many: pair of sweeps of 40 steps on
-  // 72 x 64 x 72, run-time / two-pass, 648 planes 5.80 / 6.27 ms, 1152 9.74 / 11.2, 1800 17.6 / 17.8,
+  // 72 x 64 x 72, C + A run-time / two-pass, 648 planes 5.80 / 6.27 ms, 1152 9.74 / 11.2, 1800 17.6 / 17.8,
   // 2592 27.6 / 27.7, 3528 38.9 / 37.2; on 72^2 x 96, 864 8.46 / 9.19, 1536 14.6 / 15.6, 3456 42.1 / 42.3.
   if (p2::shape_of(g.nx, g.ny).waves <= 4) return true;
   if (pick_maxe((long long)g.ny * g.nxh, kThreads) == 8) return planes <= 512;
-  return !(kind == 2 && g.nz > 64 && planes > 600 && planes <= 3300);
+  return g.nz <= 64 || planes <= 600 || planes > 3300;
 }
 
 static size_t plane_lds_bytes(const Geom& g) {
@@ -453,10 +458,9 @@ static void* p128_kernel(int kind) {
   return kind == 0 ? (void*)p128::k_rhs128<ORDER, S> : (void*)p128::k_inv_rhs128<ORDER, S>;
 }
 
-// kind 0: A (order), 1: C, 2: fused C + A (order of the next step); planes: of the launch (nz times
-// harmonics); *threads = workgroup size; S = storage type of the half spectrum; B: the batched twin
+// kind 0: A (order), 1: C, 2: fused C + A (order of the next step); *threads = workgroup size; S = storage type of the half spectrum; B: the batched twin
 template <class S, bool B>
-static void* pick_plane_kernel_t(const Geom& g, int kind, int order, int planes, size_t* lds, int* threads) {
+static void* pick_plane_kernel_t(const Geom& g, int kind, int order, size_t* lds, int* threads) {
   *lds = plane_lds_bytes(g);
   *threads = kThreads;
   if (g.nx == 64 && g.ny == 64) {  // static 32 KB plane
@@ -480,7 +484,7 @@ static void* pick_plane_kernel_t(const Geom& g, int kind, int order, int planes,
     }
     return nullptr;
   }
-  if (two_pass_plane(g, kind, planes)) {
+  if (two_pass_plane(g)) {
     *lds = p2::lds_bytes(g.nx, g.ny);
     *threads = 64 * p2::shape_of(g.nx, g.ny).waves;
     return const_cast<void*>(p2::kernel(g.nx, g.ny, kind, B));
@@ -503,20 +507,20 @@ static void* pick_plane_kernel_t(const Geom& g, int kind, int order, int planes,
   return nullptr;
 }
 
-static void* pick_plane_kernel(const Geom& g, int kind, int order, int planes, size_t* lds, int* threads,
+static void* pick_plane_kernel(const Geom& g, int kind, int order, size_t* lds, int* threads,
                                bool batch = false) {
   if (batch)
-    return g.spec32 ? pick_plane_kernel_t<float2, true>(g, kind, order, planes, lds, threads)
-                    : pick_plane_kernel_t<double2, true>(g, kind, order, planes, lds, threads);
-  return g.spec32 ? pick_plane_kernel_t<float2, false>(g, kind, order, planes, lds, threads)
-                  : pick_plane_kernel_t<double2, false>(g, kind, order, planes, lds, threads);
+    return g.spec32 ? pick_plane_kernel_t<float2, true>(g, kind, order, lds, threads)
+                    : pick_plane_kernel_t<double2, true>(g, kind, order, lds, threads);
+  return g.spec32 ? pick_plane_kernel_t<float2, false>(g, kind, order, lds, threads)
+                  : pick_plane_kernel_t<double2, false>(g, kind, order, lds, threads);
 }
 
 static hipError_t launch_plane(const Geom& g, int kind, int order, int planes, void** args,
                                hipStream_t st) {
   size_t lds = 0;
   int threads = kThreads;
-  void* k = pick_plane_kernel(g, kind, order, g.nz * planes, &lds, &threads);
+  void* k = pick_plane_kernel(g, kind, order, &lds, &threads);
   if (!k) return hipErrorInvalidValue;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -551,7 +555,7 @@ hipError_t launch_inv_rhs(const Geom& g, const InvArgs& c, const RhsArgs& a, int
 LaunchKey plane_key(const Geom& g, int kind, int order, int planes) {
   size_t lds = 0;
   int threads = kThreads;
-  const void* k = pick_plane_kernel(g, kind, order, g.nz * planes, &lds, &threads);
+  const void* k = pick_plane_kernel(g, kind, order, &lds, &threads);
   return LaunchKey{k, (unsigned)(g.nz * planes), 1u, (unsigned)threads, lds};
 }
 
@@ -560,7 +564,7 @@ static hipError_t launch_plane_batch(const Geom& g, int kind, int order, int pla
   if (n <= 0) return hipSuccess;
   size_t lds = 0;
   int threads = kThreads;
-  void* k = pick_plane_kernel(g, kind, order, g.nz * planes, &lds, &threads, true);
+  void* k = pick_plane_kernel(g, kind, order, &lds, &threads, true);
   if (!k) return hipErrorInvalidValue;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
