@@ -225,3 +225,17 @@ def test_nz128_two_parts_match_oracle(wlc, oracle):
 @pytest.mark.gpu
 def test_nz128_batched(wlc):
     _batch_matches_handles(wlc, [((128, 48, 12), 6), ((128, 48, 12), 6), ((128, 4, 12), 6), ((128, 4, 12), 5)])
+
+
+# density runs of concurrent sweeps: two fifths of the terms left, of slices whose q fit in 64 MB
+@pytest.mark.parametrize("nz,L,runs", [(48, 6, [1] * 13), (48, 5, [2, 2, 2, 1, 2, 2, 2]), (16, 3, [3, 2, 2, 3, 2, 1])])
+def test_density_runs(so, nz, L, runs):
+    out = host_hip.run(so, f"""
+        g = W.WormlikeMDE(({nz}, 48, 48), (4.0, 4.0, 4.0), (12,), ({L},), (1.0,))
+        g.set_w(np.zeros((1, {nz}, 48, 48)))
+        g.MDE_q()
+        H.host_hip_forget()
+        g.MDE_qstar()
+        print(sum("density_run" in k for k in launches()))
+    """)
+    assert int(out[0]) == len(runs)

@@ -509,10 +509,17 @@ int density_run(wlc_handle* h, int lo, int hi, int step) {
 }
 
 // the runs and marked slices of the concurrent sweeps: each run takes two fifths of the terms
-// left on its side, so the last ones, which no sweep hides, are short
+// left on its side, so the last ones, which no sweep hides, are short, and no more slices than
+// 64 MB of q hold: of those the memory-side cache (256 MB) still has a part when the run reads
+// them.  Pair of sweeps, runs of two fifths / of the limit: 64^3, Lmax 6 (103 MB a slice), FP32
+// spectrum, 200 steps 60.1 / 57.7 ms, FP64 69.4 / 68.7; 64^3, Lmax 4 (52 MB), 60 steps 9.98 / 9.66;
+// 54^3, Lmax 6 (62 MB) 17.8 / 16.8.  On small slices a launch and an event per term cost more: one
+// term a run on 24^3, Lmax 6 (5 MB), 100 steps 4.12 ms against 3.64.
 void plan_runs(wlc_handle* h) {
   const int Ns = h->Ns, mid = Ns / 2;
-  auto take = [](int left) { return left <= 2 ? left : std::max(2, (2 * left + 4) / 5); };
+  const long long slice = 8LL * h->Mmax * h->hs;
+  const int most = (int)std::max(1LL, (64LL << 20) / slice);
+  auto take = [most](int left) { return std::min(most, left <= 2 ? left : std::max(2, (2 * left + 4) / 5)); };
   for (int hi = mid; hi >= 0;) {
     const int n = take(hi + 1);
     h->runs_lo.push_back({hi - n + 1, hi});
