@@ -9,9 +9,9 @@
 namespace wlc {
 
 // One thread per x pair keeps its sum over the contour points of a run in registers: rho is read
-// and written once per run instead of once per point, and a sweep needs some 15 launches and
-// events instead of one of each per point (an event between two kernels of a stream costs about
-// 5.5 us, of 31 us per contour step at 24^3 / Lmax 6).  The harmonic loop is unrolled so that
+// and written once per run instead of once per point, and a sweep of small slices needs some 15
+// launches and events instead of one of each per point (an event between two kernels of a stream
+// costs about 5.5 us, of 31 us per contour step at 24^3 / Lmax 6).  The harmonic loop is unrolled so that
 // many independent loads are in flight; the sums run in harmonic and contour order.
 __global__ void __launch_bounds__(256) k_density_run(Geom g, DensityRun r) {
   const int nxy2 = (g.nx * g.ny) >> 1;
